@@ -117,8 +117,9 @@ int lmx_accel_intersect_noalloc(lmx_accel *accel, const lmx_ray *rays, uint32_t 
 int lmx_accel_intersect_host(const lmx_accel *accel, const lmx_ray *rays, uint32_t n,
                              lmx_hit *hits, int32_t nthreads);
 
-/* Counting walker: total wide-node visits and triangle tests the traversal
- * kernel performs for these rays (host arrays).  Feeds the kernel's
+/* Counting walker: total wide-node visits and triangle tests of the traversal
+ * kernel's one-ray-per-lane loop for these rays (host arrays; the kernel
+ * traces the last rays of each wave in another order).  Feeds the kernel's
  * algorithmic byte count. */
 int lmx_accel_count(const lmx_accel *accel, const lmx_ray *rays, uint32_t n,
                     uint64_t *node_visits, uint64_t *tri_tests, int32_t nthreads);

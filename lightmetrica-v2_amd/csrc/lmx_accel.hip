@@ -27,7 +27,11 @@
 //     its own XCD (neighbouring rays share BVH nodes in that XCD's L2), then
 //     helps the others; its first chunk is fixed by its index, and only
 //     what the fixed chunks leave is claimed through the regions' atomic
-//     cursors.
+//     cursors;
+//   * the last rays of each wave, and a batch with few rays per wave from
+//     the start, are traced by all its lanes together, eight to a node
+//     (coop_trace): the serial chain of the longest ray, not throughput,
+//     bounds them.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -77,7 +81,8 @@ struct lmx_accel {
     WNode* d_nodes = nullptr;
     WTri* d_tris = nullptr;
     uint32_t* d_counters = nullptr;   // 8 region cursors, the ray count, the stack-overflow flag; CURSOR_STRIDE words apart
-    int grid = 0;
+    int grid = 0;                     // waves of a launch
+    int grid_occl = 0;                // waves of an occlusion launch over many rays
     int stack_depth = 0;              // LDS stack entries per lane
     size_t lds_bytes = 0;
 };
@@ -89,10 +94,11 @@ namespace lmx {
 
 // Returns false when a node group did not fit the stack (a BVH deeper than
 // WBVH_STACK, which the builder refuses); the hit is then a miss.  The walk
-// is the kernel's per-lane state machine, step for step (node test while the
-// two-group triangle queue has room, one triangle per step), so the node
-// visits and triangle tests it counts, and an any-hit ray's reported
-// triangle, are the kernel's.
+// is the kernel's one-ray-per-lane state machine, step for step (node test
+// while the two-group triangle queue has room, one triangle per step), so the
+// node visits and triangle tests it counts are the kernel's for every ray but
+// the last ones of each wave: those the kernel finishes in another order
+// (coop_trace), to the same hit.
 template <int ISECT, bool ANYHIT>
 static bool walk_impl(const WbvhHost& b, const WRay& ray, WHit& hit, uint64_t* nv, uint64_t* nt)
 {
@@ -294,6 +300,205 @@ __device__ __forceinline__ void write_hit(WHit* __restrict__ hits, uint32_t ray_
     reinterpret_cast<float4*>(hits)[ray_id] = o;
 }
 
+// ---------------------------------------------------------------------------
+// The wave's last rays, traced by the whole wave
+//
+// A wave with no ray left to claim and at most COOP_RAYS rays in its lanes
+// leaves the one-ray-per-lane loop: an iteration there costs the same
+// ~1 us (the dependent node load, ~150 VALU for eight boxes and ~100 for a
+// triangle) however few lanes it serves, and the longest of 64 rays takes
+// three to five times as many as the mean one.  Here eight lanes share a node, a
+// slot each, and the wave's pending work -- nodes and triangles of all its
+// rays, tagged with the ray -- lies in two LIFO lists in LDS: a step takes
+// up to eight nodes and 64 triangles off them, whichever rays they belong
+// to, with all their loads in flight together.  One ray alone therefore
+// advances eight nodes at a time, and a step costs one memory latency.
+//
+// The hits are those of the one-ray-per-lane loop bit for bit: the same box
+// and triangle formulas, and the nearest hit (the lowest id among equal t)
+// does not depend on the order of the visits.  An occlusion query reports
+// some triangle in range.
+//
+// Measured (MI355X, against the loop alone, 16 waves per CU): 2,001 rays
+// over 20,480 triangles 40.4 -> 11.6 us, 1,000,003 incoherent rays over
+// 327,680 triangles 239 -> 176 us, 8,388,608 rays over 1.3 M triangles
+// 986 -> 927 us.  Rays left at which a wave changes over: 2 (972 us on the
+// last of these), 4 (941), 8 (931), 12 (927), 16 (929).
+#define COOP_RAYS 12
+#define COOP_SLOTS 16
+#define COOP_TAG_SHIFT 28             // list words: ray slot << 28 | node or triangle index
+#define COOP_REC_WORDS 20             // 80 B apart: the slots' 16-byte words on different banks
+#define COOP_TRI_WORDS 416            // a step leaves at most 8 x 24 triangles, and takes nodes at 64 or fewer
+
+// One slot: the ray, its set-up, its best hit so far.
+struct alignas(16) CoopRec {
+    float ox, oy, oz, tmin;
+    float dx, dy, dz;
+    uint32_t ray_id;
+    float ix, iy, iz;
+    uint32_t meta;                    // octant | kx << 3 | ky << 5 | kz << 7
+    float Sx, Sy, Sz, pad;
+    float t, h0, h1, hdet;            // of the hit named by the slot's key
+};
+static_assert(sizeof(CoopRec) == 4 * COOP_REC_WORDS, "slot record");
+
+struct CoopLds {
+    CoopRec rec[COOP_SLOTS];
+    unsigned long long key[COOP_SLOTS];   // (t as an ordered word, id): the least is the best hit
+    uint32_t tri[COOP_TRI_WORDS];
+};
+
+union alignas(16) TraceLds {
+    TraceTables tab;                  // the one-ray-per-lane loop
+    CoopLds coop;                     // after it
+};
+
+__device__ __forceinline__ void trace_wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// t as an unsigned word of the same order; -0 counts as 0, as it does for
+// the comparisons of test_tri
+__device__ __forceinline__ uint32_t coop_order(float t)
+{
+    const uint32_t u = __float_as_uint(t + 0.0f);
+    return (u & 0x80000000u) ? ~u : u | 0x80000000u;
+}
+
+__device__ __forceinline__ float coop_order_inv(uint32_t k)
+{
+    return __uint_as_float((k & 0x80000000u) ? k & 0x7fffffffu : ~k);
+}
+
+__device__ __forceinline__ unsigned long long coop_key(float t, uint32_t id)
+{
+    return ((unsigned long long)coop_order(t) << 32) | id;
+}
+
+__device__ __forceinline__ WRayPre coop_ray(const CoopRec& c)
+{
+    const float4* w = reinterpret_cast<const float4*>(&c);
+    const float4 a = w[0], b = w[1], d = w[2], e = w[3];
+    WRayPre r;
+    r.ox = a.x; r.oy = a.y; r.oz = a.z; r.tmin = a.w;
+    r.dx = b.x; r.dy = b.y; r.dz = b.z; r.tmax = 0.0f;
+    r.ix = d.x; r.iy = d.y; r.iz = d.z;
+    const uint32_t m = __float_as_uint(d.w);
+    r.oct = m & 7u;
+    r.kx = (int)((m >> 3) & 3u); r.ky = (int)((m >> 5) & 3u); r.kz = (int)((m >> 7) & 3u);
+    r.Sx = e.x; r.Sy = e.y; r.Sz = e.z;
+    return r;
+}
+
+// wb_slot_hits for one slot: the same operations on that slot's bounds
+// (q: lower bound in the low byte, upper in the next)
+__device__ __forceinline__ bool coop_slot_hit(float nox, float noy, float noz, uint32_t ew, uint32_t qx, uint32_t qy,
+                                              uint32_t qz, const WRayPre& r, float tmax)
+{
+    const float sx = __uint_as_float((ew & 0xffu) << 23) * r.ix;
+    const float sy = __uint_as_float(((ew >> 8) & 0xffu) << 23) * r.iy;
+    const float sz = __uint_as_float(((ew >> 16) & 0xffu) << 23) * r.iz;
+    const float bx = (nox - r.ox) * r.ix, by = (noy - r.oy) * r.iy, bz = (noz - r.oz) * r.iz;
+    auto q = [](uint32_t w, bool upper) { return (float)(upper ? w >> 8 : w & 0xffu) * 0x1p-24f; };
+    const bool nx = sx < 0.0f, ny = sy < 0.0f, nz = sz < 0.0f;
+    const float xn = fmaf(q(qx, nx), sx, bx), xf = fmaf(q(qx, !nx), sx, bx);
+    const float yn = fmaf(q(qy, ny), sy, by), yf = fmaf(q(qy, !ny), sy, by);
+    const float zn = fmaf(q(qz, nz), sz, bz), zf = fmaf(q(qz, !nz), sz, bz);
+    const float tn = fmaxf(fmaxf(xn, yn), fmaxf(zn, r.tmin));
+    const float tf = fminf(fminf(xf, yf), fminf(zf, tmax));
+    return tn <= tf * WBVH_FAR_SCALE;
+}
+
+// Lists on entry: node[0, nnode) and L.tri[0, ntri); cap: words of `node`.
+// A step takes more than one node only while the children of all of them
+// fit below cap - 7 depth; with one node a step the list grows by at most 7
+// a level, so it never passes cap.
+template <int ISECT, bool ANYHIT>
+__device__ __forceinline__ void coop_trace(CoopLds& L, uint32_t* node, uint32_t nnode, uint32_t ntri, uint32_t cap,
+                                           uint32_t depth, __amdgpu_buffer_rsrc_t nrs, const WTri* __restrict__ tris)
+{
+    const uint32_t lane = threadIdx.x, g = lane >> 3, s = lane & 7u;
+    const uint32_t index = (1u << COOP_TAG_SHIFT) - 1u;
+    const uint32_t room = cap - 7u * depth;
+    while (nnode | ntri) {
+        const uint32_t T = min(ntri, 64u);
+        uint32_t K = 0;
+        if (ntri <= 64u) K = nnode + 56u <= room ? min(nnode, 8u) : min(nnode, 1u);
+        // 1. take the work and issue every load
+        const bool ht = lane < T;
+        bool hn = g < K;
+        const uint32_t te = ht ? L.tri[ntri - 1u - lane] : 0u;
+        const uint32_t ne = hn ? node[nnode - 1u - g] : 0u;
+        ntri -= T;
+        nnode -= K;
+        const uint32_t ns = ne >> COOP_TAG_SHIFT, ts = te >> COOP_TAG_SHIFT;
+        const int off = (int)((ne & index) * (uint32_t)sizeof(WNode));
+        const auto n0 = __builtin_amdgcn_raw_buffer_load_b128(nrs, off, 0, 0);
+        const auto n1 = __builtin_amdgcn_raw_buffer_load_b128(nrs, off + 16, 0, 0);
+        const int qo = off + 32 + 2 * (int)s;
+        const uint32_t qx = __builtin_amdgcn_raw_buffer_load_b16(nrs, qo, 0, 0);
+        const uint32_t qy = __builtin_amdgcn_raw_buffer_load_b16(nrs, qo + 16, 0, 0);
+        const uint32_t qz = __builtin_amdgcn_raw_buffer_load_b16(nrs, qo + 32, 0, 0);
+        // 2. a triangle per lane
+        if (ht) {
+            WTri tri;
+            load_tri(tri, tris + (te & index));
+            const WRayPre r = coop_ray(L.rec[ts]);
+            const float best = coop_order_inv((uint32_t)(L.key[ts] >> 32));
+            float t, a0, a1, dt = 1.0f;
+            bool h;
+            if (ISECT == WBVH_ISECT_WATERTIGHT) h = wb_tri_watertight(tri, r, best, t, a0, a1, dt);
+            else h = wb_tri_triaccel(tri, r, best, t, a0, a1);
+            if (h) {
+                const unsigned long long k = coop_key(t, wb_tri_id(tri, ISECT));
+                atomicMin(&L.key[ts], k);
+                trace_wave_sync();
+                if (L.key[ts] == k) {
+                    float4* w = reinterpret_cast<float4*>(&L.rec[ts]);
+                    w[4] = make_float4(t, a0, a1, dt);
+                }
+            }
+        }
+        trace_wave_sync();
+        // 3. a slot per lane
+        bool inner = false;
+        uint32_t cnt = 0;
+        const uint32_t imask = n0[3] >> 24;
+        const uint64_t kw = L.key[ns];
+        if (ANYHIT) hn = hn && (uint32_t)kw == WBVH_MISS;
+        const WRayPre r = coop_ray(L.rec[ns]);
+        if (hn && coop_slot_hit(__uint_as_float(n0[0]), __uint_as_float(n0[1]), __uint_as_float(n0[2]), n0[3], qx, qy,
+                                qz, r, coop_order_inv((uint32_t)(kw >> 32)))) {
+            inner = (imask >> s) & 1u;
+            if (!inner) cnt = (uint32_t)__popc((n1[2] >> (3u * s)) & 7u);
+        }
+        // hit children onto the node list: those of the node taken first (the
+        // list's top) on top again, and a node's nearest child above the rest
+        const uint64_t im = __ballot(inner);
+        if (inner) {
+            const uint32_t gm = wb_octant_order((uint32_t)(im >> (8u * g)) & 0xffu, r.oct);
+            const uint32_t above = (uint32_t)__popcll((im >> (8u * g)) >> 8);
+            node[nnode + above + (uint32_t)__popc((gm >> (s ^ r.oct)) >> 1)] =
+                (ns << COOP_TAG_SHIFT) | (n1[0] + (uint32_t)__popc(imask & ((1u << s) - 1u)));
+        }
+        nnode += (uint32_t)__popcll(im);
+        // hit leaves' triangles onto the triangle list
+        const uint32_t first = n1[1] + (uint32_t)__popc(n1[2] & ((1u << (3u * s)) - 1u));
+#pragma unroll
+        for (uint32_t k = 0; k < WBVH_MAX_LEAF_TRIS; k++) {
+            const uint64_t m = __ballot(cnt > k);
+            if (cnt > k)
+                L.tri[ntri + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] =
+                    (ns << COOP_TAG_SHIFT) | (first + k);
+            ntri += (uint32_t)__popcll(m);
+        }
+        trace_wave_sync();
+    }
+}
+
 // The LDS stack is sized per launch to the BVH's depth (stack_depth entries
 // of 8 bytes per lane); with the 3 KB of node-test tables it bounds the
 // workgroups per CU (22 at depth 8, where the registers allow 20).
@@ -307,15 +512,21 @@ void k_trace(const WNode* __restrict__ nodes,
                                                       WHit* __restrict__ hits,
                                                       uint32_t* __restrict__ cursors,
                                                       uint32_t* __restrict__ overflow,
-                                                      int stack_depth, uint32_t refill_min, uint32_t node_bytes)
+                                                      int stack_depth, uint32_t refill_min, uint32_t node_bytes,
+                                                      uint32_t n_fixed, uint32_t coop_max)
 {
     extern __shared__ uint2 stack[];     // [stack_depth][TRACE_WAVE]
     const uint32_t lane = threadIdx.x;
-    const uint32_t nray = cursors[8 * CURSOR_STRIDE];
+    const uint32_t nray = n_fixed ? n_fixed : cursors[8 * CURSOR_STRIDE];
     if (nray == 0) return;                  // uniform over the grid
     const uint32_t claim = trace_claim(nray, gridDim.x);
-    __shared__ TraceTables s_tab;
-    {
+    // regions not yet found exhausted: none when the fixed chunks cover every
+    // region (no cursor is read then)
+    uint32_t regions_left =
+        __ballot(lane < 8u && region_dyn_start(lane & 7u, nray, gridDim.x, claim) < region_end(lane & 7u, nray)) ? 8u : 0u;
+    __shared__ TraceLds lds;
+    TraceTables& s_tab = lds.tab;
+    if (regions_left != 0 || claim > coop_max) {   // else the one-ray-per-lane loop runs no iteration
         const uint4* src = reinterpret_cast<const uint4*>(&g_trace_tables);
         uint4* dst = reinterpret_cast<uint4*>(&s_tab);
         for (uint32_t i = lane; i < (uint32_t)(sizeof(TraceTables) / 16); i += TRACE_WAVE) dst[i] = src[i];
@@ -323,7 +534,6 @@ void k_trace(const WNode* __restrict__ nodes,
     __syncthreads();
 
     uint32_t region = blockIdx.x & 7u;
-    uint32_t regions_left = 8;          // regions not yet found exhausted
     uint32_t pool_base = 0, pool_cnt = 0;   // claimed, not yet started rays
     // direction set-up of the pool's rays: lane pool_lane + k holds that of
     // ray pool_base + k (octant | kx << 3 | ky << 5 | kz << 7 in p_meta)
@@ -365,7 +575,7 @@ void k_trace(const WNode* __restrict__ nodes,
         // the lanes refilled
         const uint64_t idle = __ballot(!valid);
         const uint32_t nidle = (uint32_t)__popcll(idle);
-        if ((regions_left != 0 || pool_cnt != 0) && (nidle >= refill_min || nidle == TRACE_WAVE)) {
+        if ((first || regions_left != 0 || pool_cnt != 0) && (nidle >= refill_min || nidle == TRACE_WAVE)) {
             if (done) {
                 write_hit<ISECT>(hits, ray_id, best_t, best_id, h0, h1, hdet);
                 done = false;
@@ -400,10 +610,10 @@ void k_trace(const WNode* __restrict__ nodes,
                             regions_left--;
                         }
                     }
-                    cb = __shfl(cb, 0);
-                    cg = __shfl(cg, 0);
-                    regions_left = __shfl(regions_left, 0);
-                    region = __shfl(region, 0);
+                    cb = __builtin_amdgcn_readfirstlane(cb);
+                    cg = __builtin_amdgcn_readfirstlane(cg);
+                    regions_left = __builtin_amdgcn_readfirstlane(regions_left);
+                    region = __builtin_amdgcn_readfirstlane(region);
                 }
                 pool_base = cb;
                 pool_cnt = cg;
@@ -446,8 +656,20 @@ void k_trace(const WNode* __restrict__ nodes,
             }
         }
         // single loop back-edge: with no ray in any lane and work left, the
-        // body below does nothing but reload the root
-        if (__ballot(valid) == 0 && regions_left == 0 && pool_cnt == 0) break;
+        // body below does nothing but reload the root.  The last rays of the
+        // wave go to coop_trace.
+        if (regions_left == 0 && pool_cnt == 0) {
+            const uint32_t left = (uint32_t)__popcll(__ballot(valid));
+            if (left == 0) break;
+            if (left <= coop_max) {
+                // their queued triangles have to fit the list (12 rays could
+                // hold 576; a few iterations on they do)
+                uint32_t q = valid ? (uint32_t)(__popc(pend) + __popc(pend2)) : 0u;
+#pragma unroll
+                for (int o = TRACE_WAVE / 2; o > 0; o >>= 1) q += (uint32_t)__shfl_xor((int)q, o);
+                if (__builtin_amdgcn_readfirstlane(q) <= COOP_TRI_WORDS) break;
+            }
+        }
 
         // 1. lanes with room in their triangle queue: box test of the node
         //    loaded in the previous iteration, its leaf triangles queued, and
@@ -525,6 +747,100 @@ void k_trace(const WNode* __restrict__ nodes,
         }
     }
     if (done) write_hit<ISECT>(hits, ray_id, best_t, best_id, h0, h1, hdet);
+
+    // ---- the wave's last rays
+    const uint64_t act = __ballot(valid);
+    if (act == 0) return;
+    CoopLds& L = lds.coop;                 // over the tables
+    uint32_t* list = reinterpret_cast<uint32_t*>(stack);
+    __syncthreads();                       // the loop's LDS reads are done
+    const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(act >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)act, 0u));
+    const uint32_t tag = rank << COOP_TAG_SHIFT;
+    const uint32_t nslot = (uint32_t)__popcll(act);
+    if (valid) {
+        float4* w = reinterpret_cast<float4*>(&L.rec[rank]);
+        w[0] = make_float4(r.ox, r.oy, r.oz, r.tmin);
+        // the watertight test reads no direction: leaving it out here keeps
+        // it out of the loop's registers
+        if (ISECT == WBVH_ISECT_WATERTIGHT) L.rec[rank].ray_id = ray_id;
+        else w[1] = make_float4(r.dx, r.dy, r.dz, __uint_as_float(ray_id));
+        w[2] = make_float4(r.ix, r.iy, r.iz,
+                           __uint_as_float(r.oct | ((uint32_t)r.kx << 3) | ((uint32_t)r.ky << 5) | ((uint32_t)r.kz << 7)));
+        w[3] = make_float4(r.Sx, r.Sy, r.Sz, __int_as_float(sp));
+        w[4] = make_float4(best_t, h0, h1, hdet);
+        L.key[rank] = coop_key(best_t, best_id);
+    }
+    trace_wave_sync();
+    // queued triangles: each lane's bits from its exclusive prefix on
+    uint32_t ntri = 0;
+    {
+        uint32_t cnt = valid ? (uint32_t)(__popc(pend) + __popc(pend2)) : 0u, incl = cnt;
+#pragma unroll
+        for (int o = 1; o < TRACE_WAVE; o <<= 1) {
+            const uint32_t v = (uint32_t)__shfl_up((int)incl, o);
+            if (lane >= (uint32_t)o) incl += v;
+        }
+        ntri = (uint32_t)__shfl((int)incl, TRACE_WAVE - 1);
+        uint32_t at = incl - cnt;
+        if (valid) {
+            for (uint32_t b = pend; b; b &= b - 1u)
+                L.tri[at++] = tag | wb_tri_index(tbase, tvalid, (uint32_t)(__ffs(b) - 1));
+            for (uint32_t b = pend2; b; b &= b - 1u)
+                L.tri[at++] = tag | wb_tri_index(tbase2, tvalid2, (uint32_t)(__ffs(b) - 1));
+        }
+    }
+    // pending nodes: the lanes' stacks (lane 16 j + k takes level 4 q + j of
+    // slot k's stack), deeper levels above, each level's nearest child on
+    // top; the list overlays the stacks, so all of them are read first
+    constexpr int LEVELS = TRACE_WAVE / COOP_SLOTS;   // stack levels a round
+    const uint32_t myslot = lane % COOP_SLOTS;
+    uint32_t src_lane = 0;                 // that slot's lane
+    {
+        uint64_t m = act;
+        for (uint32_t k = 0; k < myslot; k++) m &= m - 1u;
+        src_lane = m ? (uint32_t)(__ffsll((unsigned long long)m) - 1) : 0u;
+    }
+    const int mysp = myslot < nslot ? __float_as_int(L.rec[myslot].pad) : 0;
+    const uint32_t myoct = myslot < nslot ? L.rec[myslot].meta & 7u : 0u;
+    uint2 lev[WBVH_STACK / LEVELS];
+#pragma unroll
+    for (int q = 0; q < WBVH_STACK / LEVELS; q++) {
+        const int d = LEVELS * q + (int)(lane / COOP_SLOTS);
+        lev[q] = d < mysp ? stack[d * TRACE_WAVE + src_lane] : make_uint2(0u, 0u);
+    }
+    __syncthreads();
+    uint32_t nnode = 0;
+#pragma unroll
+    for (int q = 0; q < WBVH_STACK / LEVELS; q++) {
+        if (LEVELS * q >= stack_depth) break;
+        uint32_t hm = lev[q].y & 0xffu;
+        const uint32_t im = lev[q].y >> 8, cnt = (uint32_t)__popc(hm);
+        uint32_t incl = cnt;
+#pragma unroll
+        for (int o = 1; o < TRACE_WAVE; o <<= 1) {
+            const uint32_t v = (uint32_t)__shfl_up((int)incl, o);
+            if (lane >= (uint32_t)o) incl += v;
+        }
+        uint32_t at = nnode + incl;        // filled downwards: the nearest child last in memory
+        for (; hm; hm &= hm - 1u) {
+            const uint32_t c = (uint32_t)(__ffs(hm) - 1) ^ myoct;
+            list[--at] = (myslot << COOP_TAG_SHIFT) | (lev[q].x + (uint32_t)__popc(im & ((1u << c) - 1u)));
+        }
+        nnode += (uint32_t)__shfl((int)incl, TRACE_WAVE - 1);
+    }
+    {
+        const uint64_t m = __ballot(valid && more);      // the nodes chosen next
+        if (valid && more)
+            list[nnode + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] = tag | cur;
+        nnode += (uint32_t)__popcll(m);
+    }
+    trace_wave_sync();
+    coop_trace<ISECT, ANYHIT>(L, list, nnode, ntri, 2u * TRACE_WAVE * (uint32_t)stack_depth, (uint32_t)stack_depth, nrs,
+                              tris);
+    if (lane < nslot) {
+        const CoopRec& c = L.rec[lane];
+        write_hit<ISECT>(hits, c.ray_id, c.t, (uint32_t)L.key[lane], c.h0, c.h1, c.hdet);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -639,7 +955,20 @@ int lmx_accel_upload(lmx_accel* a)
     else
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_trace<WBVH_ISECT_TRIACCEL, false>, TRACE_WAVE, a->lds_bytes);
     if (e != hipSuccess) return hip_error(e, "lmx_accel_upload: occupancy query");
-    a->grid = std::max(8, cus * std::max(1, per_cu));
+    // Waves per CU.  The 64 rays of a wave each walk their own part of the
+    // tree, and where the tree is larger than an XCD's 4 MB of L2 what more
+    // waves gain in latency hidden they lose in the 32 KB L1: 8,388,608 rays
+    // over 75 MB of tree take 947 us with 20 waves (what the registers
+    // allow), 932 with 16, 984 with 14; renderer::vcm passes over as much 5 %
+    // less with 16 than with 20.  A tree within the L2 (the Cornell box) is
+    // traced 2 % faster by 20 waves than by 16.  Shadow rays of a large
+    // batch, each from another place, thrash it sooner: 3,000,001 of them
+    // over 18 MB take 887 us with 20 waves, 836 with 16, 746 with 12, and 812
+    // with 10.
+    per_cu = std::max(1, per_cu);
+    const bool large = nb + tb > ((size_t)4 << 20);
+    a->grid = std::max(8, cus * (large ? std::min(per_cu, 16) : per_cu));
+    a->grid_occl = std::max(8, cus * (large ? std::min(per_cu, 12) : per_cu));
     a->device = dev;
     return LMX_OK;
 }
@@ -652,9 +981,11 @@ namespace lmx {
 // device, with its region cursors and ray count at `counters` (9 words,
 // CURSOR_STRIDE apart, of device memory); the stack-overflow flag is always
 // the accel's own.
-static int trace_grid(const lmx_accel* a, uint32_t n_max)
+static int trace_grid(const lmx_accel* a, uint32_t n_max, bool many_occl = false)
 {
-    return std::max(1, std::min(a->grid, (int)((n_max + TRACE_WAVE - 1) / TRACE_WAVE)));
+    // a wave per ray as long as there are waves (whole rounds of the 8
+    // regions, so that the fixed chunks cover every region)
+    return (int)std::min<uint64_t>((uint64_t)(many_occl ? a->grid_occl : a->grid), ((uint64_t)n_max + 7u) / 8u * 8u);
 }
 
 static int enqueue_trace(const lmx_accel* a, uint32_t* counters, const WRay* rays, uint32_t n,
@@ -662,22 +993,28 @@ static int enqueue_trace(const lmx_accel* a, uint32_t* counters, const WRay* ray
                          bool cursors_set = false)
 {
     uint32_t* overflow = a->d_counters + 9 * CURSOR_STRIDE;
-    const int grid = trace_grid(a, n_max);
+    // (fewer waves only pay while each has several rounds of rays: at one
+    // round, 200,000 shadow rays, 12 waves per CU take 129 us and 16 take 98)
+    const bool many_occl = anyhit && !n_dev && !cursors_set && n >= 4u * TRACE_WAVE * (uint32_t)a->grid_occl;
+    const int grid = trace_grid(a, n_max, many_occl);
     const uint32_t node_bytes = (uint32_t)(a->host.nodes.size() * sizeof(WNode));   // < 4 GB, the builder's bound
-    if (!cursors_set) k_init_cursors<<<1, 64, 0, s>>>(counters, n, n_dev, (uint32_t)grid);
+    // a count the host knows goes with the launch, and when the fixed chunks
+    // cover the rays no wave reads a cursor
+    const uint32_t n_fixed = n_dev ? 0u : n;
+    if (!cursors_set && (n_dev || trace_has_dynamic(n, (uint32_t)grid)))
+        k_init_cursors<<<1, 64, 0, s>>>(counters, n, n_dev, (uint32_t)grid);
+    // the list words of coop_trace hold 28-bit indices
+    const uint32_t coop_max =
+        a->host.nodes.size() <= (1u << COOP_TAG_SHIFT) && a->host.tris.size() <= (1u << COOP_TAG_SHIFT) ? COOP_RAYS : 0u;
     const bool wt = a->host.isect == WBVH_ISECT_WATERTIGHT;
-    if (wt && !anyhit)
-        k_trace<WBVH_ISECT_WATERTIGHT, false><<<grid, TRACE_WAVE, a->lds_bytes, s>>>(
-            a->d_nodes, a->d_tris, rays, hits, counters, overflow, a->stack_depth, REFILL_MIN, node_bytes);
-    else if (wt)
-        k_trace<WBVH_ISECT_WATERTIGHT, true><<<grid, TRACE_WAVE, a->lds_bytes, s>>>(
-            a->d_nodes, a->d_tris, rays, hits, counters, overflow, a->stack_depth, REFILL_MIN, node_bytes);
-    else if (!anyhit)
-        k_trace<WBVH_ISECT_TRIACCEL, false><<<grid, TRACE_WAVE, a->lds_bytes, s>>>(
-            a->d_nodes, a->d_tris, rays, hits, counters, overflow, a->stack_depth, REFILL_MIN, node_bytes);
-    else
-        k_trace<WBVH_ISECT_TRIACCEL, true><<<grid, TRACE_WAVE, a->lds_bytes, s>>>(
-            a->d_nodes, a->d_tris, rays, hits, counters, overflow, a->stack_depth, REFILL_MIN, node_bytes);
+    auto launch = [&](auto kernel) {
+        kernel<<<grid, TRACE_WAVE, a->lds_bytes, s>>>(a->d_nodes, a->d_tris, rays, hits, counters, overflow,
+                                                      a->stack_depth, REFILL_MIN, node_bytes, n_fixed, coop_max);
+    };
+    if (wt && !anyhit) launch(k_trace<WBVH_ISECT_WATERTIGHT, false>);
+    else if (wt) launch(k_trace<WBVH_ISECT_WATERTIGHT, true>);
+    else if (!anyhit) launch(k_trace<WBVH_ISECT_TRIACCEL, false>);
+    else launch(k_trace<WBVH_ISECT_TRIACCEL, true>);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_error(e, "trace launch");
     return LMX_OK;
@@ -710,8 +1047,8 @@ int trace_shape(lmx_accel* a, uint32_t n_max, uint32_t** counters, uint32_t* gri
 // 2,304 bytes, whatever the number of rays -- in this file-scope array
 // instead of the accel's counter block.  Every GPU the library runs on holds
 // its own copy until the process ends, shared by every call on that GPU;
-// k_init_cursors rewrites all 9 words at the start of each launch, so no
-// value carries over from the previous call (two calls that overlap on one
+// k_init_cursors rewrites all 9 words at the start of each launch that reads
+// them, so no value carries over from the previous call (two calls that overlap on one
 // GPU, on different streams, race on it).  On the host, `scratch` only
 // stands in for the device symbol: its device address comes from
 // hipGetSymbolAddress, taken once per device with that device current, and

@@ -21,12 +21,12 @@
 // sticky stack-overflow flag, each on a line of its own
 #define LMX_TRACE_COUNTER_WORDS (10 * CURSOR_STRIDE)
 
-__device__ __forceinline__ uint32_t region_start(uint32_t j, uint32_t n)
+__host__ __device__ __forceinline__ uint32_t region_start(uint32_t j, uint32_t n)
 {
     return (uint32_t)(((uint64_t)n * j) / 8u);
 }
 
-__device__ __forceinline__ uint32_t region_end(uint32_t j, uint32_t n)
+__host__ __device__ __forceinline__ uint32_t region_end(uint32_t j, uint32_t n)
 {
     return (uint32_t)(((uint64_t)n * (j + 1u)) / 8u);
 }
@@ -34,20 +34,31 @@ __device__ __forceinline__ uint32_t region_end(uint32_t j, uint32_t n)
 // Rays per claim: LMX_CLAIM_CHUNK for full queues; short queues (the tail of
 // a wavefront render) are spread over every wave of the grid, so that their
 // time is that of a few rays per wave, not of whole chunks in turn.
-__device__ __forceinline__ uint32_t trace_claim(uint32_t n, uint32_t grid)
+__host__ __device__ __forceinline__ uint32_t trace_claim(uint32_t n, uint32_t grid)
 {
-    return min((uint32_t)LMX_CLAIM_CHUNK, max(1u, (n + grid - 1u) / grid));
+    const uint32_t even = (uint32_t)(((uint64_t)n + grid - 1u) / grid);
+    return even < 1u ? 1u : even > LMX_CLAIM_CHUNK ? LMX_CLAIM_CHUNK : even;
 }
 
 // Every wave's first chunk is fixed by its index (wave b, of XCD region
 // r = b mod 8, takes chunk b / 8 of its region); the region's cursor starts
 // after those chunks, so a launch claims with atomics only what is left,
 // and one with few rays (the tail of a wavefront render) with none.
-__device__ __forceinline__ uint32_t region_dyn_start(uint32_t r, uint32_t n, uint32_t grid, uint32_t claim)
+__host__ __device__ __forceinline__ uint32_t region_dyn_start(uint32_t r, uint32_t n, uint32_t grid, uint32_t claim)
 {
     const uint64_t waves = (grid + 7u - r) / 8u;          // waves b < grid with b mod 8 = r
     const uint64_t s = (uint64_t)region_start(r, n) + waves * claim;
-    return (uint32_t)min(s, (uint64_t)region_end(r, n));
+    const uint64_t e = region_end(r, n);
+    return (uint32_t)(s < e ? s : e);
+}
+
+// Whether any ray of a launch is left to the cursors.
+__host__ __device__ __forceinline__ bool trace_has_dynamic(uint32_t n, uint32_t grid)
+{
+    const uint32_t claim = trace_claim(n, grid);
+    bool any = false;
+    for (uint32_t r = 0; r < 8; r++) any |= region_dyn_start(r, n, grid, claim) < region_end(r, n);
+    return any;
 }
 
 // Thread j of one wave: j < 8 sets region j's cursor, j == 8 the ray count,

@@ -191,3 +191,31 @@ def test_occlusion_matches_closest_hit(gpu, tmax_scale):
         tri = int(accel.hit_ids(hg)[i])
         one = orc.closest_hit_naive(v, f[tri:tri + 1], rays[i:i + 1], test=orc.TEST_WATERTIGHT)
         assert orc.hit_ids(one)[0] == 0
+
+
+@pytest.mark.parametrize("mode", [accel.ISECT_TRIACCEL, accel.ISECT_WATERTIGHT])
+@pytest.mark.parametrize("subdiv", [0, 2, 5])
+@pytest.mark.parametrize("n", [1, 7, 9, 63, 4097, 12 * 4096 + 5, 13 * 5120 + 1])
+def test_last_rays_of_a_wave(gpu, n, subdiv, mode):
+    """The part of the kernel that traces a wave's last rays with all its
+    lanes: alone (one ray per wave, up to 12), and after the one-ray-per-lane
+    loop (13 and more); trees of one level and of many; tmin below 0, finite
+    tmax, zero direction components and rays that cannot hit.  Bit-exact
+    against the host walker over the same BVH, which visits one ray at a
+    time; an occlusion query agrees with the closest hit."""
+    import torch
+    v, f = scenes.displaced_icosphere(subdiv, seed=17)
+    _, rays = scenes.traversal_rays(v, res=2, n_incoherent=n, seed=n)
+    rays = rays.copy()
+    rays[::5, 4 + np.arange(3)[n % 3]] = 0.0
+    rays[1::7, 3] = -2.0
+    rays[2::3, 7] = 0.7
+    rays[3::11, 7] = -1.0
+    a = accel.Accel(v, f, isect=mode)
+    d = torch.from_numpy(rays).to(gpu)
+    hg, ho = a.intersect(d), a.occluded(d)
+    torch.cuda.synchronize()
+    hh = a.intersect_host(rays)
+    np.testing.assert_array_equal(hg.cpu().numpy().view(np.uint32), hh.view(np.uint32))
+    np.testing.assert_array_equal(accel.hit_ids(ho.cpu().numpy()) != accel.MISS, accel.hit_ids(hh) != accel.MISS)
+    assert a.info()["stack_overflow"] == 0
