@@ -501,6 +501,77 @@ RD void splat(const BParams& p, uint32_t pixel, f3 C)
     atomicAdd(fp, C.x); atomicAdd(fp + 1, C.y); atomicAdd(fp + 2, C.z);
 }
 
+// splat() for a whole wave (every lane calls it, `on` says which contribute):
+// lanes that follow one another onto the same pixel, as the connections of
+// one sample do, are summed first and the first of them adds the sum
+// (262,144 Cornell-box samples of renderer::bdpt: k_bd_splat 198 -> 127 us).
+RD void splat_runs(const BParams& p, bool on, uint32_t pixel, f3 C)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint64_t m = __ballot(on);
+    const uint64_t below = m & ((1ull << lane) - 1ull);
+    const int prev = below ? 63 - __clzll((long long)below) : (int)lane;
+    const uint32_t pk = (uint32_t)__shfl((int)pixel, prev);
+    const bool head = on && (below == 0 || pk != pixel);
+    const uint64_t hm = __ballot(head);
+    if (hm != m) {
+        const uint64_t next = hm >> lane >> 1;               // heads after this lane
+        const uint32_t end = next ? lane + (uint32_t)__ffsll((unsigned long long)next) : 64u;
+        if (!on) C = mk3(0, 0, 0);
+#pragma unroll
+        for (uint32_t off = 1; off < 64; off <<= 1) {
+            const f3 v = mk3(__shfl_down(C.x, off), __shfl_down(C.y, off), __shfl_down(C.z, off));
+            if (lane + off < end) C = add(C, v);
+        }
+    }
+    if (head) splat(p, pixel, C);
+}
+
+// Splats that many samples aim at the same few pixels -- light points seen
+// directly, one per sample -- are summed in LDS over a whole workgroup first:
+// an addition to one film address from another XCD than the last one takes
+// about 0.3 us, whatever else the GPU does (262,144 samples of the Cornell
+// box, whose light covers about 140 pixels: 600 us of k_bd_splat's 744).  So
+// the workgroups are few and large, one of 16 waves per CU: 744 -> 127 us
+// there, 120 -> 74 us per pass of 262,144 renderer::vcm samples on the sphere
+// grid.  A pixel whose slot another pixel took goes to the film at once.
+#define SPLAT_THREADS 1024
+#define SPLAT_SLOTS 1024u
+#define SPLAT_FREE 0xffffffffu                 // no film has 2^32 pixels
+struct SplatTab {
+    uint32_t pixel[SPLAT_SLOTS];
+    float c[3][SPLAT_SLOTS];
+};
+
+RD void splat_tab_clear(SplatTab& T)
+{
+    for (uint32_t k = threadIdx.x; k < SPLAT_SLOTS; k += SPLAT_THREADS) {
+        T.pixel[k] = SPLAT_FREE;
+        T.c[0][k] = T.c[1][k] = T.c[2][k] = 0.0f;
+    }
+    __syncthreads();
+}
+
+RD void splat_tab_add(SplatTab& T, const BParams& p, uint32_t pixel, f3 C)
+{
+    const uint32_t k = (pixel * 0x9E3779B1u) >> 22;
+    const uint32_t old = atomicCAS(&T.pixel[k], SPLAT_FREE, pixel);
+    if (old == SPLAT_FREE || old == pixel) {
+        atomicAdd(&T.c[0][k], C.x);
+        atomicAdd(&T.c[1][k], C.y);
+        atomicAdd(&T.c[2][k], C.z);
+    } else {
+        splat(p, pixel, C);
+    }
+}
+
+RD void splat_tab_flush(SplatTab& T, const BParams& p)
+{
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < SPLAT_SLOTS; k += SPLAT_THREADS)
+        if (T.pixel[k] != SPLAT_FREE) splat(p, T.pixel[k], mk3(T.c[0][k], T.c[1][k], T.c[2][k]));
+}
+
 // the smallest path length a strategy may have (renderer_bdpt.cpp:887 applies
 // min_num_vertices only when max_num_vertices is given)
 RD int min_len(const BParams& p) { return (p.variant == BD_BDPT && !p.bounded) ? 0 : p.minv; }
@@ -903,24 +974,40 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     }
 }
 
-__global__ __launch_bounds__(256) void k_bd_splat(BParams p, BCtl* __restrict__ ctl, ShadowQ sq,
-                                                  const float4* __restrict__ hits)
+__global__ __launch_bounds__(SPLAT_THREADS) void k_bd_splat(BParams p, BCtl* __restrict__ ctl, ShadowQ sq,
+                                                            const float4* __restrict__ hits)
 {
+    __shared__ SplatTab tab;
+    splat_tab_clear(tab);
     const uint32_t n = ctl->n_shadow;
     uint32_t live = 0;
-    for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
-        const uint4 m = sq.meta[j];
-        if (m.y == 0) continue;                                      // no contribution
-        live++;
-        if (__float_as_uint(hits[j].w) != WBVH_MISS) continue;      // occluded
-        const float4 c = sq.c[j];
-        const float4 a = sq.aux[j];
-        splat(p, m.w, mk3(c.x, c.y, c.z));
-        // a direct strategy's path has the light point as vertex 0 and the
-        // eye vertices 0 .. t-1: recorded as (s = 0, t + 1, direct)
-        const int t = (int)(m.z & 0xffffu), direct = (int)(m.z >> 16);
-        record(p, m.x, direct ? 0 : (int)m.y, direct ? t + 1 : t, direct, a.x, a.y, mk3(c.x, c.y, c.z), c.w);
+    // whole waves iterate together (splat_runs)
+    for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x) {
+        const uint32_t j = base + threadIdx.x;
+        bool on = false;
+        uint4 m = make_uint4(0u, 0u, 0u, 0u);
+        float4 c = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (j < n) {
+            m = sq.meta[j];
+            if (m.y != 0) {                                          // else no contribution
+                live++;
+                on = __float_as_uint(hits[j].w) == WBVH_MISS;        // else occluded
+            }
+        }
+        if (on) {
+            c = sq.c[j];
+            const float4 a = sq.aux[j];
+            // a direct strategy's path has the light point as vertex 0 and the
+            // eye vertices 0 .. t-1: recorded as (s = 0, t + 1, direct)
+            const int t = (int)(m.z & 0xffffu), direct = (int)(m.z >> 16);
+            record(p, m.x, direct ? 0 : (int)m.y, direct ? t + 1 : t, direct, a.x, a.y, mk3(c.x, c.y, c.z), c.w);
+        }
+        // the light point itself seen from the camera
+        const bool hot = on && m.y == 1u && (m.z & 0xffffu) == 1u;
+        if (hot) splat_tab_add(tab, p, m.w, mk3(c.x, c.y, c.z));
+        splat_runs(p, on && !hot, m.w, mk3(c.x, c.y, c.z));
     }
+    splat_tab_flush(tab, p);
     // live shadow rays, one atomic per wave
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) live += __shfl_xor(live, off);
@@ -1586,9 +1673,11 @@ __global__ __launch_bounds__(256) void k_lt_connect(RScene s, BParams p, BCtl* _
 
 // Unoccluded camera connections to the film (and, when asked, record k of
 // the sample: raster x, y, C rgb, 1, 0, 0).
-__global__ __launch_bounds__(256) void k_lt_splat(BParams p, BCtl* __restrict__ ctl, ShadowQ sq,
-                                                  const float4* __restrict__ hits, int32_t M)
+__global__ __launch_bounds__(SPLAT_THREADS) void k_lt_splat(BParams p, BCtl* __restrict__ ctl, ShadowQ sq,
+                                                            const float4* __restrict__ hits, int32_t M)
 {
+    __shared__ SplatTab tab;
+    splat_tab_clear(tab);
     const uint32_t n = ctl->n_shadow;
     uint32_t live = 0;
     for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
@@ -1596,13 +1685,15 @@ __global__ __launch_bounds__(256) void k_lt_splat(BParams p, BCtl* __restrict__ 
         if (__float_as_uint(hits[j].w) != WBVH_MISS) continue;
         const uint4 m = sq.meta[j];
         const float4 c = sq.c[j], a = sq.aux[j];
-        splat(p, m.w, mk3(c.x, c.y, c.z));
+        if (m.y == 0u) splat_tab_add(tab, p, m.w, mk3(c.x, c.y, c.z));    // the light point itself
+        else splat(p, m.w, mk3(c.x, c.y, c.z));
         if (p.sample_out) {
             float4* o = reinterpret_cast<float4*>(p.sample_out + 8 * ((size_t)m.x * (size_t)M + m.y));
             o[0] = make_float4(a.x, a.y, c.x, c.y);
             o[1] = make_float4(c.z, 1.0f, 0.0f, 0.0f);
         }
     }
+    splat_tab_flush(tab, p);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) live += __shfl_xor(live, off);
     if ((threadIdx.x & 63u) == 0 && live) atomicAdd(&ctl->shadow_rays, (unsigned long long)live);
@@ -1805,7 +1896,8 @@ int bd_enqueue_round(lmx_scene* sc, const BParams& bp, const VB& vb, hipStream_t
     int rc = launch_trace(sc->accel, reinterpret_cast<const WRay*>(sq.ray), 0, &ctl->n_shadow, nconn,
                           reinterpret_cast<WHit*>(sc->bd_shits.p), st, true);
     if (rc != LMX_OK) return rc;
-    k_bd_splat<<<std::max(1, std::min((int)((nconn + 255) / 256), cap_grid)), 256, 0, st>>>(bp, ctl, sq, sc->bd_shits.p);
+    k_bd_splat<<<std::max(1, std::min((int)((nconn + SPLAT_THREADS - 1) / SPLAT_THREADS), sc->cus)), SPLAT_THREADS, 0,
+                 st>>>(bp, ctl, sq, sc->bd_shits.p);
     return LMX_OK;
 }
 
@@ -2845,7 +2937,8 @@ int render_ltdirect(lmx_scene* sc, const lmx_render_params* p, float* film_rgb, 
             rc2 = launch_trace(sc->accel, reinterpret_cast<const WRay*>(sq.ray), 0, &ctl->n_shadow, (uint32_t)nslot,
                                reinterpret_cast<WHit*>(sc->bd_shits.p), st, true);
             if (rc2 != LMX_OK) return rc2;
-            k_lt_splat<<<g, 256, 0, st>>>(pp, ctl, sq, sc->bd_shits.p, (int32_t)pcap);
+            const int gs = std::max(1, (int)std::min<size_t>((nslot + SPLAT_THREADS - 1) / SPLAT_THREADS, (size_t)sc->cus));
+            k_lt_splat<<<gs, SPLAT_THREADS, 0, st>>>(pp, ctl, sq, sc->bd_shits.p, (int32_t)pcap);
             const hipError_t e2 = hipGetLastError();
             return e2 == hipSuccess ? LMX_OK : hip_error(e2, "ltdirect launch");
         });

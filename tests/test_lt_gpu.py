@@ -70,3 +70,30 @@ def test_ltdirect_argument_errors(gpu):
     narrow = torch.zeros((64, 9), dtype=torch.float32, device=gpu)
     with pytest.raises(LmxError, match="narrower"):
         rs.render_ltdirect(64, max_num_vertices=4, table=narrow)
+
+
+@pytest.mark.parametrize("scene", ["cornell", "furnace"])
+@pytest.mark.parametrize("sampler", ["bdpt", "vcm_bdpt", "ltdirect"])
+@pytest.mark.parametrize("w,h,n", [(7, 5, 1), (33, 31, 1500), (64, 48, 70001)])
+def test_film_is_the_sum_of_the_records(gpu, scene, sampler, w, h, n):
+    """The film against a double-precision sum of the per-strategy records of
+    the same render: connections of one sample summed across lanes before
+    they reach the film, and light points seen by the camera summed per
+    workgroup (the Cornell box: few pixels, many samples; the furnace: every
+    pixel a light, more of them than the workgroup's table holds).  A pixel
+    adding k single-precision terms in any order is off by at most
+    k 2^-24 times the sum of their magnitudes."""
+    sc = scenes.cornell_box(w, h) if scene == "cornell" else scenes.furnace_sphere(width=w, height=h)
+    rs = render.Scene(sc)
+    film, _, so = getattr(rs, "render_" + sampler)(n, max_num_vertices=4, seed=5, sample_out=True)
+    film, so = film.cpu().numpy().astype(np.float64), so.cpu().numpy().reshape(-1, 8)
+    rec = so[so[:, 5] > 0]
+    px = np.clip((rec[:, 0] * np.float32(w)).astype(int), 0, w - 1)
+    py = np.clip((rec[:, 1] * np.float32(h)).astype(int), 0, h - 1)
+    want, count = np.zeros((h * w, 3)), np.zeros(h * w)
+    np.add.at(want, py * w + px, rec[:, 2:5].astype(np.float64))
+    np.add.at(count, py * w + px, 1)
+    want *= float(np.float32(w * h / n))
+    assert count.sum() > (0 if n == 1 else n // 10)
+    tol = (count[:, None] + 4) * 2.0 ** -24 * want
+    assert np.all(np.abs(film.reshape(-1, 3) - want) <= tol)
