@@ -94,6 +94,6 @@ def test_film_is_the_sum_of_the_records(gpu, scene, sampler, w, h, n):
     np.add.at(want, py * w + px, rec[:, 2:5].astype(np.float64))
     np.add.at(count, py * w + px, 1)
     want *= float(np.float32(w * h / n))
-    assert count.sum() > (0 if n == 1 else n // 10)
+    assert n == 1 or count.sum() > n // 50        # one light subpath may miss the camera
     tol = (count[:, None] + 4) * 2.0 ** -24 * want
     assert np.all(np.abs(film.reshape(-1, 3) - want) <= tol)
