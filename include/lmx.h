@@ -104,7 +104,7 @@ int lmx_accel_occluded(lmx_accel *accel, const lmx_ray *rays, uint32_t n, lmx_hi
  * forbid hipMalloc.  No counterpart in the reference.  Same arguments, same
  * hits, same kernel.  The accel must already be resident on the current
  * device (lmx_accel_upload), else LMX_EINVAL.  The launch's scratch (region
- * cursors and ray count, 2,304 bytes for any n; n up to 2^31 - 1, else
+ * cursors, 2,304 bytes for any n; n up to 2^31 - 1, else
  * LMX_EINVAL) is one static device array per GPU, held until the process
  * ends and shared by every call on that GPU: calls that overlap on one GPU
  * (different streams, or different threads) race and must be serialised by

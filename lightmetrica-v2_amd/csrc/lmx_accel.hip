@@ -80,7 +80,7 @@ struct lmx_accel {
     int device = -1;
     WNode* d_nodes = nullptr;
     WTri* d_tris = nullptr;
-    uint32_t* d_counters = nullptr;   // 8 region cursors, the ray count, the stack-overflow flag; CURSOR_STRIDE words apart
+    uint32_t* d_counters = nullptr;   // 8 region cursors, a free line, the stack-overflow flag; CURSOR_STRIDE words apart
     int grid = 0;                     // waves of a launch
     int grid_occl = 0;                // waves of an occlusion launch over many rays
     int stack_depth = 0;              // LDS stack entries per lane
@@ -219,13 +219,9 @@ bool wbvh_walk_anyhit(const WbvhHost& b, const WRay& ray, WHit& hit, uint64_t* n
 #endif
 #define REFILL_MIN LMX_REFILL_MIN
 
-// Sets the 8 region cursors for a launch of `grid` waves.  The ray count
-// comes from n_dev when given (a queue length written by an earlier
-// kernel), else from n; the count the trace kernel uses is stored after the
-// cursors.
-__global__ void k_init_cursors(uint32_t* cursors, uint32_t n, const uint32_t* n_dev, uint32_t grid)
+__global__ void k_clear_cursors(uint32_t* cursors)
 {
-    trace_cursors_set(cursors, n_dev ? *n_dev : n, grid, threadIdx.x);
+    trace_cursors_clear(cursors, threadIdx.x);
 }
 
 // The node test's bit shuffles as tables (the internal-child hit mask in
@@ -513,11 +509,12 @@ void k_trace(const WNode* __restrict__ nodes,
                                                       uint32_t* __restrict__ cursors,
                                                       uint32_t* __restrict__ overflow,
                                                       int stack_depth, uint32_t refill_min, uint32_t node_bytes,
-                                                      uint32_t n_fixed, uint32_t coop_max)
+                                                      uint32_t n_fixed, const uint32_t* __restrict__ n_dev,
+                                                      uint32_t coop_max)
 {
     extern __shared__ uint2 stack[];     // [stack_depth][TRACE_WAVE]
     const uint32_t lane = threadIdx.x;
-    const uint32_t nray = n_fixed ? n_fixed : cursors[8 * CURSOR_STRIDE];
+    const uint32_t nray = n_dev ? *n_dev : n_fixed;   // a queue length written by an earlier kernel, or the host's count
     if (nray == 0) return;                  // uniform over the grid
     const uint32_t claim = trace_claim(nray, gridDim.x);
     // regions not yet found exhausted: none when the fixed chunks cover every
@@ -598,8 +595,9 @@ void k_trace(const WNode* __restrict__ nodes,
                             const uint32_t end = region_end(region, nray);
                             // a region whose fixed chunks cover it has
                             // nothing for the cursor
-                            if (region_dyn_start(region, nray, gridDim.x, claim) < end) {
-                                const uint32_t old = atomicAdd(&cursors[region * CURSOR_STRIDE], claim);
+                            const uint32_t dyn = region_dyn_start(region, nray, gridDim.x, claim);
+                            if (dyn < end) {
+                                const uint32_t old = dyn + atomicAdd(&cursors[region * CURSOR_STRIDE], claim);
                                 if (old < end) {
                                     cb = old;
                                     cg = min(claim, end - old);
@@ -978,7 +976,7 @@ int lmx_accel_upload(lmx_accel* a)
 namespace lmx {
 
 // Enqueues one traversal launch of an accel already resident on the current
-// device, with its region cursors and ray count at `counters` (9 words,
+// device, with its region cursors at `counters` (8 words,
 // CURSOR_STRIDE apart, of device memory); the stack-overflow flag is always
 // the accel's own.
 static int trace_grid(const lmx_accel* a, uint32_t n_max, bool many_occl = false)
@@ -990,26 +988,24 @@ static int trace_grid(const lmx_accel* a, uint32_t n_max, bool many_occl = false
 
 static int enqueue_trace(const lmx_accel* a, uint32_t* counters, const WRay* rays, uint32_t n,
                          const uint32_t* n_dev, uint32_t n_max, WHit* hits, hipStream_t s, bool anyhit,
-                         bool cursors_set = false)
+                         bool cursors_clear = false)
 {
     uint32_t* overflow = a->d_counters + 9 * CURSOR_STRIDE;
     // (fewer waves only pay while each has several rounds of rays: at one
     // round, 200,000 shadow rays, 12 waves per CU take 129 us and 16 take 98)
-    const bool many_occl = anyhit && !n_dev && !cursors_set && n >= 4u * TRACE_WAVE * (uint32_t)a->grid_occl;
+    const bool many_occl = anyhit && !n_dev && n >= 4u * TRACE_WAVE * (uint32_t)a->grid_occl;
     const int grid = trace_grid(a, n_max, many_occl);
     const uint32_t node_bytes = (uint32_t)(a->host.nodes.size() * sizeof(WNode));   // < 4 GB, the builder's bound
     // a count the host knows goes with the launch, and when the fixed chunks
     // cover the rays no wave reads a cursor
-    const uint32_t n_fixed = n_dev ? 0u : n;
-    if (!cursors_set && (n_dev || trace_has_dynamic(n, (uint32_t)grid)))
-        k_init_cursors<<<1, 64, 0, s>>>(counters, n, n_dev, (uint32_t)grid);
+    if (!cursors_clear && (n_dev || trace_has_dynamic(n, (uint32_t)grid))) k_clear_cursors<<<1, 64, 0, s>>>(counters);
     // the list words of coop_trace hold 28-bit indices
     const uint32_t coop_max =
         a->host.nodes.size() <= (1u << COOP_TAG_SHIFT) && a->host.tris.size() <= (1u << COOP_TAG_SHIFT) ? COOP_RAYS : 0u;
     const bool wt = a->host.isect == WBVH_ISECT_WATERTIGHT;
     auto launch = [&](auto kernel) {
         kernel<<<grid, TRACE_WAVE, a->lds_bytes, s>>>(a->d_nodes, a->d_tris, rays, hits, counters, overflow,
-                                                      a->stack_depth, REFILL_MIN, node_bytes, n_fixed, coop_max);
+                                                      a->stack_depth, REFILL_MIN, node_bytes, n, n_dev, coop_max);
     };
     if (wt && !anyhit) launch(k_trace<WBVH_ISECT_WATERTIGHT, false>);
     else if (wt) launch(k_trace<WBVH_ISECT_WATERTIGHT, true>);
@@ -1021,20 +1017,18 @@ static int enqueue_trace(const lmx_accel* a, uint32_t* counters, const WRay* ray
 }
 
 int launch_trace(lmx_accel* a, const WRay* rays, uint32_t n, const uint32_t* n_dev, uint32_t n_max,
-                 WHit* hits, hipStream_t s, bool anyhit, bool cursors_set)
+                 WHit* hits, hipStream_t s, bool anyhit, bool cursors_clear)
 {
     int rc = lmx_accel_upload(a);
     if (rc != LMX_OK) return rc;
-    return enqueue_trace(a, a->d_counters, rays, n, n_dev, n_max, hits, s, anyhit, cursors_set);
+    return enqueue_trace(a, a->d_counters, rays, n, n_dev, n_max, hits, s, anyhit, cursors_clear);
 }
 
-int trace_shape(lmx_accel* a, uint32_t n_max, uint32_t** counters, uint32_t* grid)
+int trace_counters(lmx_accel* a, uint32_t** counters)
 {
-    int rc = lmx_accel_upload(a);
-    if (rc != LMX_OK) return rc;
-    *counters = a->d_counters;
-    *grid = (uint32_t)trace_grid(a, n_max);
-    return LMX_OK;
+    const int rc = lmx_accel_upload(a);
+    if (rc == LMX_OK) *counters = a->d_counters;
+    return rc;
 }
 
 }  // namespace lmx
@@ -1043,12 +1037,11 @@ int trace_shape(lmx_accel* a, uint32_t n_max, uint32_t** counters, uint32_t* gri
 // Allocation-free closest hit (lmx_accel_intersect_noalloc)
 //
 // The same launch as lmx_accel_intersect, with the launch's scratch -- the 8
-// region cursors and the ray count, each on a 256-byte line of its own,
-// 2,304 bytes, whatever the number of rays -- in this file-scope array
+// region cursors, each on a 256-byte line of its own, in 2,304 bytes,
+// whatever the number of rays -- in this file-scope array
 // instead of the accel's counter block.  Every GPU the library runs on holds
 // its own copy until the process ends, shared by every call on that GPU;
-// k_init_cursors rewrites all 9 words at the start of each launch that reads
-// them, so no value carries over from the previous call (two calls that overlap on one
+// k_clear_cursors clears them before each launch that reads them, so no value carries over from the previous call (two calls that overlap on one
 // GPU, on different streams, race on it).  On the host, `scratch` only
 // stands in for the device symbol: its device address comes from
 // hipGetSymbolAddress, taken once per device with that device current, and

@@ -34,7 +34,7 @@
 // Per batch of B samples:
 //   gen      -- the eye and light endpoints of every sample and their first
 //               rays, into one queue;
-//   (trace, shade, commit) x (max_vertices - 1)
+//   (trace, shade) x (max_vertices - 1)
 //            -- subpaths of both directions advance together in one queue, so
 //               paths of every length and direction share each launch; every
 //               vertex is stored with its throughput and with the area pdfs
@@ -61,6 +61,7 @@
 #include "lmx_internal.h"
 #include "rmath.h"
 #include "rshade.h"
+#include "trace_cursors.h"
 #include "wbvh.h"
 
 using namespace lmx;
@@ -123,10 +124,10 @@ struct BParams {
 
 // Measurement hook: copies the n rays about to be traced to out[at, ...),
 // within [lo, hi) (the slot of BCtl::cap_n[kind] counts them).
-__global__ void k_bd_capture(BCtl* __restrict__ ctl, int kind, const float4* __restrict__ ray, float4* __restrict__ out,
+__global__ void k_bd_capture(BCtl* __restrict__ ctl, int kind, int slot, const float4* __restrict__ ray, float4* __restrict__ out,
                              uint32_t lo, uint32_t hi)
 {
-    const uint32_t n = kind == 0 ? ctl->n_trace : ctl->n_shadow;
+    const uint32_t n = kind == 0 ? ctl->n_q[slot] : ctl->n_shadow;
     const uint32_t at = lo + ctl->cap_n[kind];
     const uint32_t m = at >= hi ? 0u : min(n, hi - at);
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < m; i += gridDim.x * blockDim.x) {
@@ -135,9 +136,9 @@ __global__ void k_bd_capture(BCtl* __restrict__ ctl, int kind, const float4* __r
     }
 }
 
-__global__ void k_bd_capture_advance(BCtl* ctl, int kind, uint32_t room)
+__global__ void k_bd_capture_advance(BCtl* ctl, int kind, int slot, uint32_t room)
 {
-    if (threadIdx.x == 0) ctl->cap_n[kind] = min(room, ctl->cap_n[kind] + (kind == 0 ? ctl->n_trace : ctl->n_shadow));
+    if (threadIdx.x == 0) ctl->cap_n[kind] = min(room, ctl->cap_n[kind] + (kind == 0 ? ctl->n_q[slot] : ctl->n_shadow));
 }
 
 struct VB {
@@ -246,8 +247,12 @@ RD uint32_t rb_step(uint32_t j) { return LMX_PT_SLOT_SEG0 + 8u * (j - 1u); }
 
 // ---------------------------------------------------------------------------
 
-__global__ __launch_bounds__(256) void k_bd_gen(RScene s, BParams p, BCtl* __restrict__ ctl, VB vb, Queue q)
+// Endpoints and first rays of a batch (ctl->n_q is 0 at its start); clears the
+// cursors of the first trace launch.
+__global__ __launch_bounds__(256) void k_bd_gen(RScene s, BParams p, BCtl* __restrict__ ctl, VB vb, Queue q,
+                                                uint32_t* __restrict__ cursors)
 {
+    if (blockIdx.x == 0) trace_cursors_clear(cursors, threadIdx.x);
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t sample = ctl->batch_first + i;
     const bool valid = i < p.batch && sample - ctl->pass_first < p.total;
@@ -326,7 +331,7 @@ __global__ __launch_bounds__(256) void k_bd_gen(RScene s, BParams p, BCtl* __res
         vb.nsub[1][i] = 0;
     }
     __shared__ uint32_t lds[5];
-    const uint32_t se = block_reserve<4>(&ctl->n_trace, (uint32_t)eye_ray + (uint32_t)light_ray, lds);
+    const uint32_t se = block_reserve<4>(&ctl->n_q[0], (uint32_t)eye_ray + (uint32_t)light_ray, lds);
     const uint32_t sl = se + (uint32_t)eye_ray;
     if (eye_ray) {
         q.ray[2 * se] = make_float4(s.cam_pos.x, s.cam_pos.y, s.cam_pos.z, LMX_EPS_ISECT);
@@ -343,12 +348,23 @@ __global__ __launch_bounds__(256) void k_bd_gen(RScene s, BParams p, BCtl* __res
 }
 
 __global__ __launch_bounds__(256) void k_bd_shade(RScene s, BParams p, BCtl* __restrict__ ctl, Queue in,
-                                                  const float4* __restrict__ hits, Queue out, VB vb)
+                                                  const float4* __restrict__ hits, Queue out, VB vb, int it,
+                                                  uint32_t* __restrict__ cursors)
 {
     // one thread per queue entry (the grid covers the queue's capacity;
-    // workgroups past the current count leave at once)
+    // workgroups past the current count leave at once).  Workgroup 0 ends the
+    // iteration: it clears the count that the next shade step appends to and
+    // the next trace launch's cursors, so no kernel is needed between them.
     __shared__ uint32_t lds[5];
-    const uint32_t n = ctl->n_trace;
+    const uint32_t n = ctl->n_q[it % 3];
+    uint32_t* n_next = &ctl->n_q[(it + 1) % 3];
+    if (blockIdx.x == 0) {
+        trace_cursors_clear(cursors, threadIdx.x);
+        if (threadIdx.x == 64) {
+            ctl->n_q[(it + 2) % 3] = 0u;
+            ctl->rays += n;
+        }
+    }
     {
         const uint32_t base = blockIdx.x * blockDim.x;
         if (base >= n) return;
@@ -439,22 +455,13 @@ __global__ __launch_bounds__(256) void k_bd_shade(RScene s, BParams p, BCtl* __r
                 }
             }
         }
-        const uint32_t slot = block_reserve<4>(&ctl->n_next, cont ? 1u : 0u, lds);
+        const uint32_t slot = block_reserve<4>(n_next, cont ? 1u : 0u, lds);
         if (cont) {
             out.ray[2 * slot] = o0;
             out.ray[2 * slot + 1] = o1;
             out.thr[slot] = ot;
             out.meta[slot] = om;
         }
-    }
-}
-
-__global__ void k_bd_commit(BCtl* ctl)
-{
-    if (threadIdx.x == 0) {
-        ctl->rays += ctl->n_trace;
-        ctl->n_trace = ctl->n_next;
-        ctl->n_next = 0;
     }
 }
 
@@ -826,9 +833,12 @@ __global__ __launch_bounds__(256) void k_bd_plan(RScene s, BParams p, BCtl* __re
 // possible.  The offsets are non-decreasing and no sample needs more than
 // cap slots, so every round takes at least one sample while any remain.
 // One wave: a 64-way search, each level probing 64 indices at once.
-__global__ void k_bd_round(BCtl* ctl, const uint32_t* __restrict__ off, uint32_t batch, uint32_t cap)
+// It also clears the cursors of the round's trace launch.
+__global__ void k_bd_round(BCtl* ctl, const uint32_t* __restrict__ off, uint32_t batch, uint32_t cap,
+                           uint32_t* __restrict__ cursors)
 {
     const uint32_t lane = threadIdx.x;
+    trace_cursors_clear(cursors, lane);
     const uint32_t lo = ctl->conn_next;
     if (lo >= batch) {
         if (lane == 0) { ctl->n_shadow = 0; ctl->conn_lo = batch; ctl->conn_hi = batch; }
@@ -1018,7 +1028,7 @@ __global__ void k_bd_next_batch(BCtl* ctl, uint32_t batch)
 {
     if (threadIdx.x == 0) {
         ctl->batch_first += batch;
-        ctl->n_trace = 0; ctl->n_next = 0; ctl->n_shadow = 0; ctl->n_mq = 0;
+        ctl->n_q[0] = ctl->n_q[1] = ctl->n_q[2] = 0; ctl->n_shadow = 0; ctl->n_mq = 0;
     }
 }
 
@@ -1031,7 +1041,7 @@ __global__ void k_bd_init(BCtl* ctl)
 {
     if (threadIdx.x == 0) {
         ctl->conn_next = 0; ctl->conn_lo = 0; ctl->conn_hi = 0; ctl->conn_base = 0;
-        ctl->n_trace = 0; ctl->n_next = 0; ctl->n_shadow = 0; ctl->batch_first = 0;
+        ctl->n_q[0] = ctl->n_q[1] = ctl->n_q[2] = 0; ctl->n_shadow = 0; ctl->batch_first = 0;
         ctl->rays = 0; ctl->shadow_rays = 0;
         ctl->pass_first = 0; ctl->radius = 0.0f; ctl->cell = 0.0f; ctl->c_merge = 0.0f; ctl->merges = 0; ctl->dropped = 0; ctl->cap_n[0] = 0; ctl->cap_n[1] = 0;
         ctl->n_mq = 0;
@@ -1043,7 +1053,7 @@ __global__ void k_bd_init(BCtl* ctl)
 __global__ void k_bd_phase(BCtl* ctl, uint32_t first, float radius, float cell, float c_merge)
 {
     if (threadIdx.x == 0) {
-        ctl->n_trace = 0; ctl->n_next = 0; ctl->n_shadow = 0; ctl->n_mq = 0;
+        ctl->n_q[0] = ctl->n_q[1] = ctl->n_q[2] = 0; ctl->n_shadow = 0; ctl->n_mq = 0;
         ctl->batch_first = first; ctl->pass_first = first;
         ctl->radius = radius; ctl->cell = cell; ctl->c_merge = c_merge;
     }
@@ -1702,7 +1712,7 @@ __global__ __launch_bounds__(SPLAT_THREADS) void k_lt_splat(BParams p, BCtl* __r
 __global__ void k_lt_batch(BCtl* ctl, uint32_t first)
 {
     if (threadIdx.x == 0) {
-        ctl->n_trace = 0; ctl->n_next = 0; ctl->n_shadow = 0;
+        ctl->n_q[0] = ctl->n_q[1] = ctl->n_q[2] = 0; ctl->n_shadow = 0;
         ctl->batch_first = first;
     }
 }
@@ -1875,6 +1885,32 @@ int bd_buffers(lmx_scene* sc, uint32_t B, uint32_t maxv, uint32_t conn, bool rou
     return LMX_OK;
 }
 
+// Records the subpaths of one batch of `bp` samples into vb's vertex records:
+// the endpoints, then bp.maxv - 1 times trace and shade, over queues of at
+// most `cap` rays.
+int bd_enqueue_subpaths(lmx_scene* sc, const BParams& bp, const VB& vb, const Queue (&q)[2], float4* hits, uint32_t cap,
+                        hipStream_t st)
+{
+    BCtl* ctl = sc->bd_ctl.p;
+    uint32_t* cursors = nullptr;
+    int rc = trace_counters(sc->accel, &cursors);
+    if (rc != LMX_OK) return rc;
+    k_bd_gen<<<(bp.batch + 255) / 256, 256, 0, st>>>(sc->rs, bp, ctl, vb, q[0], cursors);
+    const uint32_t half = bp.ray_out_cap / 2;
+    for (int it = 0; it < bp.maxv - 1; it++) {
+        const int a = it & 1;
+        if (bp.ray_out) {
+            k_bd_capture<<<sc->cus * 8, 256, 0, st>>>(ctl, 0, it % 3, q[a].ray, bp.ray_out, 0u, half);
+            k_bd_capture_advance<<<1, 64, 0, st>>>(ctl, 0, it % 3, half);
+        }
+        rc = launch_trace(sc->accel, reinterpret_cast<const WRay*>(q[a].ray), 0, &ctl->n_q[it % 3], cap,
+                          reinterpret_cast<WHit*>(hits), st, false, true);
+        if (rc != LMX_OK) return rc;
+        k_bd_shade<<<(cap + 255) / 256, 256, 0, st>>>(sc->rs, bp, ctl, q[a], hits, q[1 - a], vb, it, cursors);
+    }
+    return LMX_OK;
+}
+
 // Records one connection round: the next range of samples whose slots fit
 // the shadow queue, their slots, the connection terms, the any-hit trace of
 // the shadow rays, and the splat of the unoccluded ones.  A round with no
@@ -1885,16 +1921,19 @@ int bd_enqueue_round(lmx_scene* sc, const BParams& bp, const VB& vb, hipStream_t
     const int cap_grid = sc->cus * 8;
     const uint32_t nconn = sc->bd_nconn;
     ShadowQ sq{sc->bd_sray.p, sc->bd_sc.p, sc->bd_saux.p, sc->bd_smeta.p};
-    k_bd_round<<<1, 64, 0, st>>>(ctl, vb.off, bp.batch, nconn);
+    uint32_t* cursors = nullptr;
+    int rc = trace_counters(sc->accel, &cursors);
+    if (rc != LMX_OK) return rc;
+    k_bd_round<<<1, 64, 0, st>>>(ctl, vb.off, bp.batch, nconn, cursors);
     k_bd_slots<<<cap_grid, 256, 0, st>>>(sc->rs, bp, ctl, vb, sq);
     k_bd_connect<<<cap_grid, 256, 0, st>>>(sc->rs, bp, ctl, vb, sq);
     if (bp.ray_out) {
         const uint32_t half = bp.ray_out_cap / 2;
-        k_bd_capture<<<cap_grid, 256, 0, st>>>(ctl, 1, sq.ray, bp.ray_out, half, bp.ray_out_cap);
-        k_bd_capture_advance<<<1, 64, 0, st>>>(ctl, 1, bp.ray_out_cap - half);
+        k_bd_capture<<<cap_grid, 256, 0, st>>>(ctl, 1, 0, sq.ray, bp.ray_out, half, bp.ray_out_cap);
+        k_bd_capture_advance<<<1, 64, 0, st>>>(ctl, 1, 0, bp.ray_out_cap - half);
     }
-    int rc = launch_trace(sc->accel, reinterpret_cast<const WRay*>(sq.ray), 0, &ctl->n_shadow, nconn,
-                          reinterpret_cast<WHit*>(sc->bd_shits.p), st, true);
+    rc = launch_trace(sc->accel, reinterpret_cast<const WRay*>(sq.ray), 0, &ctl->n_shadow, nconn,
+                      reinterpret_cast<WHit*>(sc->bd_shits.p), st, true, true);
     if (rc != LMX_OK) return rc;
     k_bd_splat<<<std::max(1, std::min((int)((nconn + SPLAT_THREADS - 1) / SPLAT_THREADS), sc->cus)), SPLAT_THREADS, 0,
                  st>>>(bp, ctl, sq, sc->bd_shits.p);
@@ -1927,21 +1966,8 @@ int bd_enqueue_batch(lmx_scene* sc, const BParams& bp, hipStream_t st)
     for (int k = 0; k < 2; k++) { q[k].ray = sc->bd_ray[k].p; q[k].thr = sc->bd_thr[k].p; q[k].meta = sc->bd_meta[k].p; }
     BCtl* ctl = sc->bd_ctl.p;
     const int cap_grid = sc->cus * 8;
-    k_bd_gen<<<(B + 255) / 256, 256, 0, st>>>(sc->rs, bp, ctl, vb, q[0]);
-    int a = 0;
-    const uint32_t half = bp.ray_out_cap / 2;
-    for (int it = 0; it < bp.maxv - 1; it++) {
-        if (bp.ray_out) {
-            k_bd_capture<<<cap_grid, 256, 0, st>>>(ctl, 0, q[a].ray, bp.ray_out, 0u, half);
-            k_bd_capture_advance<<<1, 64, 0, st>>>(ctl, 0, half);
-        }
-        int rc = launch_trace(sc->accel, reinterpret_cast<const WRay*>(q[a].ray), 0, &ctl->n_trace, 2 * B,
-                              reinterpret_cast<WHit*>(sc->bd_hits.p), st, false);
-        if (rc != LMX_OK) return rc;
-        k_bd_shade<<<(2 * B + 255) / 256, 256, 0, st>>>(sc->rs, bp, ctl, q[a], sc->bd_hits.p, q[1 - a], vb);
-        k_bd_commit<<<1, 64, 0, st>>>(ctl);
-        a = 1 - a;
-    }
+    int rc = bd_enqueue_subpaths(sc, bp, vb, q, sc->bd_hits.p, 2 * B, st);
+    if (rc != LMX_OK) return rc;
     k_bd_plan<<<(B + 255) / 256, 256, 0, st>>>(sc->rs, bp, ctl, vb);
     // connection counts -> slot offsets; off[B] becomes the batch's total
     const uint32_t nt = (B + 1 + SCAN_TILE - 1) / SCAN_TILE;
@@ -1953,8 +1979,7 @@ int bd_enqueue_batch(lmx_scene* sc, const BParams& bp, hipStream_t st)
     k_bd_conn_start<<<1, 64, 0, st>>>(ctl);
     const int rounds = bd_graph_rounds(sc, bp);
     for (int k = 0; k < rounds; k++) {
-        const int rc = bd_enqueue_round(sc, bp, vb, st);
-        if (rc != LMX_OK) return rc;
+        if ((rc = bd_enqueue_round(sc, bp, vb, st)) != LMX_OK) return rc;
     }
     if (bp.merging) {
         VB ph = vb;
@@ -2300,16 +2325,8 @@ int vc_enqueue_photons(lmx_scene* sc, const BParams& pp, hipStream_t st, bool gr
     for (int k = 0; k < 2; k++) { q[k].ray = sc->vc_ray[k].p; q[k].thr = sc->vc_thr[k].p; q[k].meta = sc->vc_meta[k].p; }
     BCtl* ctl = sc->bd_ctl.p;
     const int cap_grid = sc->cus * 8;
-    k_bd_gen<<<(np + 255) / 256, 256, 0, st>>>(sc->rs, pp, ctl, ph, q[0]);
-    int a = 0;
-    for (int it = 0; it < pp.maxv - 1; it++) {
-        int rc = launch_trace(sc->accel, reinterpret_cast<const WRay*>(q[a].ray), 0, &ctl->n_trace, np,
-                              reinterpret_cast<WHit*>(sc->vc_hits.p), st, false);
-        if (rc != LMX_OK) return rc;
-        k_bd_shade<<<(np + 255) / 256, 256, 0, st>>>(sc->rs, pp, ctl, q[a], sc->vc_hits.p, q[1 - a], ph);
-        k_bd_commit<<<1, 64, 0, st>>>(ctl);
-        a = 1 - a;
-    }
+    const int rc = bd_enqueue_subpaths(sc, pp, ph, q, sc->vc_hits.p, np, st);
+    if (rc != LMX_OK) return rc;
     if (!grid) {
         const hipError_t e = hipGetLastError();
         return e == hipSuccess ? LMX_OK : hip_error(e, "photon launch");
@@ -2479,16 +2496,8 @@ int pm_enqueue_eye(lmx_scene* sc, const BParams& bp, const PMArgs& pa, hipStream
     for (int k = 0; k < 2; k++) { q[k].ray = sc->bd_ray[k].p; q[k].thr = sc->bd_thr[k].p; q[k].meta = sc->bd_meta[k].p; }
     BCtl* ctl = sc->bd_ctl.p;
     const int cap_grid = sc->cus * 8;
-    k_bd_gen<<<(B + 255) / 256, 256, 0, st>>>(sc->rs, bp, ctl, vb, q[0]);
-    int a = 0;
-    for (int it = 0; it < bp.maxv - 1; it++) {
-        int rc = launch_trace(sc->accel, reinterpret_cast<const WRay*>(q[a].ray), 0, &ctl->n_trace, B,
-                              reinterpret_cast<WHit*>(sc->bd_hits.p), st, false);
-        if (rc != LMX_OK) return rc;
-        k_bd_shade<<<(B + 255) / 256, 256, 0, st>>>(sc->rs, bp, ctl, q[a], sc->bd_hits.p, q[1 - a], vb);
-        k_bd_commit<<<1, 64, 0, st>>>(ctl);
-        a = 1 - a;
-    }
+    const int rc = bd_enqueue_subpaths(sc, bp, vb, q, sc->bd_hits.p, B, st);
+    if (rc != LMX_OK) return rc;
     const Grid g{sc->vc_items.p, sc->vc_start.p, sc->vc_cursor.p, sc->vc_part.p, sc->vc_H};
     k_pm_gather<<<std::max(1, std::min((int)((B + 255) / 256), cap_grid * 2)), 256, 0, st>>>(sc->rs, bp, ctl, vb,
                                                                                              ph, g, pa);
@@ -2695,13 +2704,8 @@ int render_ppm(lmx_scene* sc, const lmx_render_params* p, const lmx_ppm_params* 
         // the measurement points: endpoints and the first hit of every sample
         Queue q[2];
         for (int k = 0; k < 2; k++) { q[k].ray = sc->bd_ray[k].p; q[k].thr = sc->bd_thr[k].p; q[k].meta = sc->bd_meta[k].p; }
-        BCtl* ctl = sc->bd_ctl.p;
-        k_bd_gen<<<(N + 255) / 256, 256, 0, st>>>(sc->rs, bp, ctl, vb, q[0]);
-        rc = launch_trace(sc->accel, reinterpret_cast<const WRay*>(q[0].ray), 0, &ctl->n_trace, N,
-                          reinterpret_cast<WHit*>(sc->bd_hits.p), st, false);
+        rc = bd_enqueue_subpaths(sc, bp, vb, q, sc->bd_hits.p, N, st);
         if (rc == LMX_OK) {
-            k_bd_shade<<<(N + 255) / 256, 256, 0, st>>>(sc->rs, bp, ctl, q[0], sc->bd_hits.p, q[1], vb);
-            k_bd_commit<<<1, 64, 0, st>>>(ctl);
             k_ppm_init<<<mgrid, 256, 0, st>>>(sc->rs, bp, vb, sc->ppm_st.p, r0);
             if ((e = hipGetLastError()) != hipSuccess) rc = hip_error(e, "ppm launch");
         }
@@ -2822,13 +2826,8 @@ int render_sppm(lmx_scene* sc, const lmx_render_params* p, const lmx_ppm_params*
         rc = capture(st, &geye, [&] {
             Queue q[2];
             for (int k = 0; k < 2; k++) { q[k].ray = sc->bd_ray[k].p; q[k].thr = sc->bd_thr[k].p; q[k].meta = sc->bd_meta[k].p; }
-            BCtl* ctl = sc->bd_ctl.p;
-            k_bd_gen<<<(npix + 255) / 256, 256, 0, st>>>(sc->rs, bp, ctl, vb, q[0]);
-            int rc2 = launch_trace(sc->accel, reinterpret_cast<const WRay*>(q[0].ray), 0, &ctl->n_trace, npix,
-                                   reinterpret_cast<WHit*>(sc->bd_hits.p), st, false);
+            const int rc2 = bd_enqueue_subpaths(sc, bp, vb, q, sc->bd_hits.p, npix, st);
             if (rc2 != LMX_OK) return rc2;
-            k_bd_shade<<<(npix + 255) / 256, 256, 0, st>>>(sc->rs, bp, ctl, q[0], sc->bd_hits.p, q[1], vb);
-            k_bd_commit<<<1, 64, 0, st>>>(ctl);
             const hipError_t e2 = hipGetLastError();
             return e2 == hipSuccess ? LMX_OK : hip_error(e2, "sppm launch");
         });
@@ -2935,7 +2934,7 @@ int render_ltdirect(lmx_scene* sc, const lmx_render_params* p, float* film_rgb, 
             const int g = std::max(1, (int)std::min<size_t>((nslot + 255) / 256, (size_t)cap_grid * 2));
             k_lt_connect<<<g, 256, 0, st>>>(sc->rs, pp, ctl, ph, sq, bounded ? p->max_num_vertices : -1);
             rc2 = launch_trace(sc->accel, reinterpret_cast<const WRay*>(sq.ray), 0, &ctl->n_shadow, (uint32_t)nslot,
-                               reinterpret_cast<WHit*>(sc->bd_shits.p), st, true);
+                               reinterpret_cast<WHit*>(sc->bd_shits.p), st, true, true);   // cleared by the last shade
             if (rc2 != LMX_OK) return rc2;
             const int gs = std::max(1, (int)std::min<size_t>((nslot + SPLAT_THREADS - 1) / SPLAT_THREADS, (size_t)sc->cus));
             k_lt_splat<<<gs, SPLAT_THREADS, 0, st>>>(pp, ctl, sq, sc->bd_shits.p, (int32_t)pcap);

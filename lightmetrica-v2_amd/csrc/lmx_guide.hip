@@ -911,7 +911,7 @@ namespace {
 // (224 VGPRs: two waves per SIMD)
 constexpr int GS_WAVES = 8;
 __global__ __launch_bounds__(GS_WAVES * 64) void k_guided_shade(RScene s, RParams p, GuideLaunch gl,
-                                                                  Ctl* __restrict__ ctl, Queue in,
+                                                                  Ctl* __restrict__ ctl, int qa, Queue in,
                                                                   const float4* __restrict__ hits, Queue out)
 {
     __shared__ bf16x8 wl[N_FWD];
@@ -923,7 +923,7 @@ __global__ __launch_bounds__(GS_WAVES * 64) void k_guided_shade(RScene s, RParam
     __syncthreads();
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     NoSink dummy;
-    const uint32_t n = ctl->n_trace;
+    const uint32_t n = ctl->n_trace[qa];
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += stride) {
         const uint32_t i = base + threadIdx.x;
@@ -1028,7 +1028,7 @@ __global__ __launch_bounds__(GS_WAVES * 64) void k_guided_shade(RScene s, RParam
                 }
             }
         }
-        const uint32_t slot = block_reserve<GS_WAVES>(&ctl->n_next, cont ? 1u : 0u, lds);
+        const uint32_t slot = block_reserve<GS_WAVES>(&ctl->n_app[1 - qa], cont ? 1u : 0u, lds);
         if (cont) {
             out.ray[2 * slot] = o_ray0;
             out.ray[2 * slot + 1] = o_ray1;
@@ -1051,10 +1051,10 @@ __global__ __launch_bounds__(GS_WAVES * 64) void k_guided_shade(RScene s, RParam
 
 }  // namespace
 
-int launch_guided_shade(lmx_scene* sc, const RParams& rp, Queue qa, Queue qb, hipStream_t st)
+int launch_guided_shade(lmx_scene* sc, const RParams& rp, Queue qa, Queue qb, int a, hipStream_t st)
 {
     const int grid = std::max(1, std::min((int)((sc->cap + GS_WAVES * 64 - 1) / (GS_WAVES * 64)), sc->cus));
-    k_guided_shade<<<grid, GS_WAVES * 64, 0, st>>>(sc->rs, rp, *rp.guide, sc->ctl.p, qa, sc->hits.p, qb);
+    k_guided_shade<<<grid, GS_WAVES * 64, 0, st>>>(sc->rs, rp, *rp.guide, sc->ctl.p, a, qa, sc->hits.p, qb);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? LMX_OK : hip_error(e, "guided shade launch");
 }

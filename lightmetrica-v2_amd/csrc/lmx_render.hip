@@ -12,8 +12,8 @@
 //              atomic per wave (ballot + mbcnt), so the queue stays dense
 //              whatever the path lengths,
 //   gen     -- new camera paths fill the free capacity, so paths of all
-//              lengths share every launch,
-//   commit  -- one thread swaps the queue counts.
+//              lengths share every launch; one workgroup sets the next
+//              iteration's counts.
 // Two iterations (A->B, B->A) are captured once in a hipGraph and replayed;
 // every count lives on the device, so nothing waits for the host between
 // iterations.
@@ -106,10 +106,10 @@ RD NeeOut nee_connect(const RScene& s, const RParams& p, bool camera, const Fram
     return o;
 }
 
-RD void nee_append(const RParams& p, Ctl* ctl, uint32_t* lds, const NeeOut& o, uint32_t sample, uint32_t pixel,
+RD void nee_append(const RParams& p, uint32_t* n_shadow, uint32_t* lds, const NeeOut& o, uint32_t sample, uint32_t pixel,
                    bool camera)
 {
-    const uint32_t slot = block_reserve<4>(&ctl->n_shadow, o.emit ? 1u : 0u, lds);
+    const uint32_t slot = block_reserve<4>(n_shadow, o.emit ? 1u : 0u, lds);
     if (o.emit) {
         p.nq.ray[2 * slot] = o.r0;
         p.nq.ray[2 * slot + 1] = o.r1;
@@ -131,13 +131,13 @@ RD uint32_t shade_class(const RScene& s, uint32_t id, bool dead)
     return t == LMX_MAT_DIFFUSE ? 1u : (t == LMX_MAT_PHONG ? 2u : (t == LMX_MAT_GGX ? 3u : 0u));
 }
 
-__global__ __launch_bounds__(256) void k_bin(RScene s, Ctl* __restrict__ ctl, const uint4* __restrict__ meta,
+__global__ __launch_bounds__(256) void k_bin(RScene s, Ctl* __restrict__ ctl, int a, const uint4* __restrict__ meta,
                                              const float4* __restrict__ hits, uint32_t* __restrict__ perm,
                                              uint32_t cap)
 {
     __shared__ uint32_t wcount[SHADE_CLASSES][4];
     __shared__ uint32_t wbase[SHADE_CLASSES][4];
-    const uint32_t n = ctl->n_trace;
+    const uint32_t n = ctl->n_trace[a];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x) {
         const uint32_t i = base + threadIdx.x;
@@ -168,11 +168,11 @@ __global__ void k_bin_clear(Ctl* ctl)
     if (threadIdx.x < SHADE_CLASSES) ctl->bin[threadIdx.x] = 0;
 }
 
-__global__ __launch_bounds__(256) void k_shade(RScene s, RParams p, Ctl* __restrict__ ctl, Queue in,
+__global__ __launch_bounds__(256) void k_shade(RScene s, RParams p, Ctl* __restrict__ ctl, int a, Queue in,
                                                const float4* __restrict__ hits, Queue out)
 {
     __shared__ uint32_t lds[5];
-    const uint32_t n = ctl->n_trace;
+    const uint32_t n = ctl->n_trace[a];
     const uint32_t stride = gridDim.x * blockDim.x;
     uint32_t bend[SHADE_CLASSES];                    // class ranges in the binned order
     if (p.perm) {
@@ -264,30 +264,40 @@ __global__ __launch_bounds__(256) void k_shade(RScene s, RParams p, Ctl* __restr
                 }
             }
         }
-        const uint32_t slot = block_reserve<4>(&ctl->n_next, cont ? 1u : 0u, lds);
+        const uint32_t slot = block_reserve<4>(&ctl->n_app[1 - a], cont ? 1u : 0u, lds);
         if (cont) {
             out.ray[2 * slot] = o_ray0;
             out.ray[2 * slot + 1] = o_ray1;
             out.thr[slot] = o_thr;
             out.meta[slot] = o_meta;
         }
-        if (p.nee != NEE_NONE) nee_append(p, ctl, lds, no, no_sample, no_pixel, false);
+        if (p.nee != NEE_NONE) nee_append(p, &ctl->n_shadow[1 - a], lds, no, no_sample, no_pixel, false);
     }
 }
 
-RD uint32_t gen_count(const Ctl* ctl, uint32_t cap, uint32_t total)
-{
-    if (ctl->stop) return 0;
-    const uint32_t free_slots = cap - ctl->n_next;
-    const uint32_t left = total - ctl->issued;
-    return free_slots < left ? free_slots : left;
-}
-
-__global__ __launch_bounds__(256) void k_gen(RScene s, RParams p, Ctl* __restrict__ ctl, uint32_t cap, Queue out)
+// Fills queue b, to which shading queue a's paths appended n_app[b], with
+// camera paths, and ends the iteration: workgroup 0 sets the counts of the
+// next one and clears the next trace launch's cursors (no trace runs beside
+// this kernel).
+__global__ __launch_bounds__(256) void k_gen(RScene s, RParams p, Ctl* __restrict__ ctl, uint32_t cap, int b, Queue out,
+                                             uint32_t* __restrict__ cursors)
 {
     __shared__ uint32_t lds[5];
-    const uint32_t want = gen_count(ctl, cap, p.total);
-    const uint32_t base_slot = ctl->n_next, first = ctl->issued;
+    const int a = 1 - b;
+    const uint32_t base_slot = ctl->n_app[b], first = ctl->issued[a];
+    const uint32_t want = ctl->stop ? 0u : min(cap - base_slot, p.total - first);
+    if (blockIdx.x == 0) {
+        trace_cursors_clear(cursors, threadIdx.x);
+        if (threadIdx.x == 64) {
+            ctl->rays += ctl->n_trace[a];
+            ctl->shadow_rays += ctl->n_shadow[a];
+            ctl->n_trace[b] = base_slot + want;
+            ctl->issued[b] = first + want;
+            ctl->n_app[a] = 0;
+            ctl->n_shadow[a] = 0;
+            ctl->iterations += 1;
+        }
+    }
     // workgroup-uniform loop: the camera-vertex connections append per workgroup
     for (uint32_t base = blockIdx.x * blockDim.x; base < want; base += gridDim.x * blockDim.x) {
         const uint32_t t = base + threadIdx.x;
@@ -340,14 +350,17 @@ __global__ __launch_bounds__(256) void k_gen(RScene s, RParams p, Ctl* __restric
                 if (no.emit) pixel = raster_pixel(s, no.rx, no.ry);
             }
         }
-        if (p.nee != NEE_NONE) nee_append(p, ctl, lds, no, sample, pixel, true);
+        if (p.nee != NEE_NONE) nee_append(p, &ctl->n_shadow[b], lds, no, sample, pixel, true);
     }
 }
 
-// Splats the unoccluded next-event connections of the iteration.
-__global__ __launch_bounds__(256) void k_nee_splat(RParams p, Ctl* __restrict__ ctl)
+// Splats the unoccluded next-event connections of the iteration that filled
+// queue b, and clears the cursors their trace used.
+__global__ __launch_bounds__(256) void k_nee_splat(RParams p, const Ctl* __restrict__ ctl, int b,
+                                                   uint32_t* __restrict__ cursors)
 {
-    const uint32_t n = ctl->n_shadow;
+    if (blockIdx.x == 0) trace_cursors_clear(cursors, threadIdx.x);
+    const uint32_t n = ctl->n_shadow[b];
     for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
         if (__float_as_uint(p.nq.hits[j].w) != WBVH_MISS) continue;          // occluded
         const float4 c = p.nq.c[j];
@@ -366,41 +379,23 @@ __global__ __launch_bounds__(256) void k_nee_splat(RParams p, Ctl* __restrict__ 
     }
 }
 
-// Commits the generation: the queue just written becomes the one to trace.
-// Also sets the next trace launch's cursors (so that launch needs no cursor
-// kernel of its own), for `grid` workgroups.
-__global__ void k_commit(Ctl* ctl, uint32_t cap, uint32_t total, uint32_t* cursors, uint32_t grid)
-{
-    __shared__ uint32_t n_next;
-    if (threadIdx.x == 0) {
-        const uint32_t want = gen_count(ctl, cap, total);
-        ctl->shadow_rays += ctl->n_shadow;
-        ctl->n_shadow = 0;
-        ctl->rays += ctl->n_trace;
-        ctl->n_trace = ctl->n_next + want;
-        n_next = ctl->n_trace;
-        ctl->n_next = 0;
-        ctl->issued += want;
-        ctl->iterations += 1;
-    }
-    __syncthreads();
-    trace_cursors_set(cursors, n_next, grid, threadIdx.x);
-}
-
 __global__ void k_init_ctl(Ctl* ctl)
 {
     if (threadIdx.x == 0) {
-        ctl->n_trace = 0; ctl->n_next = 0; ctl->issued = 0; ctl->iterations = 0; ctl->rays = 0;
-        ctl->n_shadow = 0; ctl->shadow_rays = 0; ctl->stop = 0; ctl->ray_out_n = 0; ctl->film_scaled = 0;
+        for (int k = 0; k < 2; k++) {
+            ctl->n_trace[k] = 0; ctl->n_app[k] = 0; ctl->issued[k] = 0; ctl->n_shadow[k] = 0;
+        }
+        ctl->iterations = 0; ctl->rays = 0; ctl->shadow_rays = 0; ctl->stop = 0; ctl->ray_out_n = 0;
+        ctl->film_scaled = 0;
     }
 }
 
 // Measurement hook: copies the queue about to be traced (the first
 // ray_out_cap rays of the render, in launch order) out, then advances.
-__global__ void k_capture(const Ctl* __restrict__ ctl, const float4* __restrict__ ray, float4* __restrict__ out,
+__global__ void k_capture(const Ctl* __restrict__ ctl, int a, const float4* __restrict__ ray, float4* __restrict__ out,
                           uint32_t cap)
 {
-    const uint32_t n = ctl->n_trace, at = ctl->ray_out_n;
+    const uint32_t n = ctl->n_trace[a], at = ctl->ray_out_n;
     const uint32_t m = at >= cap ? 0u : min(n, cap - at);
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < m; i += gridDim.x * blockDim.x) {
         out[2 * (size_t)(at + i)] = ray[2 * (size_t)i];
@@ -408,9 +403,9 @@ __global__ void k_capture(const Ctl* __restrict__ ctl, const float4* __restrict_
     }
 }
 
-__global__ void k_capture_advance(Ctl* ctl, uint32_t cap)
+__global__ void k_capture_advance(Ctl* ctl, int a, uint32_t cap)
 {
-    if (threadIdx.x == 0) ctl->ray_out_n = min(cap, ctl->ray_out_n + ctl->n_trace);
+    if (threadIdx.x == 0) ctl->ray_out_n = min(cap, ctl->ray_out_n + ctl->n_trace[a]);
 }
 
 // Time mode: camera samples stop starting from the next iteration on.
@@ -435,7 +430,7 @@ __global__ void k_scale(float* a, size_t n, float w)
 // finds, so the host launches no scaling after it.
 __global__ void k_scale_done(Ctl* __restrict__ ctl, float* a, size_t n, uint32_t total, float w)
 {
-    const bool done = ctl->n_trace == 0 && ctl->issued >= total;
+    const bool done = ctl->n_trace[0] == 0 && ctl->issued[0] >= total;   // queue 0 was filled last
     if (blockIdx.x == 0 && threadIdx.x == 0) ctl->film_scaled = done ? 1u : 0u;
     if (!done) return;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) a[i] *= w;
@@ -483,14 +478,27 @@ int ensure_nee(lmx_scene* sc, uint32_t cap)
     return LMX_OK;
 }
 
-// The next-event connections of one iteration: any-hit trace, then splat.
-int enqueue_nee(lmx_scene* sc, const RParams& rp, hipStream_t st)
+// The next-event connections of the iteration that filled queue b: any-hit
+// trace, then splat.
+int enqueue_nee(lmx_scene* sc, const RParams& rp, int b, uint32_t* cursors, hipStream_t st)
 {
-    int rc = launch_trace(sc->accel, reinterpret_cast<const WRay*>(rp.nq.ray), 0, &sc->ctl.p->n_shadow,
-                          2 * sc->nee_cap, reinterpret_cast<WHit*>(rp.nq.hits), st, true);
+    int rc = launch_trace(sc->accel, reinterpret_cast<const WRay*>(rp.nq.ray), 0, &sc->ctl.p->n_shadow[b],
+                          2 * sc->nee_cap, reinterpret_cast<WHit*>(rp.nq.hits), st, true, true);   // cleared by k_gen
     if (rc != LMX_OK) return rc;
-    k_nee_splat<<<std::max(1, std::min((int)((2 * sc->nee_cap + 255) / 256), sc->cus * 8)), 256, 0, st>>>(rp, sc->ctl.p);
+    k_nee_splat<<<std::max(1, std::min((int)((2 * sc->nee_cap + 255) / 256), sc->cus * 8)), 256, 0, st>>>(
+        rp, sc->ctl.p, b, cursors);
     return LMX_OK;
+}
+
+// Records the generation that fills queue b, with its next-event connections.
+int enqueue_gen(lmx_scene* sc, const RParams& rp, int b, hipStream_t st)
+{
+    uint32_t* cursors = nullptr;
+    const int rc = trace_counters(sc->accel, &cursors);
+    if (rc != LMX_OK) return rc;
+    k_gen<<<std::max(1, std::min((int)((sc->cap + 255) / 256), sc->cus * 8)), 256, 0, st>>>(
+        sc->rs, rp, sc->ctl.p, sc->cap, b, Queue{sc->ray[b].p, sc->thr[b].p, sc->meta[b].p}, cursors);
+    return rp.nee != NEE_NONE ? enqueue_nee(sc, rp, b, cursors, st) : LMX_OK;
 }
 
 // Records one wavefront iteration tracing queue `a` and filling queue `b`.
@@ -500,28 +508,23 @@ int enqueue_iteration(lmx_scene* sc, const RParams& rp, int a, int b, hipStream_
     Queue qb{sc->ray[b].p, sc->thr[b].p, sc->meta[b].p};
     if (rp.ray_out) {
         k_capture<<<std::max(1, std::min((int)((sc->cap + 255) / 256), sc->cus * 4)), 256, 0, st>>>(
-            sc->ctl.p, qa.ray, rp.ray_out, rp.ray_out_cap);
-        k_capture_advance<<<1, 64, 0, st>>>(sc->ctl.p, rp.ray_out_cap);
+            sc->ctl.p, a, qa.ray, rp.ray_out, rp.ray_out_cap);
+        k_capture_advance<<<1, 64, 0, st>>>(sc->ctl.p, a, rp.ray_out_cap);
     }
-    int rc = launch_trace(sc->accel, reinterpret_cast<const WRay*>(qa.ray), 0, &sc->ctl.p->n_trace, sc->cap,
-                          reinterpret_cast<WHit*>(sc->hits.p), st, false, true);   // cursors set by k_commit
+    int rc = launch_trace(sc->accel, reinterpret_cast<const WRay*>(qa.ray), 0, &sc->ctl.p->n_trace[a], sc->cap,
+                          reinterpret_cast<WHit*>(sc->hits.p), st, false, true);   // cleared by the generation
     if (rc != LMX_OK) return rc;
     const int grid = std::max(1, std::min((int)((sc->cap + 255) / 256), sc->cus * 8));
     if (rp.guide) {
-        if ((rc = launch_guided_shade(sc, rp, qa, qb, st)) != LMX_OK) return rc;
+        if ((rc = launch_guided_shade(sc, rp, qa, qb, a, st)) != LMX_OK) return rc;
     } else {
         if (rp.perm) {
             k_bin_clear<<<1, 64, 0, st>>>(sc->ctl.p);
-            k_bin<<<grid, 256, 0, st>>>(sc->rs, sc->ctl.p, qa.meta, sc->hits.p, sc->perm.p, sc->cap);
+            k_bin<<<grid, 256, 0, st>>>(sc->rs, sc->ctl.p, a, qa.meta, sc->hits.p, sc->perm.p, sc->cap);
         }
-        k_shade<<<grid, 256, 0, st>>>(sc->rs, rp, sc->ctl.p, qa, sc->hits.p, qb);
+        k_shade<<<grid, 256, 0, st>>>(sc->rs, rp, sc->ctl.p, a, qa, sc->hits.p, qb);
     }
-    k_gen<<<grid, 256, 0, st>>>(sc->rs, rp, sc->ctl.p, sc->cap, qb);
-    if (rp.nee != NEE_NONE && (rc = enqueue_nee(sc, rp, st)) != LMX_OK) return rc;
-    uint32_t* cursors = nullptr;
-    uint32_t tgrid = 0;
-    if ((rc = trace_shape(sc->accel, sc->cap, &cursors, &tgrid)) != LMX_OK) return rc;
-    k_commit<<<1, 64, 0, st>>>(sc->ctl.p, sc->cap, rp.total, cursors, tgrid);
+    if ((rc = enqueue_gen(sc, rp, b, st)) != LMX_OK) return rc;
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? LMX_OK : hip_error(e, "wavefront launch");
 }
@@ -548,14 +551,8 @@ int wavefront_render(lmx_scene* sc, const RParams& rp_in, uint32_t cap, hipStrea
     }
     k_init_ctl<<<1, 64, 0, st>>>(sc->ctl.p);
     // the first generation: queue 0 gets camera paths (and their camera-vertex
-    // connections), then the counts commit
-    k_gen<<<std::max(1, std::min((int)((cap + 255) / 256), sc->cus * 8)), 256, 0, st>>>(
-        sc->rs, rp, sc->ctl.p, cap, Queue{sc->ray[0].p, sc->thr[0].p, sc->meta[0].p});
-    if (rp.nee != NEE_NONE && (rc = enqueue_nee(sc, rp, st)) != LMX_OK) return rc;
-    uint32_t* cursors = nullptr;
-    uint32_t tgrid = 0;
-    if ((rc = trace_shape(sc->accel, cap, &cursors, &tgrid)) != LMX_OK) return rc;
-    k_commit<<<1, 64, 0, st>>>(sc->ctl.p, cap, rp.total, cursors, tgrid);
+    // connections)
+    if ((rc = enqueue_gen(sc, rp, 0, st)) != LMX_OK) return rc;
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_error(e, "wavefront start");
     // The first two iterations (0 -> 1, 1 -> 0) run at once on the render
@@ -617,7 +614,7 @@ int wavefront_render(lmx_scene* sc, const RParams& rp_in, uint32_t cap, hipStrea
             rc = hip_error(e, "control readback");
             break;
         }
-        if (sc->h_ctl->n_trace == 0 && (sc->h_ctl->issued >= rp.total || stopped)) break;
+        if (sc->h_ctl->n_trace[0] == 0 && (sc->h_ctl->issued[0] >= rp.total || stopped)) break;
         if (render_time > 0.0 && !stopped &&
             std::chrono::duration<double>(std::chrono::steady_clock::now() - t_start).count() >= render_time) {
             k_stop<<<1, 64, 0, st>>>(sc->ctl.p);
@@ -625,9 +622,9 @@ int wavefront_render(lmx_scene* sc, const RParams& rp_in, uint32_t cap, hipStrea
         }
     }
     (void)hipGraphDestroy(graph);
-    if (rays) *rays = sc->h_ctl->rays + sc->h_ctl->shadow_rays;
+    if (rays) *rays = sc->h_ctl->rays + sc->h_ctl->shadow_rays + sc->h_ctl->n_shadow[0];
     if (iters) *iters = sc->h_ctl->iterations;
-    if (samples) *samples = sc->h_ctl->issued;
+    if (samples) *samples = sc->h_ctl->issued[0];
     return rc;
 }
 

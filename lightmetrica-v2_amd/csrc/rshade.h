@@ -48,16 +48,19 @@ struct RScene {
 };
 
 // Uniform of (sample, slot) from the table or from Philox.
-// Device-side control block.
+// Device-side control block.  The counts come in pairs: an iteration that
+// traces queue a and fills queue b = 1 - a reads [a] and writes [b], so that
+// its generation kernel can set the next iteration's counts while its own
+// workgroups still read this one's, and no kernel is needed between them.
 struct Ctl {
-    uint32_t n_trace;          // rays in the queue traced next
-    uint32_t n_next;           // continuing paths appended by shade
-    uint32_t issued;           // camera samples started
-    uint32_t iterations;
+    uint32_t n_trace[2];       // rays in queue 0 / 1 when it is traced
+    uint32_t n_app[2];         // continuing paths shading appended to queue 0 / 1
+    uint32_t issued[2];        // camera samples started, after filling queue 0 / 1
+    uint32_t n_shadow[2];      // next-event shadow rays of the iteration that filled queue 0 / 1
     unsigned long long rays;   // extension rays traced so far
-    uint32_t n_shadow;         // next-event shadow rays of the iteration
+    unsigned long long shadow_rays;   // those of the iterations before the last
+    uint32_t iterations;
     uint32_t stop;             // time mode: no new camera samples once set
-    unsigned long long shadow_rays;
     uint32_t bin[4];           // material-binned shading: paths per class this iteration
     uint32_t ray_out_n;        // rays copied to RParams::ray_out so far
     uint32_t film_scaled;      // the film was rescaled on the device at the render's end
@@ -430,8 +433,8 @@ struct lmx_scene;
 int wavefront_render(lmx_scene* sc, const lmx::RParams& rp, uint32_t cap, hipStream_t st, uint64_t* rays,
                      uint32_t* iters, double render_time = 0.0, uint64_t* samples = nullptr, size_t film_n = 0,
                      float film_w = 0.0f);
-// The guided shading step of one iteration (lmx_guide.hip).
-int launch_guided_shade(lmx_scene* sc, const lmx::RParams& rp, lmx::Queue in, lmx::Queue out, hipStream_t st);
+// The guided shading step of the iteration that traced queue a (lmx_guide.hip).
+int launch_guided_shade(lmx_scene* sc, const lmx::RParams& rp, lmx::Queue in, lmx::Queue out, int a, hipStream_t st);
 
 namespace lmx {
 
@@ -500,8 +503,8 @@ using lmx::RScene;
 
 // Control block of the bidirectional sampler (one batch of samples at a time).
 struct BCtl {
-    uint32_t n_trace;          // subpath rays queued for the next trace
-    uint32_t n_next;           // continuations appended by the shade step
+    uint32_t n_q[3];           // subpath rays of iteration i's queue at [i mod 3]; its shade step fills
+                               // [i + 1 mod 3] and clears [i + 2 mod 3]
     uint32_t n_shadow;         // shadow-queue slots of the batch (live and dead)
     uint32_t batch_first;      // first sample of the current batch
     unsigned long long rays;   // extension rays traced

@@ -1,9 +1,9 @@
 // trace_cursors.h -- the work split of the traversal kernel's launches:
 // the rays are cut into 8 regions (one per XCD), every wave takes a fixed
 // first chunk of its region, and the rest of each region is claimed through
-// an atomic cursor.  Shared by the kernel, the kernel that sets the cursors
-// before a launch, and wavefront loops whose own commit kernel sets them
-// for the next launch.
+// an atomic cursor that counts from 0.  Shared by the kernel, the kernel that
+// clears the cursors before a launch, and wavefront loops whose own kernels
+// clear them for the next launch.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -17,7 +17,7 @@
 #define LMX_CURSOR_STRIDE 64
 #endif
 #define CURSOR_STRIDE LMX_CURSOR_STRIDE
-// counter block of one trace launch: 8 region cursors, the ray count, and a
+// counter block of one trace launch: 8 region cursors, an unused line, and a
 // sticky stack-overflow flag, each on a line of its own
 #define LMX_TRACE_COUNTER_WORDS (10 * CURSOR_STRIDE)
 
@@ -41,8 +41,8 @@ __host__ __device__ __forceinline__ uint32_t trace_claim(uint32_t n, uint32_t gr
 }
 
 // Every wave's first chunk is fixed by its index (wave b, of XCD region
-// r = b mod 8, takes chunk b / 8 of its region); the region's cursor starts
-// after those chunks, so a launch claims with atomics only what is left,
+// r = b mod 8, takes chunk b / 8 of its region); the region's cursor counts
+// from the end of those chunks, so a launch claims with atomics only what is left,
 // and one with few rays (the tail of a wavefront render) with none.
 __host__ __device__ __forceinline__ uint32_t region_dyn_start(uint32_t r, uint32_t n, uint32_t grid, uint32_t claim)
 {
@@ -61,10 +61,9 @@ __host__ __device__ __forceinline__ bool trace_has_dynamic(uint32_t n, uint32_t 
     return any;
 }
 
-// Thread j of one wave: j < 8 sets region j's cursor, j == 8 the ray count,
-// for a launch over n rays with `grid` workgroups.
-__device__ __forceinline__ void trace_cursors_set(uint32_t* cursors, uint32_t n, uint32_t grid, uint32_t j)
+// Thread j of a workgroup, on a stream where no trace launch is running:
+// clears the cursors for the next one.
+__device__ __forceinline__ void trace_cursors_clear(uint32_t* cursors, uint32_t j)
 {
-    if (j < 8) cursors[j * CURSOR_STRIDE] = region_dyn_start(j, n, grid, trace_claim(n, grid));
-    if (j == 8) cursors[8 * CURSOR_STRIDE] = n;
+    if (j < 8) cursors[j * CURSOR_STRIDE] = 0u;
 }

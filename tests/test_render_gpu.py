@@ -206,3 +206,20 @@ def test_ggx_per_sample_parity(gpu, entry, mode):
         c = orc.Scene(sc).nee_samples(0, n, mode, max_num_vertices=m, table=tab)
         ok = _compare_nee(so.cpu().numpy(), c)
     assert ok.mean() >= 0.9999, f"{(~ok).sum()} of {n} samples differ"
+
+
+@pytest.mark.parametrize("n,cap", [(1, 64), (63, 64), (1000, 64), (70001, 4096), (200000, 1 << 20)])
+def test_ray_and_sample_counts(gpu, n, cap):
+    """Queue counts kept on the device between iterations, at odd queue sizes
+    and refills: inside a closed, scattering, emitting sphere without
+    roulette every path has max_num_vertices - 1 segments (but the few that
+    leave through an edge of the tessellation), every sample is started once,
+    and the film holds each segment's emission."""
+    sc = scenes.furnace_sphere(albedo=0.5, Le=1.0, subdiv=2, width=9, height=7)
+    rs = render.Scene(sc)
+    for seed in (1, 2):                       # the second render reuses the queues and the recorded graph
+        film, st, _ = rs.render_pt(n, max_num_vertices=5, rr_depth=100, seed=seed, queue_capacity=cap)
+        assert st["samples"] == n
+        assert 4 * n * (1 - 1e-4) - 4 <= st["rays"] <= 4 * n
+        got = float(film.double().mean())
+        assert abs(got - (1 + 0.5 + 0.25 + 0.125)) <= 1e-4 + 4.0 / n * (st["rays"] < 4 * n)
