@@ -147,18 +147,74 @@ __global__ void k_pack(const float* __restrict__ P, __bf16* __restrict__ out, fl
     out[t] = (__bf16)v;
 }
 
-// Sums the per-workgroup gradient partials, then one Adam step
-// (bias-corrected).  A workgroup of 16 waves owns 64 consecutive
+// Where parameter i goes: its bf16 places in the packed operands (forward, and
+// backward for W2..W5) or its place among the biases.  The inverse of k_pack.
+struct PackPlace {
+    int fwd, bwd, bias;            // -1: none
+};
+
+__device__ inline void slot_of_unit(int k, int& kc, int& g, int& j)   // inverse of unit_of_slot
+{
+    const int u = k & 31;
+    kc = k >> 5;
+    g = (u & 15) >> 2;
+    j = (u & 3) + (u < 16 ? 0 : 4);
+}
+
+__device__ inline PackPlace place_of(int i)
+{
+    PackPlace p = {-1, -1, -1};
+    auto at = [](int off, int nkc, int nt, int kc, int g, int col, int j) {
+        return (off + (nt * nkc + kc) * 64 + g * 16 + col) * 8 + j;
+    };
+    if (i < GP_W2) {
+        const int row = i / 64, n = i % 64;
+        // feature row -> input dimension and its slot (feat_of_slot); the bias row is slot 24 of group 3
+        const int d = row == 168 ? 7 : row / 24, L = (d < 4 ? 0 : 24) + (row == 168 ? 0 : row % 24);
+        p.fwd = at(OFF_A1, 6, n >> 4, L >> 3, d & 3, n & 15, L & 7);
+        return p;
+    }
+    int layer, rel;                 // 0..2: W2..W4 with their biases, 3: W5
+    if (i < GP_W5) {
+        layer = (i - GP_W2) / (64 * 64 + 64);
+        rel = (i - GP_W2) % (64 * 64 + 64);
+        if (rel >= 64 * 64) { p.bias = 64 * layer + rel - 64 * 64; return p; }
+    } else {
+        layer = 3;
+        rel = i - GP_W5;
+        if (rel >= 64 * 41) { p.bias = 192 + rel - 64 * 41; return p; }
+    }
+    const int N = layer == 3 ? 41 : 64, k = rel / N, n = rel % N;
+    int kc, g, j;
+    slot_of_unit(k, kc, g, j);
+    if (layer == 3) {
+        p.fwd = at(OFF_A5, 2, n >> 4, kc, g, n & 15, j);
+        p.bwd = at(OFF_B5, 2, k >> 4, n >> 5, (n & 31) >> 3, k & 15, n & 7);
+    } else {
+        p.fwd = at(OFF_A2 + layer * N_AH, 2, n >> 4, kc, g, n & 15, j);
+        slot_of_unit(n, kc, g, j);
+        p.bwd = at(OFF_B4 + (2 - layer) * N_AH, 2, k >> 4, kc, g, k & 15, j);
+    }
+    return p;
+}
+
+// Sums the per-workgroup gradient partials (GP_PAD floats apart) and, with lr,
+// takes one Adam step (bias-corrected) and writes the new weights into the
+// packed operands, where a kernel of its own cost 6 us.  Workgroup 0 also
+// sums the workgroups' losses.  A workgroup of 16 waves owns 64 consecutive
 // parameters: wave q sums the partials q, q + 16, q + 32, ... with eight
 // loads in flight per lane (a 128-partial sum is one round of loads), and
 // the first wave adds the 16 sums.  The reduction is latency-bound: with 4
 // waves and 4 loads in flight a 2^15-record step spent 31 us here.
 constexpr int ADAM_PARAMS = 64;
 constexpr int ADAM_WAVES = 16;
+constexpr int GP_PAD = (GP_N + 3) / 4 * 4;
 __global__ __launch_bounds__(ADAM_WAVES * 64) void k_adam(float* __restrict__ P, float* __restrict__ m,
                                                           float* __restrict__ v, const float* __restrict__ partial,
-                                                          int nparts, float scale, float lr, float b1, float b2,
-                                                          float c1, float c2, float eps, float* __restrict__ grad_out)
+                                                          int nparts, float lr, float b1, float b2,
+                                                          float c1, float c2, float eps, float* __restrict__ grad_out,
+                                                          const float* __restrict__ loss_part, float* __restrict__ loss,
+                                                          __bf16* __restrict__ pack, float* __restrict__ bias)
 {
     __shared__ float red[ADAM_WAVES][ADAM_PARAMS];
     const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
@@ -168,25 +224,36 @@ __global__ __launch_bounds__(ADAM_WAVES * 64) void k_adam(float* __restrict__ P,
         int k = q;
         for (; k + 7 * ADAM_WAVES < nparts; k += 8 * ADAM_WAVES) {
 #pragma unroll
-            for (int u = 0; u < 8; u++) g[u] += partial[(size_t)(k + u * ADAM_WAVES) * GP_N + i];
+            for (int u = 0; u < 8; u++) g[u] += partial[(size_t)(k + u * ADAM_WAVES) * GP_PAD + i];
         }
-        for (; k < nparts; k += ADAM_WAVES) g[0] += partial[(size_t)k * GP_N + i];
+        for (; k < nparts; k += ADAM_WAVES) g[0] += partial[(size_t)k * GP_PAD + i];
     }
     red[q][lane] = ((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7]));
+    if (blockIdx.x == 0 && q == 1) {
+        float s = 0.0f;
+        for (int k = lane; k < nparts; k += 64) s += loss_part[k];
+        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+        if (lane == 0) *loss = s;
+    }
     __syncthreads();
     if (q != 0 || i >= GP_N) return;
     float h[4];
 #pragma unroll
     for (int w = 0; w < 4; w++)
         h[w] = (red[4 * w][lane] + red[4 * w + 1][lane]) + (red[4 * w + 2][lane] + red[4 * w + 3][lane]);
-    float gs = ((h[0] + h[1]) + (h[2] + h[3])) * scale;
+    const float gs = (h[0] + h[1]) + (h[2] + h[3]);
     if (grad_out) grad_out[i] = gs;
     if (lr == 0.0f) return;
     const float mi = b1 * m[i] + (1.0f - b1) * gs;
     const float vi = b2 * v[i] + (1.0f - b2) * gs * gs;
     m[i] = mi;
     v[i] = vi;
-    P[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    const float w = P[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    P[i] = w;
+    const PackPlace pl = place_of(i);
+    if (pl.bias >= 0) bias[pl.bias] = w;
+    if (pl.fwd >= 0) pack[pl.fwd] = (__bf16)w;
+    if (pl.bwd >= 0) pack[pl.bwd] = (__bf16)w;
 }
 
 // ---------------------------------------------------------------------------
@@ -264,9 +331,11 @@ struct NoSink {
 };
 
 // Forward pass of MT tiles of 16 queries (inputs xs[MT*16][8]) for one wave;
-// outputs to ys[MT*16][YS].
+// outputs to ys[MT*16][YS].  W: the packed operands of layer 1; Wh: those of
+// the other layers (from OFF_A2 on), which may lie elsewhere.
 template <int MT, class Sink>
-RD void mlp_forward(const bf16x8* __restrict__ W, const float* __restrict__ bias, const float* xs, float* ys,
+RD void mlp_forward(const bf16x8* __restrict__ W, const bf16x8* __restrict__ Wh, const float* __restrict__ bias,
+                    const float* xs, float* ys,
                     Sink& sink)
 {
     const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
@@ -302,7 +371,7 @@ RD void mlp_forward(const bf16x8* __restrict__ W, const float* __restrict__ bias
         }
 #pragma unroll
     for (int L = 0; L < 3; L++) {
-        const bf16x8* A = W + OFF_A2 + L * N_AH;
+        const bf16x8* A = Wh + L * N_AH;
         const float* bl = bias + 64 * L;
 #pragma unroll
         for (int nt = 0; nt < 4; nt++) {
@@ -339,7 +408,7 @@ RD void mlp_forward(const bf16x8* __restrict__ W, const float* __restrict__ bias
     for (int kc = 0; kc < 2; kc++)
 #pragma unroll
         for (int nt = 0; nt < 3; nt++) {
-            const bf16x8 a = W[OFF_A5 + (nt * 2 + kc) * 64 + lane];
+            const bf16x8 a = Wh[OFF_A5 - OFF_A2 + (nt * 2 + kc) * 64 + lane];
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) o[nt][mt] = MFMA16(a, h[mt][kc], o[nt][mt]);
         }
@@ -463,26 +532,61 @@ RD int mix_lobe(const Mix& m, float u, f3& mu, float& kap)
     return lobe;
 }
 
-// d(-w log q)/dy of one record (q = alpha pb + (1 - alpha) p_vmf(dir))
-RD float out_grad(const float* y, f3 dir, float pb, float w, float* g)
+// Sum (or maximum) over the four lanes 4 r .. 4 r + 3 of a record.
+RD float quad_sum(float x) { x += __shfl_xor(x, 1); return x + __shfl_xor(x, 2); }
+RD float quad_max(float x) { x = fmaxf(x, __shfl_xor(x, 1)); return fmaxf(x, __shfl_xor(x, 2)); }
+
+// d(-w log q)/dy of one record (q = alpha pb + (1 - alpha) p_vmf(dir)), in
+// place in its 41 outputs y; the loss.  Four lanes share a record, two lobes
+// each (lane part = 0..3); all of them must call it together.
+RD float out_grad_quad(float* y, int part, f3 dir, float pb, float w)
 {
-    Mix m;
-    mix_decode(y, m);
-    float v[8];
-    const float pv = mix_pdf(m, dir, v);
-    const float q = m.alpha * pb + (1.0f - m.alpha) * pv;
-    const float gq = q > 0.0f ? -w / q : 0.0f;
-    g[40] = gq * (pb - pv) * ALPHA_SPAN * m.sig * (1.0f - m.sig);
+    f3 mu[2];
+    float len[2], kap[2], pi[2], v[2];
+    bool clamped[2];
+    float mx = -3.4e38f;
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-        const float base = gq * (1.0f - m.alpha) * m.pi[k];
-        g[32 + k] = base * (v[k] - pv);
-        const float kap = m.kap[k], c = dot(m.mu[k], dir);
-        g[24 + k] = m.kclamp[k] ? 0.0f : base * v[k] * (1.0f - 2.0f * kap / expm1f(2.0f * kap) + kap * (c - 1.0f));
-        const float s = m.mlen[k] > 0.0f ? base * v[k] * kap / m.mlen[k] : 0.0f;
-        g[3 * k] = s * (dir.x - c * m.mu[k].x);
-        g[3 * k + 1] = s * (dir.y - c * m.mu[k].y);
-        g[3 * k + 2] = s * (dir.z - c * m.mu[k].z);
+    for (int u = 0; u < 2; u++) {
+        const int k = 2 * part + u;
+        const f3 r = mk3(y[3 * k], y[3 * k + 1], y[3 * k + 2]);
+        len[u] = mx_sqrt(dot(r, r));
+        const float il = mx_div(1.0f, len[u]);
+        mu[u] = len[u] > 0.0f ? mk3(r.x * il, r.y * il, r.z * il) : mk3(0.0f, 0.0f, 1.0f);
+        const float lk = y[24 + k];
+        clamped[u] = lk < LOGK_MIN || lk > LOGK_MAX;
+        kap[u] = mx_exp(fminf(fmaxf(lk, LOGK_MIN), LOGK_MAX));
+        pi[u] = y[32 + k];
+        mx = fmaxf(mx, pi[u]);
+    }
+    mx = quad_max(mx);
+#pragma unroll
+    for (int u = 0; u < 2; u++) pi[u] = mx_exp(pi[u] - mx);
+    const float is = mx_div(1.0f, quad_sum(pi[0] + pi[1]));
+    const float sig = mx_div(1.0f, 1.0f + mx_exp(-y[40]));
+    const float alpha = ALPHA_MIN + ALPHA_SPAN * sig;
+    float pv = 0.0f;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        pi[u] *= is;
+        v[u] = vmf_pdf(mu[u], kap[u], dir);
+        pv += pi[u] * v[u];
+    }
+    pv = quad_sum(pv);
+    const float q = alpha * pb + (1.0f - alpha) * pv;
+    const float gq = q > 0.0f ? -w / q : 0.0f;
+    wave_sync();                                   // every lane of the record has read y[40]
+    if (part == 0) y[40] = gq * (pb - pv) * ALPHA_SPAN * sig * (1.0f - sig);
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int k = 2 * part + u;
+        const float base = gq * (1.0f - alpha) * pi[u];
+        y[32 + k] = base * (v[u] - pv);
+        const float c = dot(mu[u], dir);
+        y[24 + k] = clamped[u] ? 0.0f : base * v[u] * (1.0f - 2.0f * kap[u] / expm1f(2.0f * kap[u]) + kap[u] * (c - 1.0f));
+        const float s = len[u] > 0.0f ? base * v[u] * kap[u] / len[u] : 0.0f;
+        y[3 * k] = s * (dir.x - c * mu[u].x);
+        y[3 * k + 1] = s * (dir.y - c * mu[u].y);
+        y[3 * k + 2] = s * (dir.z - c * mu[u].z);
     }
     return q > 0.0f ? -w * logf(q) : 0.0f;
 }
@@ -523,7 +627,7 @@ __global__ __launch_bounds__(EVAL_WAVES * 64) void k_eval(GuideDev G, const floa
             for (uint32_t k = (uint32_t)lane; k < 64u * 7u; k += 64u) yw[k] = k < nq * 7u ? x[(size_t)base * 7 + k] : 0.0f;
         }
         wave_sync();
-        mlp_forward<4>(wl, bl, yw, yw, dummy);
+        mlp_forward<4>(wl, wl + OFF_A2, bl, yw, yw, dummy);
         wave_sync();
         if (nq == 64u && vec) {
             float4* dst = reinterpret_cast<float4*>(y + (size_t)base * 41);
@@ -563,269 +667,219 @@ __global__ void k_mix_sample(const float* __restrict__ y, const float* __restric
 // throughput at the vertex, the loss weight, and the path's contribution so
 // far (the weight is finished once the path has ended).
 
-// Two kernels per step.  k_train_fb: forward (keeping the layer inputs),
-// the loss gradient and the backward pass, 32 records per wave pass; it
-// writes every layer input A_l and every layer-output delta D_l as bf16 rows
-// [unit][record] to a scratch array.  k_wgrad: dW_l^T = D_l A_{l-1}^T as a
-// split-K GEMM over records, each workgroup staging 32-record slices of all
-// rows in LDS and its waves accumulating all 108 output tiles in registers;
-// one gradient partial per workgroup, summed by k_adam.
+// One kernel per gradient (k_train), then k_adam.  A workgroup of 4 waves
+// takes 64 records a step: each wave runs forward, loss gradient and backward
+// over 16 of them, writing every layer input A_l and every layer-output delta
+// D_l as bf16 rows [unit][record] into LDS; then the 4 waves accumulate
+// dW_l^T = D_l A_{l-1}^T over the 64 records in registers, 27 of the 108
+// 16 x 16 tiles each.  One gradient partial per workgroup.
 //
-// Scratch layout: one block of NROWS x 32 bf16 per 32-record pass,
-// [pass][row][record], so that a pass's rows are one contiguous 47 KB span:
+// Latency bounds it: 32,768 records are two steps for every CU (the rows of
+// 64 records take 108 KB of its LDS), and a step is a chain of ten layers of
+// 8 MFMAs, each fed by the one before.  The rows stay in LDS because the
+// chain leaves no time for memory: as two kernels with the rows in HBM (1.5 KB
+// a record, written and read back two bytes at a time) the same gradient took
+// 48 + 45 us, 41 us as one.  The weights a layer waits for are in LDS too, as
+// far as it holds them (the forward layers but the first, 30 KB): 7.7
+// us less than from the L2.  Two column tiles a wave, which would halve the
+// reads of the rest, spill (94 registers) and take longer.
 constexpr int ROW_A0 = 0;              // encoding, 192 slots (layer-1 operand order)
 constexpr int ROW_A1 = 192;            // h1..h4, 64 units each, natural order
 constexpr int ROW_D1 = ROW_A1 + 256;   // deltas of layers 1..4 (pre-activation), 64 each
 constexpr int ROW_D5 = ROW_D1 + 256;   // output gradient, 48 (41 used)
 constexpr int NROWS = ROW_D5 + 48;     // 752
-constexpr int FB_WAVES = 4;
-constexpr int WG_WAVES = 4;
-constexpr int SROW = 40;               // bf16 per staged row (32 records + bank padding)
+constexpr int TR_WAVES = 4;
+constexpr int TR_RECS = 16 * TR_WAVES; // records a step
+constexpr int TR_ROW = TR_RECS + 8;    // bf16 per row: 36 banks on, so that 16 rows read 16 bytes each without conflicts
 
-// one operand-layout chunk (tile mt, chunk kc: units unit_of_slot(kc, g, j))
-// -> rows [row0 + unit][record] of a pass block
-RD void store_chunk(__bf16* blk, int row0, int mt, int kc, const bf16x8& v, int lane)
+// one operand-layout chunk (chunk kc: units unit_of_slot(kc, g, j)) -> rows
+// [row0 + unit], column col
+RD void store_chunk(__bf16* rows, int row0, int col, int kc, int g, const bf16x8& v)
 {
-    const int g = lane >> 4, r = lane & 15;
-    __bf16* base = blk + mt * 16 + r;
 #pragma unroll
-    for (int j = 0; j < 8; j++) base[(row0 + unit_of_slot(kc, g, j)) * 32] = v[j];
+    for (int j = 0; j < 8; j++) rows[(row0 + unit_of_slot(kc, g, j)) * TR_ROW + col] = v[j];
 }
 
-// ReLU mask of an operand-layout activation: bit 16 mt + 8 c + j
-RD uint32_t relu_bits(int mt, int c, const bf16x8& h)
+// ReLU mask of an operand-layout activation: bit 8 c + j
+RD uint32_t relu_bits(int c, const bf16x8& h)
 {
     uint32_t m = 0;
 #pragma unroll
-    for (int j = 0; j < 8; j++) m |= ((float)h[j] > 0.0f ? 1u : 0u) << (16 * mt + 8 * c + j);
+    for (int j = 0; j < 8; j++) m |= ((float)h[j] > 0.0f ? 1u : 0u) << (8 * c + j);
     return m;
 }
 
 // forward observer of training: the encoding (layer-1 slot order) and
-// h1..h4 go to the scratch rows; the ReLU masks stay in registers
+// h1..h4 go to the LDS rows; the ReLU masks stay in registers
 struct TrainSink {
-    __bf16* blk;
-    int lane;
+    __bf16* rows;
+    int col, g;
     uint32_t mask[4];
-    RD void enc(int kc, int mt, const bf16x8& b)
+    RD void enc(int kc, int, const bf16x8& b)
     {
-        const int g = lane >> 4, r = lane & 15;
-        __bf16* base = blk + mt * 16 + r;
 #pragma unroll
-        for (int j = 0; j < 8; j++) base[(ROW_A0 + kc * 32 + 8 * g + j) * 32] = b[j];
+        for (int j = 0; j < 8; j++) rows[(ROW_A0 + kc * 32 + 8 * g + j) * TR_ROW + col] = b[j];
     }
-    RD void hidden(int L, int mt, int c, const bf16x8& h)
+    RD void hidden(int L, int, int c, const bf16x8& h)
     {
-        store_chunk(blk, ROW_A1 + 64 * L, mt, c, h, lane);
-        const uint32_t m = relu_bits(mt, c, h);
-        mask[L] = (mt == 0 && c == 0) ? m : (mask[L] | m);
+        store_chunk(rows, ROW_A1 + 64 * L, col, c, g, h);
+        const uint32_t m = relu_bits(c, h);
+        mask[L] = c == 0 ? m : (mask[L] | m);
     }
 };
 
 // one backward layer: delta of the layer input = W (natural rows) * delta,
 // masked by the ReLU of that input (bits of relu_bits)
-RD void back_layer(const bf16x8* __restrict__ Wb, const bf16x8 (&din)[2][2], uint32_t mask, bf16x8 (&dout)[2][2],
-                   int lane)
+RD void back_layer(const bf16x8* __restrict__ Wb, const bf16x8 (&din)[2], uint32_t mask, bf16x8 (&dout)[2], int lane)
 {
-    f32x4 acc[4][2];
+    f32x4 acc[4];
 #pragma unroll
-    for (int nt = 0; nt < 4; nt++)
-#pragma unroll
-        for (int mt = 0; mt < 2; mt++) acc[nt][mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int nt = 0; nt < 4; nt++) acc[nt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int kc = 0; kc < 2; kc++)
 #pragma unroll
-        for (int nt = 0; nt < 4; nt++) {
-            const bf16x8 a = Wb[(nt * 2 + kc) * 64 + lane];
+        for (int nt = 0; nt < 4; nt++) acc[nt] = MFMA16(Wb[(nt * 2 + kc) * 64 + lane], din[kc], acc[nt]);
 #pragma unroll
-            for (int mt = 0; mt < 2; mt++) acc[nt][mt] = MFMA16(a, din[mt][kc], acc[nt][mt]);
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            dout[c][i] = (mask >> (8 * c + i)) & 1u ? (__bf16)acc[2 * c][i] : (__bf16)0.0f;
+            dout[c][4 + i] = (mask >> (8 * c + 4 + i)) & 1u ? (__bf16)acc[2 * c + 1][i] : (__bf16)0.0f;
         }
-#pragma unroll
-    for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-        for (int c = 0; c < 2; c++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int bit = 16 * mt + 8 * c;
-                dout[mt][c][i] = (mask >> (bit + i)) & 1u ? (__bf16)acc[2 * c][mt][i] : (__bf16)0.0f;
-                dout[mt][c][4 + i] = (mask >> (bit + 4 + i)) & 1u ? (__bf16)acc[2 * c + 1][mt][i] : (__bf16)0.0f;
-            }
-}
-
-// Forward, loss gradient and backward over `n` records (indices idx, or
-// 0..n-1), padded to whole 32-record passes (padding records have weight 0);
-// writes the scratch blocks of all passes.
-__global__ __launch_bounds__(FB_WAVES * 64) void k_train_fb(GuideDev G, const float4* __restrict__ recs,
-                                                           const uint32_t* __restrict__ idx, uint32_t n,
-                                                           float wnorm, float wclamp, float inv_n,
-                                                           __bf16* __restrict__ act, float* __restrict__ loss)
-{
-    __shared__ float xs_all[FB_WAVES][32 * 8];
-    __shared__ float ys_all[FB_WAVES][32 * YS];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
-    float* xs = xs_all[wave];
-    float* ys = ys_all[wave];
-    float lsum = 0.0f;
-    const uint32_t npass = (n + 31) / 32;
-    for (uint32_t pass = blockIdx.x * FB_WAVES + wave; pass < npass; pass += gridDim.x * FB_WAVES) {
-        __bf16* blk = act + (size_t)pass * NROWS * 32;
-        const uint32_t j = pass * 32 + (uint32_t)lane;
-        const bool mine = lane < 32 && j < n;
-        f3 dir = mk3(0, 0, 0);
-        float pb = 0.0f, w = 0.0f;
-        if (lane < 32) {
-            float x[7] = {0, 0, 0, 0, 0, 0, 0};
-            if (mine) {
-                const size_t q = idx ? idx[j] : j;
-                const float4 a = recs[5 * q], b = recs[5 * q + 1], c = recs[5 * q + 2], d = recs[5 * q + 3];
-                x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w; x[4] = b.x; x[5] = b.y; x[6] = b.z;
-                pb = b.w;
-                dir = mk3(c.x, c.y, c.z);
-                w = fminf(d.w * wnorm, wclamp) * inv_n;
-            }
-            for (int k = 0; k < 7; k++) xs[lane * XS + k] = x[k];
-        }
-        wave_sync();
-        TrainSink sink{blk, lane, {0u, 0u, 0u, 0u}};
-        mlp_forward<2>(G.pack, G.bias, xs, ys, sink);
-        wave_sync();
-        // output gradient (rows of ys, in place; pre-scaled by 1/n) and D5
-        if (lane < 32) {
-            float gy[41];
-            if (mine) lsum += out_grad(ys + lane * YS, dir, pb, w, gy);
-            else for (int o = 0; o < 41; o++) gy[o] = 0.0f;
-            for (int o = 0; o < 41; o++) {
-                ys[lane * YS + o] = gy[o];
-                blk[(ROW_D5 + o) * 32 + lane] = (__bf16)gy[o];
-            }
-            for (int o = 41; o < 48; o++) blk[(ROW_D5 + o) * 32 + lane] = (__bf16)0.0f;
-        }
-        wave_sync();
-        // backward: W5 (natural output order) * dY, then W4, W3, W2
-        bf16x8 dy[2][2], d[2][2], dn[2][2];
-#pragma unroll
-        for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-            for (int kc = 0; kc < 2; kc++)
-#pragma unroll
-                for (int jj = 0; jj < 8; jj++) {
-                    const int o = 32 * kc + 8 * g + jj;
-                    dy[mt][kc][jj] = o < 41 ? (__bf16)ys[(mt * 16 + r) * YS + o] : (__bf16)0.0f;
-                }
-        back_layer(G.pack + OFF_B5, dy, sink.mask[3], d, lane);     // D4
-#pragma unroll
-        for (int L = 3; L >= 0; L--) {                              // store D_L+1, make D_L
-#pragma unroll
-            for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-                for (int kc = 0; kc < 2; kc++) store_chunk(blk, ROW_D1 + 64 * L, mt, kc, d[mt][kc], lane);
-            if (L == 0) break;
-            back_layer(G.pack + OFF_B4 + (3 - L) * N_AH, d, sink.mask[L - 1], dn, lane);
-#pragma unroll
-            for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-                for (int kc = 0; kc < 2; kc++) d[mt][kc] = dn[mt][kc];
-        }
-        wave_sync();
-    }
-    for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off);
-    if (lane == 0 && loss) atomicAdd(loss, lsum);
 }
 
 // The 108 weight-gradient tiles of the network (16 x 16 each, rows n of a
 // layer's outputs, columns k of its inputs): layer 1 4 x 12, layers 2-4
-// 4 x 4 each, layer 5 3 x 4.  Tile t: its layer, the first scratch row of its
-// delta rows and of its input rows.
-struct WTile {
-    int layer, nt, kt, drow, arow;
-};
-RD WTile tile_of(int t)
-{
-    WTile T;
-    if (t < 48) {
-        T.layer = 1; T.nt = t / 12; T.kt = t % 12;
-        T.drow = ROW_D1 + 16 * T.nt; T.arow = ROW_A0 + 16 * T.kt;
-    } else if (t < 96) {
-        const int u = t - 48;
-        T.layer = 2 + u / 16; T.nt = (u % 16) / 4; T.kt = u % 4;
-        T.drow = ROW_D1 + 64 * (T.layer - 1) + 16 * T.nt; T.arow = ROW_A1 + 64 * (T.layer - 2) + 16 * T.kt;
-    } else {
-        const int u = t - 96;
-        T.layer = 5; T.nt = u / 4; T.kt = u % 4;
-        T.drow = ROW_D5 + 16 * T.nt; T.arow = ROW_A1 + 192 + 16 * T.kt;
-    }
-    return T;
-}
-constexpr int TILES_PER_WAVE = 27;
-static_assert(TILES_PER_WAVE * WG_WAVES == 108, "every tile has one wave");
+// 4 x 4 each, layer 5 3 x 4.  Wave w has row tile w of layers 1..4 (its 12 or
+// 4 column tiles share one operand) and column tile w of layer 5, so that
+// which layer an accumulator belongs to is known to the compiler.
+constexpr int T_L2 = 12, T_L5 = 24, TILES_PER_WAVE = 27;
+static_assert(TR_WAVES == 4, "a row tile per wave");
 
-// Split-K weight gradients: workgroup b sums the passes [b*chunk, (b+1)*chunk)
-// of the scratch into partial[b] (every parameter written).
-__global__ __launch_bounds__(WG_WAVES * 64) void k_wgrad(const __bf16* __restrict__ act, uint32_t npass,
-                                                         uint32_t chunk, float* __restrict__ partial)
+// Gradient partial (and loss) of each workgroup over `n` records (indices
+// idx, or 0..n-1); records past n have weight 0.
+__global__ __launch_bounds__(TR_WAVES * 64) void k_train(GuideDev G, const float4* __restrict__ recs,
+                                                         const uint32_t* __restrict__ idx, uint32_t n, float wnorm,
+                                                         float wclamp, float inv_n, float* __restrict__ partial,
+                                                         float* __restrict__ loss_part)
 {
-    __shared__ alignas(16) __bf16 st[NROWS * SROW];
+    __shared__ alignas(16) __bf16 rows[NROWS * TR_ROW];
+    __shared__ float ys_all[TR_WAVES][16 * YS];            // inputs at the start of each wave's outputs
+    __shared__ float lsum_all[TR_WAVES];
+    __shared__ bf16x8 wh[N_FWD - OFF_A2];                  // forward operands of layers 2..5
+    __shared__ float bl[N_BIAS];
+    for (int t = threadIdx.x; t < N_FWD - OFF_A2; t += TR_WAVES * 64) wh[t] = G.pack[OFF_A2 + t];
+    for (int t = threadIdx.x; t < N_BIAS; t += TR_WAVES * 64) bl[t] = G.bias[t];
+    __syncthreads();
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
+    const int quad = lane >> 2, part = lane & 3;
+    float* ys = ys_all[wave];
+    const int col = 16 * wave + r;
     f32x4 acc[TILES_PER_WAVE];
 #pragma unroll
     for (int t = 0; t < TILES_PER_WAVE; t++) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float bsum = 0.0f;                                   // thread t < 240: bias row t of D2..D5
-    const uint32_t p_begin = blockIdx.x * chunk;
-    const uint32_t p_end = min(npass, p_begin + chunk);
-    // software pipeline: the next pass block is loaded into registers while
-    // the MFMAs of the current one run (752 rows x 64 B = 12 x 16 B per thread)
-    constexpr int NPRE = (NROWS * 4 + WG_WAVES * 64 - 1) / (WG_WAVES * 64);
-    uint4 pre[NPRE];
-    auto fetch = [&](uint32_t pass) {
-        const uint4* src = reinterpret_cast<const uint4*>(act + (size_t)pass * NROWS * 32);
-#pragma unroll
-        for (int u = 0; u < NPRE; u++) {
-            const int t = (int)threadIdx.x + u * WG_WAVES * 64;
-            if (t < NROWS * 4) pre[u] = src[t];
+    float bsum = 0.0f;                                     // thread t < 240: bias row t of D2..D5
+    float lsum = 0.0f;
+    const uint32_t steps = (n + TR_RECS - 1) / TR_RECS;
+    for (uint32_t step = blockIdx.x; step < steps; step += gridDim.x) {
+        // the record of this lane's quad: its lanes load one float4 each
+        const uint32_t jq = step * TR_RECS + 16u * (uint32_t)wave + (uint32_t)quad;
+        float4 f = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (jq < n) f = recs[5 * (size_t)(idx ? idx[jq] : jq) + part];
+        if (part == 0) {
+            ys[quad * XS] = f.x; ys[quad * XS + 1] = f.y; ys[quad * XS + 2] = f.z; ys[quad * XS + 3] = f.w;
+        } else if (part == 1) {
+            ys[quad * XS + 4] = f.x; ys[quad * XS + 5] = f.y; ys[quad * XS + 6] = f.z;
         }
-    };
-    if (p_begin < p_end) fetch(p_begin);
-    for (uint32_t pass = p_begin; pass < p_end; pass++) {
+        const int q0 = lane & ~3;
+        const float pb = __shfl(f.w, q0 + 1);
+        const f3 dir = mk3(__shfl(f.x, q0 + 2), __shfl(f.y, q0 + 2), __shfl(f.z, q0 + 2));
+        const float wrec = __shfl(f.w, q0 + 3);
+        const float w = jq < n ? fminf(wrec * wnorm, wclamp) * inv_n : 0.0f;
+        wave_sync();
+        TrainSink sink{rows, col, g, {0u, 0u, 0u, 0u}};
+        mlp_forward<1>(G.pack, wh, bl, ys, ys, sink);
+        wave_sync();
+        // output gradient, in place (pre-scaled by 1/n); records past n: exactly 0
+        const float l = out_grad_quad(ys + quad * YS, part, dir, pb, w);
+        if (part == 0) lsum += l;
+        wave_sync();
+        bf16x8 d[2], dn[2];
+#pragma unroll
+        for (int kc = 0; kc < 2; kc++)
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const int o = 32 * kc + 8 * g + j;
+                d[kc][j] = o < 41 && step * TR_RECS + (uint32_t)col < n ? (__bf16)ys[r * YS + o] : (__bf16)0.0f;
+                if (o < 48) rows[(ROW_D5 + o) * TR_ROW + col] = d[kc][j];
+            }
+        // backward: W5 (natural output order) * dY, then W4, W3, W2
+        back_layer(G.pack + OFF_B5, d, sink.mask[3], dn, lane);     // D4
+#pragma unroll
+        for (int L = 3; L >= 0; L--) {                              // store D_L+1, make D_L
+#pragma unroll
+            for (int kc = 0; kc < 2; kc++) {
+                d[kc] = dn[kc];
+                store_chunk(rows, ROW_D1 + 64 * L, col, kc, g, d[kc]);
+            }
+            if (L > 0) back_layer(G.pack + OFF_B4 + (3 - L) * N_AH, d, sink.mask[L - 1], dn, lane);
+        }
         __syncthreads();
-        // stage one pass block: 752 rows x 64 B, 16 B per thread per step
+        // weight gradients over the step's records, 32 at a time
+        {
+            const __bf16* at = rows + r * TR_ROW + 8 * g;              // row r of a tile, this lane's 8 records
+            auto op = [&](int row, int k) { return *reinterpret_cast<const bf16x8*>(at + row * TR_ROW + 32 * k); };
+            auto tile = [&](f32x4& c, const bf16x8& a0, const bf16x8& a1, int row) {
+                c = MFMA16(a0, op(row, 0), c);
+                c = MFMA16(a1, op(row, 1), c);
+            };
+            {
+                const bf16x8 d0 = op(ROW_D1 + 16 * wave, 0), d1 = op(ROW_D1 + 16 * wave, 1);
 #pragma unroll
-        for (int u = 0; u < NPRE; u++) {
-            const int t = (int)threadIdx.x + u * WG_WAVES * 64;
-            if (t < NROWS * 4) *reinterpret_cast<uint4*>(&st[(t >> 2) * SROW + (t & 3) * 8]) = pre[u];
-        }
-        __syncthreads();
-        if (pass + 1 < p_end) fetch(pass + 1);
+                for (int i = 0; i < T_L2; i++) tile(acc[i], d0, d1, ROW_A0 + 16 * i);
+            }
 #pragma unroll
-        for (int i = 0; i < TILES_PER_WAVE; i++) {
-            const WTile T = tile_of(wave * TILES_PER_WAVE + i);
-            const bf16x8 a = *reinterpret_cast<const bf16x8*>(&st[(T.drow + r) * SROW + 8 * g]);
-            const bf16x8 b = *reinterpret_cast<const bf16x8*>(&st[(T.arow + r) * SROW + 8 * g]);
-            acc[i] = MFMA16(a, b, acc[i]);
-        }
-        if (threadIdx.x < 240) {
-            const int row = ROW_D1 + 64 + threadIdx.x;      // D2, D3, D4 (64 each), D5 (48)
-            for (int q = 0; q < 32; q++) bsum += (float)st[row * SROW + q];
-        }
-    }
-    float* P = partial + (size_t)blockIdx.x * GP_N;
+            for (int L = 0; L < 3; L++) {
+                const int row = ROW_D1 + 64 * (L + 1) + 16 * wave;
+                const bf16x8 d0 = op(row, 0), d1 = op(row, 1);
 #pragma unroll
-    for (int i = 0; i < TILES_PER_WAVE; i++) {
-        const WTile T = tile_of(wave * TILES_PER_WAVE + i);
-        const int k = T.kt * 16 + r;
+                for (int i = 0; i < 4; i++) tile(acc[T_L2 + 4 * L + i], d0, d1, ROW_A1 + 64 * L + 16 * i);
+            }
+            const bf16x8 a0 = op(ROW_A1 + 192 + 16 * wave, 0), a1 = op(ROW_A1 + 192 + 16 * wave, 1);
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int nn = T.nt * 16 + 4 * g + e;
-            if (T.layer == 1) {
-                const int row = feat_of_slot(k >> 5, (k & 31) >> 3, k & 7);
-                if (row >= 0) P[GP_W1 + row * 64 + nn] = acc[i][e];
-            } else if (T.layer == 5) {
-                if (nn < 41) P[GP_W5 + k * 41 + nn] = acc[i][e];
-            } else {
-                const int W = T.layer == 2 ? GP_W2 : (T.layer == 3 ? GP_W3 : GP_W4);
-                P[W + k * 64 + nn] = acc[i][e];
+            for (int i = 0; i < 3; i++) {
+                acc[T_L5 + i] = MFMA16(op(ROW_D5 + 16 * i, 0), a0, acc[T_L5 + i]);
+                acc[T_L5 + i] = MFMA16(op(ROW_D5 + 16 * i, 1), a1, acc[T_L5 + i]);
             }
         }
+        if (threadIdx.x < 240) {                                    // D2, D3, D4 (64 each), D5 (48)
+            const __bf16* row = &rows[(ROW_D1 + 64 + (int)threadIdx.x) * TR_ROW];
+#pragma unroll
+            for (int q = 0; q < TR_RECS / 8; q++) {
+                const bf16x8 v = *reinterpret_cast<const bf16x8*>(row + 8 * q);
+#pragma unroll
+                for (int j = 0; j < 8; j++) bsum += (float)v[j];
+            }
+        }
+        __syncthreads();
     }
+    for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off);
+    if (lane == 0) lsum_all[wave] = lsum;
+    float* P = partial + (size_t)blockIdx.x * GP_PAD;
+    const int nn = 16 * wave + 4 * g;                      // layers 1..4: this lane's 4 outputs
+#pragma unroll
+    for (int i = 0; i < T_L2; i++) {
+        const int k = 16 * i + r, row = feat_of_slot(k >> 5, (k & 31) >> 3, k & 7);
+        if (row >= 0) *reinterpret_cast<f32x4*>(&P[GP_W1 + row * 64 + nn]) = acc[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 12; i++)
+        *reinterpret_cast<f32x4*>(&P[GP_W2 + (i / 4) * (GP_W3 - GP_W2) + (16 * (i & 3) + r) * 64 + nn]) = acc[T_L2 + i];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (16 * i + 4 * g + e < 41) P[GP_W5 + (16 * wave + r) * 41 + 16 * i + 4 * g + e] = acc[T_L5 + i][e];
     if (threadIdx.x < 240) {
         const int t = threadIdx.x;
         if (t < 64) P[GP_B2 + t] = bsum;
@@ -833,7 +887,10 @@ __global__ __launch_bounds__(WG_WAVES * 64) void k_wgrad(const __bf16* __restric
         else if (t < 192) P[GP_B4 + t - 128] = bsum;
         else if (t - 192 < 41) P[GP_B5 + t - 192] = bsum;
     }
+    __syncthreads();
+    if (threadIdx.x == 0) loss_part[blockIdx.x] = (lsum_all[0] + lsum_all[1]) + (lsum_all[2] + lsum_all[3]);
 }
+static_assert(GP_W4 - GP_W3 == GP_W3 - GP_W2 && GP_W1 % 4 == 0 && GP_W2 % 4 == 0 && GP_W3 % 4 == 0 && GP_W4 % 4 == 0, "16-byte partial stores");
 
 // Loss weights of the records of one pass: w = mean over channels of
 // (contribution after the vertex) / (throughput at the vertex); their sum.
@@ -986,7 +1043,7 @@ __global__ __launch_bounds__(GS_WAVES * 64) void k_guided_shade(RScene s, RParam
 #pragma unroll
         for (int k = 0; k < 7; k++) ys[wave][lane * XS + k] = x[k];
         __syncthreads();
-        if (__ballot(guided)) mlp_forward<4>(wl, bl, ys[wave], ys[wave], dummy);   // wave-uniform
+        if (__ballot(guided)) mlp_forward<4>(wl, wl + OFF_A2, bl, ys[wave], ys[wave], dummy);   // wave-uniform
         __syncthreads();
         if (guided) {
             Mix mx;
@@ -1065,8 +1122,9 @@ int launch_guided_shade(lmx_scene* sc, const RParams& rp, Queue qa, Queue qb, in
 struct lmx_guide {
     lmx_scene* scene = nullptr;
     lmx_guide_opts opts;
-    DevBuf<float> P, m, v, grad, partial, loss, wsum;
-    DevBuf<__bf16> pack, act;
+    DevBuf<float> P, m, v, grad, partial, loss_part, wsum;
+    float* h_loss = nullptr;       // pinned; k_adam writes the step's mean loss here
+    DevBuf<__bf16> pack;
     DevBuf<float> bias;
     DevBuf<float4> recs;
     DevBuf<uint32_t> rec_count, idx, nz, nz_count;
@@ -1084,6 +1142,7 @@ struct lmx_guide {
         return G;
     }
     f3 lo, inv_ext;
+    ~lmx_guide() { if (h_loss) (void)hipHostFree(h_loss); }
 };
 
 namespace {
@@ -1099,22 +1158,9 @@ int guide_pack(lmx_guide* g, hipStream_t st)
 int guide_train_step(lmx_guide* g, const float4* recs, const uint32_t* idx, uint32_t n, float wnorm, float wclamp,
                      bool adam, float* grad_out, hipStream_t st)
 {
-    hipError_t e;
-    const uint32_t npass = std::max<uint32_t>((n + 31) / 32, 1);
-    if (g->act.n < (size_t)NROWS * 32 * npass) {
-        if ((e = hipStreamSynchronize(st)) != hipSuccess || (e = g->act.alloc((size_t)NROWS * 32 * npass)) != hipSuccess)
-            return hip_error(e, "guide training scratch");
-    }
-    // forward/backward: one wave per 32-record pass, up to 8 waves per CU
-    const int fb_wg = std::max(1, std::min((int)((npass + FB_WAVES - 1) / FB_WAVES), 2 * g->nparts));
-    // weight gradients: at least 4 passes per workgroup (a 2^15-record step
-    // fills the CUs with one workgroup each)
-    const int nwg = std::max(1, std::min((int)((npass + 3) / 4), g->nparts));
-    const uint32_t chunk = (npass + nwg - 1) / nwg;
-    k_fill<<<1, 64, 0, st>>>(g->loss.p, 1, 0.0f);
-    k_train_fb<<<fb_wg, FB_WAVES * 64, 0, st>>>(g->dev(), recs, idx, n, wnorm, wclamp, 1.0f / (float)n, g->act.p,
-                                                g->loss.p);
-    k_wgrad<<<nwg, WG_WAVES * 64, 0, st>>>(g->act.p, npass, chunk, g->partial.p);
+    const int nwg = (int)std::min<uint32_t>((n + TR_RECS - 1) / TR_RECS, (uint32_t)g->nparts);
+    k_train<<<nwg, TR_WAVES * 64, 0, st>>>(g->dev(), recs, idx, n, wnorm, wclamp, 1.0f / (float)n, g->partial.p,
+                                           g->loss_part.p);
     float lr = 0.0f, c1 = 1.0f, c2 = 1.0f;
     if (adam) {
         g->step++;
@@ -1122,10 +1168,11 @@ int guide_train_step(lmx_guide* g, const float4* recs, const uint32_t* idx, uint
         c1 = 1.0f - powf(g->opts.beta1, (float)g->step);
         c2 = 1.0f - powf(g->opts.beta2, (float)g->step);
     }
-    k_adam<<<(GP_N + ADAM_PARAMS - 1) / ADAM_PARAMS, ADAM_WAVES * 64, 0, st>>>(g->P.p, g->m.p, g->v.p, g->partial.p, nwg, 1.0f, lr, g->opts.beta1,
-                                               g->opts.beta2, c1, c2, g->opts.eps, grad_out);
-    if ((e = hipGetLastError()) != hipSuccess) return hip_error(e, "guide train launch");
-    return adam ? guide_pack(g, st) : LMX_OK;
+    k_adam<<<(GP_N + ADAM_PARAMS - 1) / ADAM_PARAMS, ADAM_WAVES * 64, 0, st>>>(
+        g->P.p, g->m.p, g->v.p, g->partial.p, nwg, lr, g->opts.beta1, g->opts.beta2, c1, c2, g->opts.eps, grad_out,
+        g->loss_part.p, g->h_loss, g->pack.p, g->bias.p);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? LMX_OK : hip_error(e, "guide train launch");
 }
 
 void init_params(std::vector<float>& P, uint64_t seed)
@@ -1170,11 +1217,12 @@ int lmx_guide_create(lmx_scene* sc, const lmx_guide_opts* o, lmx_guide** out)
     g->nparts = std::max(1, sc->cus);
     if ((e = g->P.alloc(GP_N)) != hipSuccess || (e = g->m.alloc(GP_N)) != hipSuccess ||
         (e = g->v.alloc(GP_N)) != hipSuccess || (e = g->grad.alloc(GP_N)) != hipSuccess ||
-        (e = g->partial.alloc((size_t)g->nparts * GP_N)) != hipSuccess || (e = g->loss.alloc(1)) != hipSuccess ||
+        (e = g->partial.alloc((size_t)g->nparts * GP_PAD)) != hipSuccess ||
+        (e = g->loss_part.alloc(g->nparts)) != hipSuccess ||
+        (e = hipHostMalloc((void**)&g->h_loss, sizeof(float), hipHostMallocDefault)) != hipSuccess ||
         (e = g->wsum.alloc(1)) != hipSuccess || (e = g->pack.alloc((size_t)N_PACK * 8)) != hipSuccess ||
         (e = g->bias.alloc(N_BIAS)) != hipSuccess || (e = g->rec_count.alloc(1)) != hipSuccess ||
-        (e = g->idx.alloc(g->opts.batch)) != hipSuccess || (e = g->nz_count.alloc(1)) != hipSuccess ||
-        (e = g->act.alloc((size_t)NROWS * ((g->opts.batch + 31) / 32 * 32))) != hipSuccess)
+        (e = g->idx.alloc(g->opts.batch)) != hipSuccess || (e = g->nz_count.alloc(1)) != hipSuccess)
         return hip_error(e, "lmx_guide_create: device memory");
     std::vector<float> P;
     init_params(P, g->opts.seed);
@@ -1254,10 +1302,8 @@ int lmx_guide_grad(lmx_guide* g, const float* recs, uint32_t n, float* grad, flo
     int rc = guide_train_step(g, reinterpret_cast<const float4*>(recs), nullptr, n, 1.0f, 3.0e38f, adam != 0,
                               grad ? grad : g->grad.p, st);
     hipError_t e;
-    if (rc == LMX_OK && loss &&
-        (e = hipMemcpyAsync(loss, g->loss.p, sizeof(float), hipMemcpyDeviceToHost, st)) != hipSuccess)
-        rc = hip_error(e, "lmx_guide_grad: loss");
     if (rc == LMX_OK && (e = hipStreamSynchronize(st)) != hipSuccess) rc = hip_error(e, "lmx_guide_grad: sync");
+    if (rc == LMX_OK && loss) *loss = *g->h_loss;
     return rc;
 }
 
@@ -1365,13 +1411,10 @@ int lmx_render_guided(lmx_scene* sc, lmx_guide* g, const lmx_render_params* p, i
                                                          make_uint2((uint32_t)g->opts.seed, (uint32_t)(g->opts.seed >> 32)),
                                                          (uint32_t)g->step);
                 rc = guide_train_step(g, g->recs.p, g->idx.p, m, wnorm, g->opts.wclamp, true, nullptr, st);
-                float l = 0.0f;
-                if (rc == LMX_OK && k + 1 == g->opts.steps_per_pass) {
-                    if ((e = hipMemcpyAsync(&l, g->loss.p, 4, hipMemcpyDeviceToHost, st)) != hipSuccess ||
-                        (e = hipStreamSynchronize(st)) != hipSuccess)
-                        rc = hip_error(e, "guide loss readback");
-                    loss_sum = l;
-                }
+            }
+            if (rc == LMX_OK && g->opts.steps_per_pass > 0) {
+                if ((e = hipStreamSynchronize(st)) != hipSuccess) rc = hip_error(e, "guide loss readback");
+                else loss_sum = *g->h_loss;
             }
         }
         nrec_nz = nnz;

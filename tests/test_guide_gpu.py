@@ -164,3 +164,35 @@ def test_guided_render_unbiased_and_training_helps(gpu, cornell):
     mg, mp = G.mean(axis=(1, 2, 3)), P.mean(axis=(1, 2, 3))
     se = np.sqrt(mg.var(ddof=1) / kg + mp.var(ddof=1) / kp)
     assert abs(mg.mean() - mp.mean()) < 3.5 * se, (mg.mean(), mp.mean(), se)
+
+
+@pytest.mark.parametrize("n", [1, 15, 17, 64, 65, 1000, 16384 + 33])
+def test_training_step_edges(gpu, cornell, n):
+    """Record counts around the kernel's 16 records per wave, 64 per step and
+    one step per workgroup: gradient and loss against the oracle's bf16
+    network (the bars of the minibatch test), and, after an Adam step, the
+    operands the optimiser wrote against those packed from the parameters:
+    the same outputs and the same gradient, bit for bit."""
+    import torch
+    g = guide.Guide(cornell, lr=1e-2)
+    P = _params(3)
+    g.params = P.astype(np.float32)
+    rng = np.random.default_rng(n)
+    rec, x, d, pb, w = _records(n, n)
+    recs = torch.from_numpy(rec).to(gpu)
+    grad, loss = g.grad(recs)
+    again, loss2 = g.grad(recs)
+    assert torch.equal(grad, again) and loss == loss2
+    lo, go = orc.guide_loss(P, x, d, pb, w, bf16=True)
+    gg = grad.cpu().numpy().astype(np.float64)
+    assert abs(loss - lo) < 2e-3 * abs(lo) + 1e-3, (loss, lo)
+    # the minibatch test's bar; few records: about ten bf16 roundings (2^-8) in a row, unaveraged
+    assert np.linalg.norm(gg - go) <= (0.03 if n >= 1000 else 0.05) * np.linalg.norm(go)
+    g.grad(recs, adam=True)
+    xs = torch.from_numpy(rng.random((500, 7)).astype(np.float32)).to(gpu)
+    y, (g1, l1) = g.eval(xs), g.grad(recs)
+    p = g.params
+    assert np.abs(p - P.astype(np.float32)).max() > 1e-3
+    g.params = p                                   # packs every operand from the parameters
+    y2, (g2, l2) = g.eval(xs), g.grad(recs)
+    assert torch.equal(y, y2) and torch.equal(g1, g2) and l1 == l2
