@@ -46,7 +46,7 @@
 //               re-evaluation per strategy), and appends a shadow ray;
 //   trace    -- any-hit traversal of the shadow rays;
 //   splat    -- unoccluded contributions to the film.
-// The whole batch is captured once as a hipGraph and replayed per batch.
+// A batch that comes again is captured as a hipGraph and replayed.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1810,7 +1810,19 @@ uint32_t bd_conn_per_sample(uint32_t maxv, int variant, bool bounded, bool conne
 // for unbounded renderer::bdpt).
 #define BD_ROUND_SLOTS 24u
 
+// But while the worst case of the whole batch takes at most this many bytes,
+// the queue holds it: then one round is certain to be enough and nothing has
+// to be read back to know that no sample is left (about 50 us per batch, 1.2
+// GB for 262,144 samples of renderer::vcm at 10 vertices).
+#define BD_WHOLE_QUEUE_BYTES (4ull << 30)
+#define BD_SLOT_BYTES 96u
+
 uint32_t bd_round_slots(uint32_t worst) { return std::min(worst, BD_ROUND_SLOTS); }
+
+size_t bd_round_queue(uint32_t B, uint32_t worst)
+{
+    return std::max((size_t)B * bd_round_slots(worst), (size_t)worst);
+}
 
 // Device bytes of one batch slot: two subpaths of vertex records, their
 // queues and hits, the connection count, and the shadow-ray records of one
@@ -1847,11 +1859,11 @@ size_t bd_held_bytes(const lmx_scene* sc)
 
 // Buffers for batches of B samples of up to maxv vertices and `conn`
 // shadow-queue slots per sample.  With `rounds` (the samplers that connect
-// in rounds), conn is a sample's worst case and the queue holds one round:
-// B x bd_round_slots(conn) slots, never fewer than one sample's worst case.
-int bd_buffers(lmx_scene* sc, uint32_t B, uint32_t maxv, uint32_t conn, bool rounds = false)
+// in rounds), conn is a sample's worst case and the queue holds the whole
+// batch's where that is small, else one round (never less than one sample's
+// worst case).
+int bd_buffers_of(lmx_scene* sc, uint32_t B, uint32_t maxv, uint32_t conn, size_t nconn)
 {
-    const size_t nconn = rounds ? std::max((size_t)B * bd_round_slots(conn), (size_t)conn) : (size_t)B * conn;
     if (nconn > 0xffffffffull) return set_error(LMX_EINVAL, "bdpt buffers: more than 2^32 - 1 connection slots");
     if (B <= sc->bd_batch && maxv <= sc->bd_maxv && nconn <= sc->bd_nconn) return LMX_OK;
     bd_release(sc);
@@ -1883,6 +1895,31 @@ int bd_buffers(lmx_scene* sc, uint32_t B, uint32_t maxv, uint32_t conn, bool rou
     sc->bd_conn = conn;
     sc->bd_nconn = (uint32_t)nconn;
     return LMX_OK;
+}
+
+int bd_buffers(lmx_scene* sc, uint32_t B, uint32_t maxv, uint32_t conn, bool rounds = false)
+{
+    const size_t whole = (size_t)B * conn;
+    if (!rounds) return bd_buffers_of(sc, B, maxv, conn, whole);
+    if ((uint64_t)whole * BD_SLOT_BYTES <= BD_WHOLE_QUEUE_BYTES) {
+        if (bd_buffers_of(sc, B, maxv, conn, whole) == LMX_OK) return LMX_OK;
+        (void)hipGetLastError();               // no room for that: rounds need less
+    }
+    return bd_buffers_of(sc, B, maxv, conn, bd_round_queue(B, conn));
+}
+
+// The batch's buffers.
+VB bd_vertex_buffers(const lmx_scene* sc)
+{
+    VB vb;
+    vb.v[0] = sc->bd_vert[0].p; vb.v[1] = sc->bd_vert[1].p;
+    vb.nsub[0] = sc->bd_nsub[0].p; vb.nsub[1] = sc->bd_nsub[1].p;
+    vb.epix = sc->bd_epix.p; vb.eraster = sc->bd_eraster.p;
+    vb.V = sc->bd_V.p;
+    vb.mq = sc->vc_mq.p;
+    vb.off = sc->bd_off.p;
+    vb.dmask = sc->bd_dmask.p;
+    return vb;
 }
 
 // Records the subpaths of one batch of `bp` samples into vb's vertex records:
@@ -1940,13 +1977,13 @@ int bd_enqueue_round(lmx_scene* sc, const BParams& bp, const VB& vb, hipStream_t
     return LMX_OK;
 }
 
-// Connection rounds a batch graph holds: one when a round can take every
-// sample at its worst case, else two, after which the host checks for
-// samples left over (rarely any: the round slots exceed the typical count).
-int bd_graph_rounds(const lmx_scene* sc, const BParams& bp)
+// Whether one connection round is certain to take every sample of a batch.
+// If not, the host reads the round cursor after each round (the first mostly
+// is enough: the round slots exceed the typical count).
+bool bd_one_round(const lmx_scene* sc, const BParams& bp)
 {
     const uint32_t worst = bd_conn_per_sample((uint32_t)bp.maxv, bp.variant, bp.bounded != 0, bp.connect != 0);
-    return (uint64_t)sc->bd_nconn >= (uint64_t)bp.batch * worst ? 1 : 2;
+    return (uint64_t)sc->bd_nconn >= (uint64_t)bp.batch * worst;
 }
 
 // Records one batch: generation, subpath iterations, connections, shadow
@@ -1954,14 +1991,7 @@ int bd_graph_rounds(const lmx_scene* sc, const BParams& bp)
 int bd_enqueue_batch(lmx_scene* sc, const BParams& bp, hipStream_t st)
 {
     const uint32_t B = bp.batch;
-    VB vb;
-    vb.v[0] = sc->bd_vert[0].p; vb.v[1] = sc->bd_vert[1].p;
-    vb.nsub[0] = sc->bd_nsub[0].p; vb.nsub[1] = sc->bd_nsub[1].p;
-    vb.epix = sc->bd_epix.p; vb.eraster = sc->bd_eraster.p;
-    vb.V = sc->bd_V.p;
-    vb.mq = sc->vc_mq.p;
-    vb.off = sc->bd_off.p;
-    vb.dmask = sc->bd_dmask.p;
+    const VB vb = bd_vertex_buffers(sc);
     Queue q[2];
     for (int k = 0; k < 2; k++) { q[k].ray = sc->bd_ray[k].p; q[k].thr = sc->bd_thr[k].p; q[k].meta = sc->bd_meta[k].p; }
     BCtl* ctl = sc->bd_ctl.p;
@@ -1977,10 +2007,7 @@ int bd_enqueue_batch(lmx_scene* sc, const BParams& bp, hipStream_t st)
         k_scan_add<<<std::max(1, std::min((int)((B + 1 + 255) / 256), cap_grid)), 256, 0, st>>>(vb.off, B + 1, sc->bd_part.p);
     }
     k_bd_conn_start<<<1, 64, 0, st>>>(ctl);
-    const int rounds = bd_graph_rounds(sc, bp);
-    for (int k = 0; k < rounds; k++) {
-        if ((rc = bd_enqueue_round(sc, bp, vb, st)) != LMX_OK) return rc;
-    }
+    if ((rc = bd_enqueue_round(sc, bp, vb, st)) != LMX_OK) return rc;
     if (bp.merging) {
         VB ph = vb;
         ph.v[1] = sc->vc_vert.p; ph.nsub[1] = sc->vc_nsub.p;
@@ -1993,22 +2020,14 @@ int bd_enqueue_batch(lmx_scene* sc, const BParams& bp, hipStream_t st)
     return e == hipSuccess ? LMX_OK : hip_error(e, "bdpt launch");
 }
 
-// Captures one connection round as a graph.
-int bd_round_graph(lmx_scene* sc, const BParams& bp, hipStream_t st, hipGraphExec_t* exec)
+// Captures what `record` enqueues on a stream as an executable graph.
+template <typename F>
+int capture(hipStream_t st, hipGraphExec_t* exec, F&& record)
 {
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return hip_error(e, "capture");
-    VB vb;
-    vb.v[0] = sc->bd_vert[0].p; vb.v[1] = sc->bd_vert[1].p;
-    vb.nsub[0] = sc->bd_nsub[0].p; vb.nsub[1] = sc->bd_nsub[1].p;
-    vb.epix = sc->bd_epix.p; vb.eraster = sc->bd_eraster.p;
-    vb.V = sc->bd_V.p;
-    vb.mq = sc->vc_mq.p;
-    vb.off = sc->bd_off.p;
-    vb.dmask = sc->bd_dmask.p;
-    int rc = bd_enqueue_round(sc, bp, vb, st);
-    if (rc == LMX_OK && (e = hipGetLastError()) != hipSuccess) rc = hip_error(e, "bdpt launch");
+    int rc = record();
     e = hipStreamEndCapture(st, &graph);
     if (rc == LMX_OK && e != hipSuccess) rc = hip_error(e, "capture end");
     if (rc == LMX_OK && (e = hipGraphInstantiate(exec, graph, nullptr, nullptr, 0)) != hipSuccess)
@@ -2017,52 +2036,61 @@ int bd_round_graph(lmx_scene* sc, const BParams& bp, hipStream_t st, hipGraphExe
     return rc;
 }
 
-// The graphs of one batch shape: the batch itself (with its in-graph
-// connection rounds) and, when those rounds may not be enough, one more
-// round to replay until every sample is connected.
-struct BGraphs {
-    hipGraphExec_t batch = nullptr, round = nullptr;
-    uint32_t B = 0;
-    ~BGraphs()
-    {
-        if (batch) (void)hipGraphExecDestroy(batch);
-        if (round) (void)hipGraphExecDestroy(round);
-    }
-};
-
-// Captures one batch as a graph (and the extra round when needed).
-int bd_graph(lmx_scene* sc, const BParams& bp, hipStream_t st, BGraphs& g)
+// The stream graphs are recorded on; it runs nothing.
+int bd_record_stream(lmx_scene* sc, hipStream_t* cs)
 {
-    hipGraph_t graph = nullptr;
-    hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
-    if (e != hipSuccess) return hip_error(e, "capture");
-    int rc = bd_enqueue_batch(sc, bp, st);
-    e = hipStreamEndCapture(st, &graph);
-    if (rc == LMX_OK && e != hipSuccess) rc = hip_error(e, "capture end");
-    if (rc == LMX_OK && (e = hipGraphInstantiate(&g.batch, graph, nullptr, nullptr, 0)) != hipSuccess)
-        rc = hip_error(e, "graph instantiate");
-    if (graph) (void)hipGraphDestroy(graph);
-    g.B = bp.batch;
-    if (rc == LMX_OK && bd_graph_rounds(sc, bp) > 1) rc = bd_round_graph(sc, bp, st, &g.round);
-    return rc;
+    if (!sc->cap_stream) {
+        const hipError_t e = hipStreamCreateWithFlags(&sc->cap_stream, hipStreamNonBlocking);
+        if (e != hipSuccess) {
+            sc->cap_stream = nullptr;
+            return hip_error(e, "capture stream");
+        }
+    }
+    *cs = sc->cap_stream;
+    return LMX_OK;
 }
 
-// Runs one batch: its graph; then, when its rounds may have left samples
-// unconnected, a read of the round cursor and further rounds until none is
-// left; then the advance to the next batch.
-int bd_run_batch(lmx_scene* sc, const BGraphs& g, hipStream_t st)
+// A step that a render repeats (a photon phase, an eye batch): the first
+// time it is enqueued kernel by kernel, and only a step that comes again is
+// recorded as a graph, while the GPU works on the first.  Instantiating the
+// graph first left the GPU idle for 150 to 380 us a render, as long as a
+// small frame's own work.
+struct BStep {
+    hipGraphExec_t exec = nullptr;
+    ~BStep() { if (exec) (void)hipGraphExecDestroy(exec); }
+};
+
+template <typename F>
+int bd_step(lmx_scene* sc, BStep& g, bool again, hipStream_t st, F&& record)
 {
-    hipError_t e = hipGraphLaunch(g.batch, st);
-    if (e != hipSuccess) return hip_error(e, "graph launch");
-    while (g.round) {
+    if (g.exec) {
+        const hipError_t e = hipGraphLaunch(g.exec, st);
+        return e == hipSuccess ? LMX_OK : hip_error(e, "graph launch");
+    }
+    int rc = record(st);
+    if (rc != LMX_OK || !again) return rc;
+    hipStream_t cs = nullptr;
+    if ((rc = bd_record_stream(sc, &cs)) != LMX_OK) return rc;
+    return capture(cs, &g.exec, [&] { return record(cs); });
+}
+
+// Runs one batch; when its round may have left samples unconnected, a read
+// of the round cursor and further rounds until none is left; then the advance
+// to the next batch.  again: more batches of this shape will follow.
+int bd_run_batch(lmx_scene* sc, const BParams& bp, BStep& g, bool again, hipStream_t st)
+{
+    int rc = bd_step(sc, g, again, st, [&](hipStream_t s) { return bd_enqueue_batch(sc, bp, s); });
+    if (rc != LMX_OK) return rc;
+    hipError_t e;
+    while (!bd_one_round(sc, bp)) {
         if ((e = hipMemcpyAsync(&sc->bd_hctl->conn_next, &sc->bd_ctl.p->conn_next, sizeof(uint32_t),
                                 hipMemcpyDeviceToHost, st)) != hipSuccess ||
             (e = hipStreamSynchronize(st)) != hipSuccess)
             return hip_error(e, "connection rounds");
-        if (sc->bd_hctl->conn_next >= g.B) break;
-        if ((e = hipGraphLaunch(g.round, st)) != hipSuccess) return hip_error(e, "graph launch");
+        if (sc->bd_hctl->conn_next >= bp.batch) break;
+        if ((rc = bd_enqueue_round(sc, bp, bd_vertex_buffers(sc), st)) != LMX_OK) return rc;
     }
-    k_bd_next_batch<<<1, 64, 0, st>>>(sc->bd_ctl.p, g.B);
+    k_bd_next_batch<<<1, 64, 0, st>>>(sc->bd_ctl.p, bp.batch);
     e = hipGetLastError();
     return e == hipSuccess ? LMX_OK : hip_error(e, "bdpt launch");
 }
@@ -2111,18 +2139,18 @@ int bd_autotune(lmx_scene* sc, BParams bp, uint64_t num_samples, float* film, hi
         if (B != cands[0] && ((size_t)B * per > budget || B > want)) break;
         bp.batch = B;
         bp.total = 2u * B;
-        BGraphs g;
+        BStep g;
         if ((rc = bd_buffers(sc, B, (uint32_t)bp.maxv, conn, true)) != LMX_OK ||
-            (rc = bd_graph(sc, bp, st, g)) != LMX_OK) {
+            (rc = capture(st, &g.exec, [&] { return bd_enqueue_batch(sc, bp, st); })) != LMX_OK) {
             if (best_rate < 0.0) break;        // not even the smallest size fits: report it
             (void)hipGetLastError();           // a larger candidate failed: keep the best so far
             rc = LMX_OK;
             break;
         }
         k_bd_init<<<1, 64, 0, st>>>(sc->bd_ctl.p);
-        if ((rc = bd_run_batch(sc, g, st)) != LMX_OK) break;
+        if ((rc = bd_run_batch(sc, bp, g, true, st)) != LMX_OK) break;
         (void)hipEventRecord(e0, st);
-        rc = bd_run_batch(sc, g, st);
+        rc = bd_run_batch(sc, bp, g, true, st);
         (void)hipEventRecord(e1, st);
         const hipError_t es = hipEventSynchronize(e1);
         if (rc != LMX_OK) break;
@@ -2143,8 +2171,8 @@ int bd_autotune(lmx_scene* sc, BParams bp, uint64_t num_samples, float* film, hi
     return rc;
 }
 
-// One render of either variant: batches of B samples, each replayed from one
-// captured graph; the film scaled by W H / N at the end.
+// One render of either variant: batches of B samples, all but the first
+// replayed from one captured graph; the film scaled by W H / N at the end.
 int render_bidir(lmx_scene* sc, const lmx_render_params* p, int variant, const char* name, float* film_rgb,
                  void* stream, lmx_render_stats* stats)
 {
@@ -2221,23 +2249,22 @@ int render_bidir(lmx_scene* sc, const lmx_render_params* p, int variant, const c
     if (rc == LMX_OK) rc = bd_buffers(sc, B, maxv, bd_conn_per_sample(maxv, variant, bounded), true);
     const size_t npix = (size_t)sc->width * (size_t)sc->height;
     const int zgrid = std::max(1, std::min((int)((3 * npix + 255) / 256), sc->cus * 8));
-    BGraphs g;
+    BStep g;
     if (rc == LMX_OK) {
         k_bd_zero<<<zgrid, 256, 0, st>>>(film_rgb, 3 * npix);
         k_bd_init<<<1, 64, 0, st>>>(sc->bd_ctl.p);
-        rc = bd_graph(sc, bp, st, g);
     }
     uint64_t nbatch = (num_samples + B - 1) / B;
     uint64_t taken = p->num_samples;
     if (!timed) {
-        for (uint64_t b = 0; rc == LMX_OK && b < nbatch; b++) rc = bd_run_batch(sc, g, st);
+        for (uint64_t b = 0; rc == LMX_OK && b < nbatch; b++) rc = bd_run_batch(sc, bp, g, nbatch > 1, st);
     } else {
         // the scheduler's time mode: whole batches until the deadline, each
         // finished before the clock is read (scheduler.cpp:108,191-199)
         const auto ts = std::chrono::steady_clock::now();
         uint64_t b = 0;
         while (rc == LMX_OK && b < nbatch) {
-            if ((rc = bd_run_batch(sc, g, st)) != LMX_OK) break;
+            if ((rc = bd_run_batch(sc, bp, g, true, st)) != LMX_OK) break;
             if ((e = hipStreamSynchronize(st)) != hipSuccess) {
                 rc = hip_error(e, "graph launch");
                 break;
@@ -2345,22 +2372,6 @@ int vc_enqueue_photons(lmx_scene* sc, const BParams& pp, hipStream_t st, bool gr
     return e == hipSuccess ? LMX_OK : hip_error(e, "vcm photon launch");
 }
 
-// Captures a phase (photons, or one eye batch) as a graph.
-template <typename F>
-int capture(hipStream_t st, hipGraphExec_t* exec, F&& record)
-{
-    hipGraph_t graph = nullptr;
-    hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
-    if (e != hipSuccess) return hip_error(e, "capture");
-    int rc = record();
-    e = hipStreamEndCapture(st, &graph);
-    if (rc == LMX_OK && e != hipSuccess) rc = hip_error(e, "capture end");
-    if (rc == LMX_OK && (e = hipGraphInstantiate(exec, graph, nullptr, nullptr, 0)) != hipSuccess)
-        rc = hip_error(e, "graph instantiate");
-    if (graph) (void)hipGraphDestroy(graph);
-    return rc;
-}
-
 // renderer::vcm, modes vcm and bdpm: per pass the photon graph, then the eye
 // batches (each one graph: subpaths, connections, shadow rays, merges); the
 // film holds the sum of every pass's splats, scaled at the end by
@@ -2435,8 +2446,7 @@ int render_vcm(lmx_scene* sc, const lmx_render_params* p, const lmx_vcm_params* 
     if (rc == LMX_OK) rc = vc_buffers(sc, np, maxv, B);
     const size_t npix = (size_t)sc->width * (size_t)sc->height;
     const int zgrid = std::max(1, std::min((int)((3 * npix + 255) / 256), sc->cus * 8));
-    hipGraphExec_t gph = nullptr;
-    BGraphs geye;
+    BStep gph, geye;
     if (rc == LMX_OK) {
         k_bd_zero<<<zgrid, 256, 0, st>>>(film_rgb, 3 * npix);
         if (p->sample_out) {
@@ -2445,9 +2455,7 @@ int render_vcm(lmx_scene* sc, const lmx_render_params* p, const lmx_vcm_params* 
                 p->sample_out, ns);
         }
         k_bd_init<<<1, 64, 0, st>>>(sc->bd_ctl.p);
-        rc = capture(st, &gph, [&] { return vc_enqueue_photons(sc, pp, st); });
     }
-    if (rc == LMX_OK) rc = bd_graph(sc, bp, st, geye);
     const uint64_t nbatch = ((uint64_t)Ne + B - 1) / B;
     double r = v->initial_radius;
     for (uint32_t q = 0; rc == LMX_OK && q < v->num_iteration_pass; q++) {
@@ -2455,9 +2463,11 @@ int render_vcm(lmx_scene* sc, const lmx_render_params* p, const lmx_vcm_params* 
         const double a = 3.14159265358979323846 * r * r;
         const float rf = (float)r, cell = (float)(2.0 * r), cm = (float)((double)np * a * a);
         k_bd_phase<<<1, 64, 0, st>>>(sc->bd_ctl.p, q * np, rf, cell, cm);
-        if ((e = hipGraphLaunch(gph, st)) != hipSuccess) { rc = hip_error(e, "graph launch"); break; }
+        rc = bd_step(sc, gph, v->num_iteration_pass > 1, st, [&](hipStream_t cs) { return vc_enqueue_photons(sc, pp, cs); });
+        if (rc != LMX_OK) break;
         k_bd_phase<<<1, 64, 0, st>>>(sc->bd_ctl.p, q * Ne, rf, cell, cm);
-        for (uint64_t b = 0; rc == LMX_OK && b < nbatch; b++) rc = bd_run_batch(sc, geye, st);
+        for (uint64_t b = 0; rc == LMX_OK && b < nbatch; b++)
+            rc = bd_run_batch(sc, bp, geye, v->num_iteration_pass > 1 || nbatch > 1, st);
     }
     if (rc == LMX_OK) {
         k_bd_scale<<<zgrid, 256, 0, st>>>(film_rgb, 3 * npix,
@@ -2466,7 +2476,6 @@ int render_vcm(lmx_scene* sc, const lmx_render_params* p, const lmx_vcm_params* 
             (e = hipStreamSynchronize(st)) != hipSuccess)
             rc = hip_error(e, "lmx_render_vcm: sync");
     }
-    if (gph) (void)hipGraphExecDestroy(gph);
     if (own) (void)hipStreamDestroy(own);
     if (stats) {
         stats->rays = rc == LMX_OK ? sc->bd_hctl->rays + sc->bd_hctl->shadow_rays : 0;
@@ -2577,30 +2586,26 @@ int render_pm(lmx_scene* sc, const lmx_render_params* p, const lmx_pm_params* v,
     if (rc == LMX_OK) rc = vc_buffers(sc, np, pcap, 1);
     const size_t npix = (size_t)sc->width * (size_t)sc->height;
     const int zgrid = std::max(1, std::min((int)((3 * npix + 255) / 256), sc->cus * 8));
-    hipGraphExec_t gph = nullptr, geye = nullptr;
+    BStep geye;
     if (rc == LMX_OK) {
         k_bd_zero<<<zgrid, 256, 0, st>>>(film_rgb, 3 * npix);
         k_bd_init<<<1, 64, 0, st>>>(sc->bd_ctl.p);
-        rc = capture(st, &gph, [&] { return vc_enqueue_photons(sc, pp, st); });
     }
-    if (rc == LMX_OK) rc = capture(st, &geye, [&] { return pm_enqueue_eye(sc, bp, pa, st); });
     const float r = v->radius;
     if (rc == LMX_OK) {
         k_bd_phase<<<1, 64, 0, st>>>(sc->bd_ctl.p, 0u, r, (float)(2.0 * (double)r), 0.0f);
-        if ((e = hipGraphLaunch(gph, st)) != hipSuccess) rc = hip_error(e, "graph launch");
+        rc = vc_enqueue_photons(sc, pp, st);
     }
     const uint64_t nbatch = ((uint64_t)N + B - 1) / B;
     if (rc == LMX_OK) k_bd_phase<<<1, 64, 0, st>>>(sc->bd_ctl.p, 0u, r, (float)(2.0 * (double)r), 0.0f);
     for (uint64_t b = 0; rc == LMX_OK && b < nbatch; b++)
-        if ((e = hipGraphLaunch(geye, st)) != hipSuccess) rc = hip_error(e, "graph launch");
+        rc = bd_step(sc, geye, nbatch > 1, st, [&](hipStream_t cs) { return pm_enqueue_eye(sc, bp, pa, cs); });
     if (rc == LMX_OK) {
         k_bd_scale<<<zgrid, 256, 0, st>>>(film_rgb, 3 * npix, (float)((double)npix / (double)N));
         if ((e = hipMemcpyAsync(sc->bd_hctl, sc->bd_ctl.p, sizeof(BCtl), hipMemcpyDeviceToHost, st)) != hipSuccess ||
             (e = hipStreamSynchronize(st)) != hipSuccess)
             rc = hip_error(e, "lmx_render_pm: sync");
     }
-    if (gph) (void)hipGraphExecDestroy(gph);
-    if (geye) (void)hipGraphExecDestroy(geye);
     if (own) (void)hipStreamDestroy(own);
     if (stats) {
         stats->rays = rc == LMX_OK ? sc->bd_hctl->rays : 0;
@@ -2685,7 +2690,7 @@ int render_ppm(lmx_scene* sc, const lmx_render_params* p, const lmx_ppm_params* 
     const int zgrid = std::max(1, std::min((int)((3 * npix + 255) / 256), sc->cus * 8));
     const int mgrid = std::max(1, std::min((int)((N + 255) / 256), sc->cus * 16));
     const float r0 = v->initial_radius, cell = (float)(2.0 * (double)r0);
-    hipGraphExec_t gph = nullptr;
+    BStep gph;
     VB vb;
     vb.v[0] = sc->bd_vert[0].p; vb.v[1] = sc->bd_vert[1].p;
     vb.nsub[0] = sc->bd_nsub[0].p; vb.nsub[1] = sc->bd_nsub[1].p;
@@ -2710,10 +2715,10 @@ int render_ppm(lmx_scene* sc, const lmx_render_params* p, const lmx_ppm_params* 
             if ((e = hipGetLastError()) != hipSuccess) rc = hip_error(e, "ppm launch");
         }
     }
-    if (rc == LMX_OK) rc = capture(st, &gph, [&] { return vc_enqueue_photons(sc, pp, st); });
     for (uint32_t q = 0; rc == LMX_OK && q < v->num_iteration_pass; q++) {
         k_bd_phase<<<1, 64, 0, st>>>(sc->bd_ctl.p, q * np, r0, cell, 0.0f);
-        if ((e = hipGraphLaunch(gph, st)) != hipSuccess) { rc = hip_error(e, "graph launch"); break; }
+        rc = bd_step(sc, gph, v->num_iteration_pass > 1, st, [&](hipStream_t cs) { return vc_enqueue_photons(sc, pp, cs); });
+        if (rc != LMX_OK) break;
         k_ppm_update<<<mgrid, 256, 0, st>>>(sc->rs, bp, sc->bd_ctl.p, vb, ph, g, pa, sc->ppm_st.p, v->alpha);
     }
     if (rc == LMX_OK) {
@@ -2726,7 +2731,6 @@ int render_ppm(lmx_scene* sc, const lmx_render_params* p, const lmx_ppm_params* 
         ((e = hipMemcpyAsync(sc->bd_hctl, sc->bd_ctl.p, sizeof(BCtl), hipMemcpyDeviceToHost, st)) != hipSuccess ||
          (e = hipStreamSynchronize(st)) != hipSuccess))
         rc = hip_error(e, "lmx_render_ppm: sync");
-    if (gph) (void)hipGraphExecDestroy(gph);
     if (own) (void)hipStreamDestroy(own);
     if (stats) {
         stats->rays = rc == LMX_OK ? sc->bd_hctl->rays : 0;
@@ -2816,26 +2820,26 @@ int render_sppm(lmx_scene* sc, const lmx_render_params* p, const lmx_ppm_params*
     VB ph = vb;
     ph.v[1] = sc->vc_vert.p; ph.nsub[1] = sc->vc_nsub.p;
     const Grid g{sc->vc_items.p, sc->vc_start.p, sc->vc_cursor.p, sc->vc_part.p, sc->vc_H};
-    hipGraphExec_t gph = nullptr, geye = nullptr;
+    BStep gph, geye;
     if (rc == LMX_OK) {
         k_bd_init<<<1, 64, 0, st>>>(sc->bd_ctl.p);
         k_sppm_init<<<mgrid, 256, 0, st>>>(sc->ppm_st.p, npix, r0);
-        rc = capture(st, &gph, [&] { return vc_enqueue_photons(sc, pp, st); });
     }
-    if (rc == LMX_OK)
-        rc = capture(st, &geye, [&] {
-            Queue q[2];
-            for (int k = 0; k < 2; k++) { q[k].ray = sc->bd_ray[k].p; q[k].thr = sc->bd_thr[k].p; q[k].meta = sc->bd_meta[k].p; }
-            const int rc2 = bd_enqueue_subpaths(sc, bp, vb, q, sc->bd_hits.p, npix, st);
-            if (rc2 != LMX_OK) return rc2;
-            const hipError_t e2 = hipGetLastError();
-            return e2 == hipSuccess ? LMX_OK : hip_error(e2, "sppm launch");
-        });
+    auto eye = [&](hipStream_t cs) {
+        Queue q[2];
+        for (int k = 0; k < 2; k++) { q[k].ray = sc->bd_ray[k].p; q[k].thr = sc->bd_thr[k].p; q[k].meta = sc->bd_meta[k].p; }
+        const int rc2 = bd_enqueue_subpaths(sc, bp, vb, q, sc->bd_hits.p, npix, cs);
+        if (rc2 != LMX_OK) return rc2;
+        const hipError_t e2 = hipGetLastError();
+        return e2 == hipSuccess ? LMX_OK : hip_error(e2, "sppm launch");
+    };
+    const bool again = v->num_iteration_pass > 1;
     for (uint32_t q = 0; rc == LMX_OK && q < v->num_iteration_pass; q++) {
         k_bd_phase<<<1, 64, 0, st>>>(sc->bd_ctl.p, q * npix, r0, cell, 0.0f);
-        if ((e = hipGraphLaunch(geye, st)) != hipSuccess) { rc = hip_error(e, "graph launch"); break; }
+        if ((rc = bd_step(sc, geye, again, st, eye)) != LMX_OK) break;
         k_bd_phase<<<1, 64, 0, st>>>(sc->bd_ctl.p, q * np, r0, cell, 0.0f);
-        if ((e = hipGraphLaunch(gph, st)) != hipSuccess) { rc = hip_error(e, "graph launch"); break; }
+        rc = bd_step(sc, gph, again, st, [&](hipStream_t cs) { return vc_enqueue_photons(sc, pp, cs); });
+        if (rc != LMX_OK) break;
         k_sppm_update<<<mgrid, 256, 0, st>>>(sc->rs, bp, sc->bd_ctl.p, vb, ph, g, pa, sc->ppm_st.p, v->alpha);
     }
     if (rc == LMX_OK) {
@@ -2847,8 +2851,6 @@ int render_sppm(lmx_scene* sc, const lmx_render_params* p, const lmx_ppm_params*
         ((e = hipMemcpyAsync(sc->bd_hctl, sc->bd_ctl.p, sizeof(BCtl), hipMemcpyDeviceToHost, st)) != hipSuccess ||
          (e = hipStreamSynchronize(st)) != hipSuccess))
         rc = hip_error(e, "lmx_render_sppm: sync");
-    if (gph) (void)hipGraphExecDestroy(gph);
-    if (geye) (void)hipGraphExecDestroy(geye);
     if (own) (void)hipStreamDestroy(own);
     if (stats) {
         stats->rays = rc == LMX_OK ? sc->bd_hctl->rays : 0;
@@ -2910,7 +2912,7 @@ int render_ltdirect(lmx_scene* sc, const lmx_render_params* p, float* film_rgb, 
     const size_t npix = (size_t)sc->width * (size_t)sc->height;
     const int zgrid = std::max(1, std::min((int)((3 * npix + 255) / 256), sc->cus * 8));
     const int cap_grid = sc->cus * 8;
-    hipGraphExec_t gb = nullptr;
+    BStep gb;
     if (rc == LMX_OK) {
         k_bd_zero<<<zgrid, 256, 0, st>>>(film_rgb, 3 * npix);
         if (p->sample_out) {
@@ -2919,33 +2921,33 @@ int render_ltdirect(lmx_scene* sc, const lmx_render_params* p, float* film_rgb, 
                 p->sample_out, ns);
         }
         k_bd_init<<<1, 64, 0, st>>>(sc->bd_ctl.p);
-        rc = capture(st, &gb, [&] {
-            int rc2 = vc_enqueue_photons(sc, pp, st, false);
-            if (rc2 != LMX_OK) return rc2;
-            VB ph;
-            ph.v[0] = sc->bd_vert[0].p; ph.v[1] = sc->vc_vert.p;
-            ph.nsub[0] = sc->bd_nsub[0].p; ph.nsub[1] = sc->vc_nsub.p;
-            ph.epix = sc->bd_epix.p; ph.eraster = sc->bd_eraster.p;
-            ph.V = sc->bd_V.p;
-            ph.mq = nullptr;
-            ShadowQ sq{sc->bd_sray.p, sc->bd_sc.p, sc->bd_saux.p, sc->bd_smeta.p};
-            BCtl* ctl = sc->bd_ctl.p;
-            const size_t nslot = (size_t)B * pcap;
-            const int g = std::max(1, (int)std::min<size_t>((nslot + 255) / 256, (size_t)cap_grid * 2));
-            k_lt_connect<<<g, 256, 0, st>>>(sc->rs, pp, ctl, ph, sq, bounded ? p->max_num_vertices : -1);
-            rc2 = launch_trace(sc->accel, reinterpret_cast<const WRay*>(sq.ray), 0, &ctl->n_shadow, (uint32_t)nslot,
-                               reinterpret_cast<WHit*>(sc->bd_shits.p), st, true, true);   // cleared by the last shade
-            if (rc2 != LMX_OK) return rc2;
-            const int gs = std::max(1, (int)std::min<size_t>((nslot + SPLAT_THREADS - 1) / SPLAT_THREADS, (size_t)sc->cus));
-            k_lt_splat<<<gs, SPLAT_THREADS, 0, st>>>(pp, ctl, sq, sc->bd_shits.p, (int32_t)pcap);
-            const hipError_t e2 = hipGetLastError();
-            return e2 == hipSuccess ? LMX_OK : hip_error(e2, "ltdirect launch");
-        });
     }
+    auto batch = [&](hipStream_t cs) {
+        int rc2 = vc_enqueue_photons(sc, pp, cs, false);
+        if (rc2 != LMX_OK) return rc2;
+        VB ph;
+        ph.v[0] = sc->bd_vert[0].p; ph.v[1] = sc->vc_vert.p;
+        ph.nsub[0] = sc->bd_nsub[0].p; ph.nsub[1] = sc->vc_nsub.p;
+        ph.epix = sc->bd_epix.p; ph.eraster = sc->bd_eraster.p;
+        ph.V = sc->bd_V.p;
+        ph.mq = nullptr;
+        ShadowQ sq{sc->bd_sray.p, sc->bd_sc.p, sc->bd_saux.p, sc->bd_smeta.p};
+        BCtl* ctl = sc->bd_ctl.p;
+        const size_t nslot = (size_t)B * pcap;
+        const int g = std::max(1, (int)std::min<size_t>((nslot + 255) / 256, (size_t)cap_grid * 2));
+        k_lt_connect<<<g, 256, 0, cs>>>(sc->rs, pp, ctl, ph, sq, bounded ? p->max_num_vertices : -1);
+        rc2 = launch_trace(sc->accel, reinterpret_cast<const WRay*>(sq.ray), 0, &ctl->n_shadow, (uint32_t)nslot,
+                           reinterpret_cast<WHit*>(sc->bd_shits.p), cs, true, true);   // cleared by the last shade
+        if (rc2 != LMX_OK) return rc2;
+        const int gs = std::max(1, (int)std::min<size_t>((nslot + SPLAT_THREADS - 1) / SPLAT_THREADS, (size_t)sc->cus));
+        k_lt_splat<<<gs, SPLAT_THREADS, 0, cs>>>(pp, ctl, sq, sc->bd_shits.p, (int32_t)pcap);
+        const hipError_t e2 = hipGetLastError();
+        return e2 == hipSuccess ? LMX_OK : hip_error(e2, "ltdirect launch");
+    };
     const uint64_t nbatch = ((uint64_t)N + B - 1) / B;
     for (uint64_t b = 0; rc == LMX_OK && b < nbatch; b++) {
         k_lt_batch<<<1, 64, 0, st>>>(sc->bd_ctl.p, (uint32_t)(b * B));
-        if ((e = hipGraphLaunch(gb, st)) != hipSuccess) rc = hip_error(e, "graph launch");
+        rc = bd_step(sc, gb, nbatch > 1, st, batch);
     }
     if (rc == LMX_OK) {
         k_bd_scale<<<zgrid, 256, 0, st>>>(film_rgb, 3 * npix, (float)((double)npix / (double)N));
@@ -2953,7 +2955,6 @@ int render_ltdirect(lmx_scene* sc, const lmx_render_params* p, float* film_rgb, 
             (e = hipStreamSynchronize(st)) != hipSuccess)
             rc = hip_error(e, "lmx_render_ltdirect: sync");
     }
-    if (gb) (void)hipGraphExecDestroy(gb);
     if (own) (void)hipStreamDestroy(own);
     if (stats) {
         stats->rays = rc == LMX_OK ? sc->bd_hctl->rays + sc->bd_hctl->shadow_rays : 0;

@@ -145,3 +145,22 @@ def test_bdpt_per_strategy_parity_ggx(gpu):
                                                 sample_out=True, batch=4096)
     c = orc.Scene(sc).bdpt_samples(0, n, max_num_vertices=m, table=tab)
     _check(so.cpu().numpy(), c)
+
+
+@pytest.mark.parametrize("sampler,maxv,n", [("vcm_bdpt", 32, 100003), ("bdpt", -1, 50021), ("vcm_bdpt", 10, 4099)])
+def test_connection_rounds_beyond_the_queue(gpu, sampler, maxv, n):
+    """Batches whose worst case does not fit the connection queue's budget
+    (many rounds: a closed scattering sphere at 32 vertices, where nearly
+    every sample holds 497 connections and the queue 24 per sample; and
+    unbounded subpaths with roulette), and one that fits: the film equals
+    that of the same samples in small batches, up to the order of the
+    additions (k single-precision terms: k 2^-24 of their sum)."""
+    sc = scenes.furnace_sphere(albedo=0.5, Le=1.0, subdiv=2, width=8, height=8)
+    rs = render.Scene(sc)
+    one, st, _ = getattr(rs, "render_" + sampler)(n, max_num_vertices=maxv, seed=3, batch=n)
+    many, sm, _ = getattr(rs, "render_" + sampler)(n, max_num_vertices=maxv, seed=3, batch=8000)
+    assert st["batches"] == 1 and sm["batches"] == (n + 7999) // 8000
+    assert st["rays"] == sm["rays"] and st["rays"] > 3 * n
+    a, b = one.cpu().numpy().astype(np.float64), many.cpu().numpy().astype(np.float64)
+    per_pixel = st["rays"] / 64.0
+    assert a.min() > 0.5 and np.abs(a - b).max() <= per_pixel * 2.0 ** -24 * b.max()
