@@ -1024,6 +1024,12 @@ int launch_trace(lmx_accel* a, const WRay* rays, uint32_t n, const uint32_t* n_d
     return enqueue_trace(a, a->d_counters, rays, n, n_dev, n_max, hits, s, anyhit, cursors_clear);
 }
 
+const WTri* trace_triangles(const lmx_accel* a, uint32_t* n)
+{
+    *n = (uint32_t)a->host.tris.size();
+    return a->host.isect == WBVH_ISECT_WATERTIGHT ? a->d_tris : nullptr;
+}
+
 int trace_counters(lmx_accel* a, uint32_t** counters)
 {
     const int rc = lmx_accel_upload(a);

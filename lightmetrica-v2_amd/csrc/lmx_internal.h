@@ -24,4 +24,8 @@ int launch_trace(lmx_accel* a, const WRay* rays, uint32_t n, const uint32_t* n_d
 // The accel's counter block on the current device (uploads the accel first).
 int trace_counters(lmx_accel* a, uint32_t** counters);
 
+// The device triangles of an uploaded accel built for the watertight test, and
+// how many; NULL of one built for the other test.
+const WTri* trace_triangles(const lmx_accel* a, uint32_t* n);
+
 }  // namespace lmx

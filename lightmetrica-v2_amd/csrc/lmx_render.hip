@@ -33,6 +33,7 @@
 #include "rmath.h"
 #include "rshade.h"
 #include "wbvh.h"
+#include "wbvh_math.h"
 
 using namespace lmx;
 
@@ -168,6 +169,79 @@ __global__ void k_bin_clear(Ctl* ctl)
     if (threadIdx.x < SHADE_CLASSES) ctl->bin[threadIdx.x] = 0;
 }
 
+// What a path does at the surface it hit (renderer_pt.cpp:118-230 and the next-
+// event variants): adds the emission it meets, plays roulette, connects to a
+// light (`no`), samples the BSDF.  t4: throughput rgb and the BSDF density of
+// d at the previous vertex times its cosine there; h: t, b0, b1 of the hit.
+// True when the path goes on, along `next`, as segment seg + 1.
+struct PathNext {
+    f3 p, wo;
+    float4 thr;
+};
+
+RD bool path_shade(const RScene& s, const RParams& p, f3 o, f3 d, float4 t4, float4 h, uint32_t id, uint32_t sample,
+                   uint32_t seg, uint32_t pixel, NeeOut& no, PathNext& next)
+{
+    f3 thr = mk3(t4.x, t4.y, t4.z);
+    Frame fr;
+    surface_at(s, o, d, h.x, h.y, h.z, id, fr);
+    const RMat m = s.mats[s.tri_mat[id]];
+    int nv = (int)seg + 1;                  // numVertices when this segment was traced
+    // hit with a light (renderer_pt.cpp:183-194; renderer_ptmis.cpp:229-257
+    // weighs it against light sampling; renderer::ptdirect ignores it)
+    if (p.nee != NEE_DIRECT && (m.Le[0] > 0.0f || m.Le[1] > 0.0f || m.Le[2] > 0.0f)) {
+        const float cl = to_local(fr, neg(d)).z;
+        if (nv + 1 >= p.min_nv && cl > 0.0f) {
+            float w = 1.0f;
+            if (p.nee == NEE_MIS) {
+                // t4.w: the BSDF density of d at the previous vertex times its cosine there
+                const int l = s.tri_light[id];
+                const float pL = s.lights[l].inv_area * h.x * h.x / cl * (1.0f / (float)s.nlight);
+                w = t4.w / (t4.w + pL);
+            }
+            const f3 C = mk3(thr.x * m.Le[0] * w, thr.y * m.Le[1] * w, thr.z * m.Le[2] * w);
+            float* fp = p.film + 3 * (size_t)pixel;
+            atomicAdd(fp, C.x); atomicAdd(fp + 1, C.y); atomicAdd(fp + 2, C.z);
+            if (p.sample_out) {
+                float* so = p.sample_out + p.so_stride * (size_t)sample;
+                so[2] += C.x; so[3] += C.y; so[4] += C.z; so[5] += 1.0f;
+            }
+        }
+    }
+    const Uniforms<RParams> U{p, sample};
+    bool alive = true;
+    // Russian roulette (renderer_pt.cpp:207-215), from rr_depth on
+    if ((int)seg + 1 >= p.rr_depth) {
+        const float q = rr_continue(p, thr);
+        if (!(q > 0.0f) || U.one(LMX_PT_SLOT_SEG0 + p.seg_stride * seg + 3u) > q) alive = false;
+        else thr = mk3(thr.x / q, thr.y / q, thr.z / q);
+    }
+    nv++;
+    if (alive && p.max_nv != -1 && nv >= p.max_nv) alive = false;
+    if (alive && is_scatterer(m)) {
+        const uint32_t seg2 = seg + 1u;
+        const f3 wi = neg(d);
+        if (p.nee != NEE_NONE && (p.nee == NEE_DIRECT || nv + 1 >= p.min_nv)) {
+            const float4 un = U.block(LMX_PT_SLOT_SEG0 + p.seg_stride * seg2 + 4u);
+            no = nee_connect(s, p, false, fr, m, wi, thr, un.x, un.y, un.z);
+        }
+        const float4 u = U.block(LMX_PT_SLOT_SEG0 + p.seg_stride * seg2);
+        f3 wo;
+        if (bsdf_sample(m, fr, wi, u.x, u.y, wo)) {
+            const float pdf = bsdf_pdf(m, fr, wi, wo);
+            const f3 fs = bsdf_eval(m, fr, wi, wo);
+            if (!(fs.x == 0.0f && fs.y == 0.0f && fs.z == 0.0f)) {
+                thr = mk3(thr.x * (fs.x / pdf), thr.y * (fs.y / pdf), thr.z * (fs.z / pdf));
+                next.p = fr.p;
+                next.wo = wo;
+                next.thr = make_float4(thr.x, thr.y, thr.z, pdf * fabsf(to_local(fr, wo).z));
+                return true;
+            }
+        }
+    }
+    return false;
+}
+
 __global__ __launch_bounds__(256) void k_shade(RScene s, RParams p, Ctl* __restrict__ ctl, int a, Queue in,
                                                const float4* __restrict__ hits, Queue out)
 {
@@ -200,67 +274,16 @@ __global__ __launch_bounds__(256) void k_shade(RScene s, RParams p, Ctl* __restr
             if (!(meta.w & META_DEAD) && id != WBVH_MISS) {
                 const float4 r0 = in.ray[2 * i], r1 = in.ray[2 * i + 1];
                 const float4 t4 = in.thr[i];
-                f3 thr = mk3(t4.x, t4.y, t4.z);
-                const f3 o = mk3(r0.x, r0.y, r0.z), d = mk3(r1.x, r1.y, r1.z);
-                const uint32_t sample = meta.x, seg = meta.y, pixel = meta.z;
-                Frame fr;
-                surface_at(s, o, d, h.x, h.y, h.z, id, fr);
-                const RMat m = s.mats[s.tri_mat[id]];
-                int nv = (int)seg + 1;                  // numVertices when this segment was traced
-                // hit with a light (renderer_pt.cpp:183-194; renderer_ptmis.cpp:229-257
-                // weighs it against light sampling; renderer::ptdirect ignores it)
-                if (p.nee != NEE_DIRECT && (m.Le[0] > 0.0f || m.Le[1] > 0.0f || m.Le[2] > 0.0f)) {
-                    const float cl = to_local(fr, neg(d)).z;
-                    if (nv + 1 >= p.min_nv && cl > 0.0f) {
-                        float w = 1.0f;
-                        if (p.nee == NEE_MIS) {
-                            // t4.w: the BSDF density of d at the previous vertex times its cosine there
-                            const int l = s.tri_light[id];
-                            const float pL = s.lights[l].inv_area * h.x * h.x / cl * (1.0f / (float)s.nlight);
-                            w = t4.w / (t4.w + pL);
-                        }
-                        const f3 C = mk3(thr.x * m.Le[0] * w, thr.y * m.Le[1] * w, thr.z * m.Le[2] * w);
-                        float* fp = p.film + 3 * (size_t)pixel;
-                        atomicAdd(fp, C.x); atomicAdd(fp + 1, C.y); atomicAdd(fp + 2, C.z);
-                        if (p.sample_out) {
-                            float* so = p.sample_out + p.so_stride * (size_t)sample;
-                            so[2] += C.x; so[3] += C.y; so[4] += C.z; so[5] += 1.0f;
-                        }
-                    }
-                }
-                const Uniforms<RParams> U{p, sample};
-                bool alive = true;
-                // Russian roulette (renderer_pt.cpp:207-215), from rr_depth on
-                if ((int)seg + 1 >= p.rr_depth) {
-                    const float q = rr_continue(p, thr);
-                    if (!(q > 0.0f) || U.one(LMX_PT_SLOT_SEG0 + p.seg_stride * seg + 3u) > q) alive = false;
-                    else thr = mk3(thr.x / q, thr.y / q, thr.z / q);
-                }
-                nv++;
-                if (alive && p.max_nv != -1 && nv >= p.max_nv) alive = false;
-                if (alive && is_scatterer(m)) {
-                    const uint32_t seg2 = seg + 1u;
-                    const f3 wi = neg(d);
-                    if (p.nee != NEE_NONE && (p.nee == NEE_DIRECT || nv + 1 >= p.min_nv)) {
-                        const float4 un = U.block(LMX_PT_SLOT_SEG0 + p.seg_stride * seg2 + 4u);
-                        no = nee_connect(s, p, false, fr, m, wi, thr, un.x, un.y, un.z);
-                        no_sample = sample;
-                        no_pixel = pixel;
-                    }
-                    const float4 u = U.block(LMX_PT_SLOT_SEG0 + p.seg_stride * seg2);
-                    f3 wo;
-                    if (bsdf_sample(m, fr, wi, u.x, u.y, wo)) {
-                        const float pdf = bsdf_pdf(m, fr, wi, wo);
-                        const f3 fs = bsdf_eval(m, fr, wi, wo);
-                        if (!(fs.x == 0.0f && fs.y == 0.0f && fs.z == 0.0f)) {
-                            thr = mk3(thr.x * (fs.x / pdf), thr.y * (fs.y / pdf), thr.z * (fs.z / pdf));
-                            o_ray0 = make_float4(fr.p.x, fr.p.y, fr.p.z, LMX_EPS_ISECT);
-                            o_ray1 = make_float4(wo.x, wo.y, wo.z, LMX_FLT_MAX);
-                            o_thr = make_float4(thr.x, thr.y, thr.z, pdf * fabsf(to_local(fr, wo).z));
-                            o_meta = make_uint4(sample, seg2, pixel, 0u);
-                            cont = true;
-                        }
-                    }
+                PathNext next;
+                cont = path_shade(s, p, mk3(r0.x, r0.y, r0.z), mk3(r1.x, r1.y, r1.z), t4, h, id, meta.x, meta.y, meta.z,
+                                  no, next);
+                no_sample = meta.x;
+                no_pixel = meta.z;
+                if (cont) {
+                    o_ray0 = make_float4(next.p.x, next.p.y, next.p.z, LMX_EPS_ISECT);
+                    o_ray1 = make_float4(next.wo.x, next.wo.y, next.wo.z, LMX_FLT_MAX);
+                    o_thr = next.thr;
+                    o_meta = make_uint4(meta.x, meta.y + 1u, meta.z, 0u);
                 }
             }
         }
@@ -273,6 +296,60 @@ __global__ __launch_bounds__(256) void k_shade(RScene s, RParams p, Ctl* __restr
         }
         if (p.nee != NEE_NONE) nee_append(p, &ctl->n_shadow[1 - a], lds, no, no_sample, no_pixel, false);
     }
+}
+
+// The camera ray of a sample (renderer_pt.cpp:64-116): its pixel, its
+// direction, whether it misses the film, the direction's density at the
+// camera (for MIS at a light hit); clears the sample's record and, with
+// next-event estimation, connects the camera vertex (`no`).
+struct PathStart {
+    f3 wo;
+    uint32_t pixel, flags;
+    float pdf;
+};
+
+RD PathStart path_start(const RScene& s, const RParams& p, uint32_t sample, NeeOut& no, uint32_t& no_pixel)
+{
+    PathStart o;
+    const Uniforms<RParams> U{p, sample};
+    const float ux = U.one(LMX_PT_SLOT_RASTER), uy = U.one(LMX_PT_SLOT_RASTER + 1);
+    float rx, ry;
+    o.flags = 0;
+    float out_rx, out_ry;
+    if (p.raster_mode == LMX_RASTER_STRATIFIED) {
+        const uint32_t npix = (uint32_t)s.width * (uint32_t)s.height;
+        o.pixel = sample % npix;
+        const uint32_t px = o.pixel % (uint32_t)s.width, py = o.pixel / (uint32_t)s.width;
+        rx = ((float)px + ux) / (float)s.width;
+        ry = ((float)py + uy) / (float)s.height;
+        o.wo = camera_dir(s, rx, ry);
+        out_rx = ((float)px + 0.5f) / (float)s.width;
+        out_ry = ((float)py + 0.5f) / (float)s.height;
+    } else {
+        o.wo = camera_dir(s, ux, uy);
+        if (!camera_raster(s, o.wo, rx, ry)) { o.flags = META_DEAD; rx = ry = 0.0f; }
+        o.pixel = raster_pixel(s, rx, ry);
+        out_rx = rx; out_ry = ry;
+    }
+    if (o.flags & META_DEAD) { out_rx = 0.0f; out_ry = 0.0f; }
+    o.pdf = p.nee == NEE_MIS ? importance(s, o.wo) : 0.0f;
+    if (p.sample_out) {
+        float4* so = reinterpret_cast<float4*>(p.sample_out + p.so_stride * (size_t)sample);
+        so[0] = make_float4(out_rx, out_ry, 0.0f, 0.0f);
+        so[1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (p.so_stride == 16) { so[2] = so[1]; so[3] = so[1]; }
+    }
+    // next-event estimation at the camera vertex
+    // (none for a sample whose raster position failed, renderer_ptmis.cpp:95-103)
+    no_pixel = o.pixel;
+    if (p.nee != NEE_NONE && !(o.flags & META_DEAD) && (p.nee == NEE_DIRECT || 2 >= p.min_nv)) {
+        const float4 un = U.block(LMX_PT_SLOT_SEG0 + 4u);
+        Frame fr;
+        RMat m;
+        no = nee_connect(s, p, true, fr, m, mk3(0, 0, 0), mk3(1.0f, 1.0f, 1.0f), un.x, un.y, un.z);
+        if (no.emit) no_pixel = raster_pixel(s, no.rx, no.ry);
+    }
+    return o;
 }
 
 // Fills queue b, to which shading queue a's paths appended n_app[b], with
@@ -307,50 +384,30 @@ __global__ __launch_bounds__(256) void k_gen(RScene s, RParams p, Ctl* __restric
         if (t < want) {
             sample = first + t;
             const uint32_t slot = base_slot + t;
-            const Uniforms<RParams> U{p, sample};
-            const float ux = U.one(LMX_PT_SLOT_RASTER), uy = U.one(LMX_PT_SLOT_RASTER + 1);
-            float rx, ry;
-            f3 wo;
-            uint32_t flags = 0;
-            float out_rx, out_ry;
-            if (p.raster_mode == LMX_RASTER_STRATIFIED) {
-                const uint32_t npix = (uint32_t)s.width * (uint32_t)s.height;
-                pixel = sample % npix;
-                const uint32_t px = pixel % (uint32_t)s.width, py = pixel / (uint32_t)s.width;
-                rx = ((float)px + ux) / (float)s.width;
-                ry = ((float)py + uy) / (float)s.height;
-                wo = camera_dir(s, rx, ry);
-                out_rx = ((float)px + 0.5f) / (float)s.width;
-                out_ry = ((float)py + 0.5f) / (float)s.height;
-            } else {
-                wo = camera_dir(s, ux, uy);
-                if (!camera_raster(s, wo, rx, ry)) { flags = META_DEAD; rx = ry = 0.0f; }
-                pixel = raster_pixel(s, rx, ry);
-                out_rx = rx; out_ry = ry;
-            }
-            if (flags & META_DEAD) { out_rx = 0.0f; out_ry = 0.0f; }
-            // thr.w: the direction's density at the camera (importance), for MIS at a light hit
+            const PathStart ps = path_start(s, p, sample, no, pixel);
             out.ray[2 * slot] = make_float4(s.cam_pos.x, s.cam_pos.y, s.cam_pos.z, LMX_EPS_ISECT);
-            out.ray[2 * slot + 1] = make_float4(wo.x, wo.y, wo.z, (flags & META_DEAD) ? -1.0f : LMX_FLT_MAX);
-            out.thr[slot] = make_float4(1.0f, 1.0f, 1.0f, p.nee == NEE_MIS ? importance(s, wo) : 0.0f);
-            out.meta[slot] = make_uint4(sample, 0u, pixel, flags);
-            if (p.sample_out) {
-                float4* so = reinterpret_cast<float4*>(p.sample_out + p.so_stride * (size_t)sample);
-                so[0] = make_float4(out_rx, out_ry, 0.0f, 0.0f);
-                so[1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if (p.so_stride == 16) { so[2] = so[1]; so[3] = so[1]; }
-            }
-            // next-event estimation at the camera vertex
-            // (none for a sample whose raster position failed, renderer_ptmis.cpp:95-103)
-            if (p.nee != NEE_NONE && !(flags & META_DEAD) && (p.nee == NEE_DIRECT || 2 >= p.min_nv)) {
-                const float4 un = U.block(LMX_PT_SLOT_SEG0 + 4u);
-                Frame fr;
-                RMat m;
-                no = nee_connect(s, p, true, fr, m, mk3(0, 0, 0), mk3(1.0f, 1.0f, 1.0f), un.x, un.y, un.z);
-                if (no.emit) pixel = raster_pixel(s, no.rx, no.ry);
-            }
+            out.ray[2 * slot + 1] = make_float4(ps.wo.x, ps.wo.y, ps.wo.z, (ps.flags & META_DEAD) ? -1.0f : LMX_FLT_MAX);
+            out.thr[slot] = make_float4(1.0f, 1.0f, 1.0f, ps.pdf);
+            out.meta[slot] = make_uint4(sample, 0u, ps.pixel, ps.flags);
         }
         if (p.nee != NEE_NONE) nee_append(p, &ctl->n_shadow[b], lds, no, sample, pixel, true);
+    }
+}
+
+// An unoccluded next-event connection of `sample`, from the camera vertex
+// (seen at raster rx, ry) or a later one.
+RD void nee_splat(const RParams& p, f3 c, uint32_t sample, uint32_t pixel, bool camera, float rx, float ry)
+{
+    float* fp = p.film + 3 * (size_t)pixel;
+    atomicAdd(fp, c.x); atomicAdd(fp + 1, c.y); atomicAdd(fp + 2, c.z);
+    if (p.sample_out) {
+        float* so = p.sample_out + p.so_stride * (size_t)sample;
+        if (camera) {
+            so[8] = rx; so[9] = ry;
+            so[10] += c.x; so[11] += c.y; so[12] += c.z; so[13] += 1.0f;
+        } else {
+            so[2] += c.x; so[3] += c.y; so[4] += c.z; so[5] += 1.0f;
+        }
     }
 }
 
@@ -365,17 +422,153 @@ __global__ __launch_bounds__(256) void k_nee_splat(RParams p, const Ctl* __restr
         if (__float_as_uint(p.nq.hits[j].w) != WBVH_MISS) continue;          // occluded
         const float4 c = p.nq.c[j];
         const uint4 m = p.nq.meta[j];
-        float* fp = p.film + 3 * (size_t)m.y;
-        atomicAdd(fp, c.x); atomicAdd(fp + 1, c.y); atomicAdd(fp + 2, c.z);
-        if (p.sample_out) {
-            float* so = p.sample_out + p.so_stride * (size_t)m.x;
-            if (m.z) {
-                so[8] = __uint_as_float(m.w); so[9] = p.nq.ry[j];
-                so[10] += c.x; so[11] += c.y; so[12] += c.z; so[13] += 1.0f;
-            } else {
-                so[2] += c.x; so[3] += c.y; so[4] += c.z; so[5] += 1.0f;
+        nee_splat(p, mk3(c.x, c.y, c.z), m.x, m.y, m.z != 0u, __uint_as_float(m.w), p.nq.ry[j]);
+    }
+}
+
+// Scenes of a few triangles (the Cornell box): a path runs from its camera ray
+// to its end in one lane, and its rays are tested against every triangle in
+// turn, which costs less than the divergent steps of a traversal and than the
+// queues and launches between them.  The arithmetic and the uniforms are those
+// of the wavefront pipeline: the same contributions bit for bit, added to the
+// film in another order.
+//
+// Bound by vector instructions, half of them triangle tests.  So the triangles
+// lie in LDS in each of the six orders of axes that the watertight test can
+// want: a lane reads its order, three 16-byte reads with at most six addresses
+// in a wave, instead of choosing each coordinate (18 of 62 instructions of a
+// test; a 1 M path Cornell box with up to 9 vertices, 34 triangles: 545 -> 460
+// us).  A workgroup owns a contiguous share of the samples and its lanes take
+// the next one when a path ends (a fixed stride of samples per lane: 460, this:
+// 379), at 5 waves a SIMD (4: 379, 5: 362, 6 with spills: 364).  With
+// next-event estimation the connection from the camera is a second pass over
+// the triangles for the starting lanes alone, so a wave starts new samples when
+// 40 lanes are idle (1: 1866 us, 32: 1561, 40: 1547; 4 waves a SIMD, the
+// registers' limit).  The wavefront pipeline takes 690 and 2370.
+//
+// SMALL_TRIS: Cornell boxes of split triangles, 16.8 M paths, us here and in
+// the wavefront pipeline: 34: 3700 / 9150, 48: 6350 / 6860 to 7750,
+// 64: 8420 / 8100, 80: 10440 / 8410; 1 M paths with next-event estimation:
+// 34: 1545 / 2365, 48: 1680 / 2440, 64: 1790 / 2500.
+#define SMALL_TRIS 48u
+#define SMALL_BLOCK 256
+#define SMALL_WAVES 5           // waves per SIMD, also workgroups per CU
+#define SMALL_WAVES_NEE 4
+#define SMALL_IDLE_NEE 40       // idle lanes for which a wave starts new samples
+
+// Which of the six orders of axes: kz's successor as kx, or swapped.
+RD uint32_t small_order(int kx, int ky) { return (uint32_t)(2 * kx + ((kx + 1) % 3 == ky ? 0 : 1)); }
+
+template <bool ANYHIT>
+RD uint32_t small_hit(const float4* tris, uint32_t ntri, f3 o, f3 d, float tmin, float tmax, float4& h)
+{
+    WRayPre r;
+    wb_ray_setup(r, o.x, o.y, o.z, tmin, d.x, d.y, d.z, tmax);
+    const float ok[3] = {wb_sel3(r.kx, o.x, o.y, o.z), wb_sel3(r.ky, o.x, o.y, o.z), wb_sel3(r.kz, o.x, o.y, o.z)};
+    const float4* tri = tris + 3u * ntri * small_order(r.kx, r.ky);
+    float best = tmax, V = 0.0f, W = 0.0f, det = 1.0f;
+    uint32_t id = WBVH_MISS;
+    for (uint32_t k = 0; k < ntri; k++, tri += 3) {
+        const float4 A = tri[0], B = tri[1], C = tri[2];
+        float t, v, w, dt;
+        if (wb_tri_watertight_k(A.x - ok[0], A.y - ok[1], A.z - ok[2], B.x - ok[0], B.y - ok[1], B.z - ok[2], C.x - ok[0],
+                                C.y - ok[1], C.z - ok[2], r, best, t, v, w, dt)) {
+            const uint32_t ti = __float_as_uint(A.w);
+            if (t < best || ti < id) { best = t; id = ti; V = v; W = w; det = dt; }
+        }
+        if (ANYHIT && __ballot(id == WBVH_MISS) == 0) break;
+    }
+    if (!ANYHIT && id != WBVH_MISS) h = make_float4(best, V / det, W / det, 0.0f);
+    return id;
+}
+
+// counts[block] (pinned): rays traced (extension and shadow) by the workgroup.
+template <bool NEE>
+__global__ __launch_bounds__(SMALL_BLOCK, NEE ? SMALL_WAVES_NEE : SMALL_WAVES) void k_small_paths(
+    RScene s, RParams p, const WTri* __restrict__ tris, uint32_t ntri, uint64_t* __restrict__ counts)
+{
+    extern __shared__ float4 ordered[];          // 6 orders x ntri x the three vertices; .w of the first: the id
+    __shared__ unsigned long long sum[SMALL_BLOCK / 64];
+    __shared__ uint32_t taken;
+    for (uint32_t k = threadIdx.x; k < 18u * ntri; k += SMALL_BLOCK) {
+        const uint32_t ord = k / (3u * ntri), j = k % (3u * ntri);
+        const int kx = (int)(ord >> 1), ky = (kx + 1 + (int)(ord & 1u)) % 3, kz = 3 - kx - ky;
+        const float* v = tris[j / 3u].f + 4u * (j % 3u);
+        ordered[k] = make_float4(wb_sel3(kx, v[0], v[1], v[2]), wb_sel3(ky, v[0], v[1], v[2]), wb_sel3(kz, v[0], v[1], v[2]),
+                                 v[3]);
+    }
+    if (threadIdx.x == 0) taken = 0;
+    __syncthreads();
+    const uint32_t first = (uint32_t)((uint64_t)p.total * blockIdx.x / gridDim.x);          // the workgroup's samples
+    const uint32_t count = (uint32_t)((uint64_t)p.total * (blockIdx.x + 1u) / gridDim.x) - first;
+    bool live = false, start = false, more = true;
+    uint32_t rays = 0, sample = 0, seg = 0, pixel = 0;
+    f3 o = mk3(0, 0, 0), d = mk3(0, 0, 0);
+    float4 thr = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float tmax = 0.0f;
+    auto connect = [&](const NeeOut& no, uint32_t pix, bool camera) {
+        float4 h;
+        rays++;
+        if (small_hit<true>(ordered, ntri, mk3(no.r0.x, no.r0.y, no.r0.z), mk3(no.r1.x, no.r1.y, no.r1.z), no.r0.w, no.r1.w,
+                            h) == WBVH_MISS)
+            nee_splat(p, no.C, sample, pix, camera, no.rx, no.ry);
+    };
+    while (true) {
+        const unsigned long long running = __ballot(live);
+        if (more && 64 - __popcll(running) >= (running ? (NEE ? SMALL_IDLE_NEE : 1) : 1)) {
+            if (!live) {
+                const uint32_t k = atomicAdd(&taken, 1u);
+                start = k < count;
+                sample = first + k;
+            }
+            more = __ballot(!live && !start) == 0;       // the share is used up
+        }
+        if (start) {
+            start = false;
+            NeeOut no;
+            no.emit = false;
+            uint32_t no_pixel;
+            const PathStart ps = path_start(s, p, sample, no, no_pixel);
+            pixel = ps.pixel;
+            seg = 0;
+            o = s.cam_pos;
+            d = ps.wo;
+            tmax = (ps.flags & META_DEAD) ? -1.0f : LMX_FLT_MAX;
+            thr = make_float4(1.0f, 1.0f, 1.0f, ps.pdf);
+            live = true;
+            if (NEE && no.emit) connect(no, no_pixel, true);
+        }
+        if (__ballot(live) == 0) break;
+        if (live) {
+            float4 h;
+            rays++;
+            const uint32_t id = small_hit<false>(ordered, ntri, o, d, LMX_EPS_ISECT, tmax, h);
+            live = false;
+            if (id != WBVH_MISS) {
+                NeeOut no;
+                no.emit = false;
+                PathNext next;
+                live = path_shade(s, p, o, d, thr, h, id, sample, seg, pixel, no, next);
+                if (NEE && no.emit) connect(no, pixel, false);
+                if (live) {
+                    seg++;
+                    o = next.p;
+                    d = next.wo;
+                    tmax = LMX_FLT_MAX;
+                    thr = next.thr;
+                }
             }
         }
+    }
+    unsigned long long wave = rays;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) wave += __shfl_xor(wave, off);
+    if ((threadIdx.x & 63u) == 0) sum[threadIdx.x >> 6] = wave;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint64_t t = 0;
+        for (int w = 0; w < SMALL_BLOCK / 64; w++) t += sum[w];
+        counts[blockIdx.x] = t;
     }
 }
 
@@ -671,6 +864,35 @@ int autotune_capacity(lmx_scene* sc, const RParams& rp, hipStream_t st)
 
 }  // namespace
 
+// One frame by k_small_paths, with about `cap` paths in flight at most.
+static int render_small(lmx_scene* sc, const RParams& rp, const WTri* tris, uint32_t ntri, uint32_t cap, hipStream_t st,
+                        size_t npix, uint64_t* rays, uint32_t* flight)
+{
+    const uint32_t most = (uint32_t)sc->cus * (rp.nee == NEE_NONE ? SMALL_WAVES : SMALL_WAVES_NEE);
+    const uint32_t want = (uint32_t)(((uint64_t)std::min(rp.total, cap) + SMALL_BLOCK - 1) / SMALL_BLOCK);
+    // a workgroup's share stays within 2^31, so that its counter cannot wrap
+    const uint32_t grid = std::max(rp.total >> 31 ? 2u : 1u, std::min(most, want));
+    const size_t lds = 18 * (size_t)ntri * sizeof(float4);
+    hipError_t e;
+    if (!sc->h_counts) {
+        const size_t bytes = (size_t)sc->cus * std::max(SMALL_WAVES, SMALL_WAVES_NEE) * sizeof(uint64_t);
+        if ((e = hipHostMalloc((void**)&sc->h_counts, bytes, hipHostMallocDefault)) != hipSuccess) {
+            sc->h_counts = nullptr;
+            return hip_error(e, "pinned ray counts");
+        }
+    }
+    if (rp.nee == NEE_NONE) k_small_paths<false><<<grid, SMALL_BLOCK, lds, st>>>(sc->rs, rp, tris, ntri, sc->h_counts);
+    else k_small_paths<true><<<grid, SMALL_BLOCK, lds, st>>>(sc->rs, rp, tris, ntri, sc->h_counts);
+    k_scale<<<std::max(1, std::min((int)((3 * npix + 255) / 256), sc->cus * 8)), 256, 0, st>>>(
+        rp.film, 3 * npix, (float)((double)npix / (double)rp.total));
+    if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(st)) != hipSuccess)
+        return hip_error(e, "small-scene render");
+    *rays = 0;
+    for (uint32_t k = 0; k < grid; k++) *rays += sc->h_counts[k];
+    *flight = grid * SMALL_BLOCK;
+    return LMX_OK;
+}
+
 static int render_unidir(lmx_scene* sc, const lmx_render_params* p, int nee, const char* name, float* film_rgb, void* stream,
                          lmx_render_stats* stats)
 {
@@ -724,18 +946,30 @@ static int render_unidir(lmx_scene* sc, const lmx_render_params* p, int nee, con
     rp.ray_out_cap = rp.ray_out ? p->ray_out_cap : 0u;
     const int zgrid = std::max(1, std::min((int)((3 * npix + 255) / 256), sc->cus * 8));
     int rc = LMX_OK;
-    if (p->queue_capacity == 0 && sc->tuned_cap == 0) rc = autotune_capacity(sc, rp, st);
-    uint32_t cap = p->queue_capacity ? p->queue_capacity : sc->tuned_cap;
-    if (!timed) cap = (uint32_t)std::min<uint64_t>(cap, std::max<uint64_t>(p->num_samples, 64));
+    uint32_t cap = 0, iters = 0;
     uint64_t rays = 0, taken = 0;
-    uint32_t iters = 0;
-    if (rc == LMX_OK) {
+    // few triangles (SMALL_TRIS), and nothing asked for that belongs to the queues
+    uint32_t ntri = 0;
+    const WTri* tris = trace_triangles(sc->accel, &ntri);
+    const bool small = tris && ntri <= SMALL_TRIS && !timed && !rp.ray_out && p->shade_order == LMX_SHADE_QUEUE;
+    if (small) {
+        k_zero<<<zgrid, 256, 0, st>>>(film_rgb, 3 * npix);
+        rc = render_small(sc, rp, tris, ntri, p->queue_capacity ? p->queue_capacity : 0xffffffffu, st, npix, &rays, &cap);
+        if (p->queue_capacity) cap = (uint32_t)std::min<uint64_t>(p->queue_capacity, std::max<uint64_t>(p->num_samples, 64));
+        taken = p->num_samples;
+        iters = 1;
+    } else {
+        if (p->queue_capacity == 0 && sc->tuned_cap == 0) rc = autotune_capacity(sc, rp, st);
+        cap = p->queue_capacity ? p->queue_capacity : sc->tuned_cap;
+        if (!timed) cap = (uint32_t)std::min<uint64_t>(cap, std::max<uint64_t>(p->num_samples, 64));
+    }
+    if (!small && rc == LMX_OK) {
         k_zero<<<zgrid, 256, 0, st>>>(film_rgb, 3 * npix);
         // a fixed sample count is rescaled on the device as the render ends
         rc = wavefront_render(sc, rp, cap, st, &rays, &iters, timed ? p->render_time : 0.0, &taken,
                               timed ? 0 : 3 * npix, (float)((double)npix / (double)p->num_samples));
     }
-    if (rc == LMX_OK) {
+    if (!small && rc == LMX_OK) {
         // Film::Rescale by W H / the samples taken (scheduler.cpp:281-288)
         if (!sc->h_ctl->film_scaled)
             k_scale<<<zgrid, 256, 0, st>>>(film_rgb, 3 * npix, (float)((double)npix / (double)std::max<uint64_t>(taken, 1)));

@@ -555,6 +555,7 @@ struct lmx_scene {
     DevBuf<uint32_t> perm;              // material-binned shading, SHADE_CLASSES x cap
     DevBuf<Ctl> ctl;
     Ctl* h_ctl = nullptr;      // pinned
+    uint64_t* h_counts = nullptr;       // pinned: rays per workgroup of a small-scene render
     hipGraphExec_t wf_exec = nullptr;   // the wavefront iterations' graph, updated in place per render
     hipStream_t cap_stream = nullptr;   // records that graph and runs nothing
     uint32_t tuned_cap = 0;
@@ -592,6 +593,7 @@ struct lmx_scene {
         if (wf_exec) (void)hipGraphExecDestroy(wf_exec);
         if (cap_stream) (void)hipStreamDestroy(cap_stream);
         if (h_ctl) (void)hipHostFree(h_ctl);
+        if (h_counts) (void)hipHostFree(h_counts);
         if (bd_hctl) (void)hipHostFree(bd_hctl);
         lmx_accel_free(accel);
     }

@@ -212,21 +212,17 @@ WB_HD float wb_dop(float a, float b, float c, float d)
     return f + e;
 }
 
-// Watertight test.  On a hit with t in [tmin, tmax] writes t and the
-// unnormalised (V, W, det); b0 = V/det (2nd vertex), b1 = W/det (3rd vertex).
-WB_HD bool wb_tri_watertight(const WTri& tri, const WRayPre& r, float tmax,
-                             float& t, float& V, float& W, float& det)
+// The test proper, of vertices relative to the ray's origin with their axes in
+// the ray's order.
+WB_HD bool wb_tri_watertight_k(float Akx, float Aky, float Akz, float Bkx, float Bky, float Bkz, float Ckx, float Cky,
+                               float Ckz, const WRayPre& r, float tmax, float& t, float& V, float& W, float& det)
 {
-    const float Ax0 = tri.f[0] - r.ox, Ay0 = tri.f[1] - r.oy, Az0 = tri.f[2] - r.oz;
-    const float Bx0 = tri.f[4] - r.ox, By0 = tri.f[5] - r.oy, Bz0 = tri.f[6] - r.oz;
-    const float Cx0 = tri.f[8] - r.ox, Cy0 = tri.f[9] - r.oy, Cz0 = tri.f[10] - r.oz;
-    const float Akz = wb_sel3(r.kz, Ax0, Ay0, Az0), Bkz = wb_sel3(r.kz, Bx0, By0, Bz0), Ckz = wb_sel3(r.kz, Cx0, Cy0, Cz0);
-    const float Ax = fmaf(-r.Sx, Akz, wb_sel3(r.kx, Ax0, Ay0, Az0));
-    const float Ay = fmaf(-r.Sy, Akz, wb_sel3(r.ky, Ax0, Ay0, Az0));
-    const float Bx = fmaf(-r.Sx, Bkz, wb_sel3(r.kx, Bx0, By0, Bz0));
-    const float By = fmaf(-r.Sy, Bkz, wb_sel3(r.ky, Bx0, By0, Bz0));
-    const float Cx = fmaf(-r.Sx, Ckz, wb_sel3(r.kx, Cx0, Cy0, Cz0));
-    const float Cy = fmaf(-r.Sy, Ckz, wb_sel3(r.ky, Cx0, Cy0, Cz0));
+    const float Ax = fmaf(-r.Sx, Akz, Akx);
+    const float Ay = fmaf(-r.Sy, Akz, Aky);
+    const float Bx = fmaf(-r.Sx, Bkz, Bkx);
+    const float By = fmaf(-r.Sy, Bkz, Bky);
+    const float Cx = fmaf(-r.Sx, Ckz, Ckx);
+    const float Cy = fmaf(-r.Sy, Ckz, Cky);
     const float U = wb_dop(Cx, By, Cy, Bx);
     const float Vv = wb_dop(Ax, Cy, Ay, Cx);
     const float Ww = wb_dop(Bx, Ay, By, Ax);
@@ -239,6 +235,21 @@ WB_HD bool wb_tri_watertight(const WTri& tri, const WRayPre& r, float tmax,
     if (!(tt >= r.tmin && tt <= tmax)) return false;
     t = tt; V = Vv; W = Ww; det = dt;
     return true;
+}
+
+// Watertight test.  On a hit with t in [tmin, tmax] writes t and the
+// unnormalised (V, W, det); b0 = V/det (2nd vertex), b1 = W/det (3rd vertex).
+WB_HD bool wb_tri_watertight(const WTri& tri, const WRayPre& r, float tmax,
+                             float& t, float& V, float& W, float& det)
+{
+    const float Ax0 = tri.f[0] - r.ox, Ay0 = tri.f[1] - r.oy, Az0 = tri.f[2] - r.oz;
+    const float Bx0 = tri.f[4] - r.ox, By0 = tri.f[5] - r.oy, Bz0 = tri.f[6] - r.oz;
+    const float Cx0 = tri.f[8] - r.ox, Cy0 = tri.f[9] - r.oy, Cz0 = tri.f[10] - r.oz;
+    return wb_tri_watertight_k(
+        wb_sel3(r.kx, Ax0, Ay0, Az0), wb_sel3(r.ky, Ax0, Ay0, Az0), wb_sel3(r.kz, Ax0, Ay0, Az0),
+        wb_sel3(r.kx, Bx0, By0, Bz0), wb_sel3(r.ky, Bx0, By0, Bz0), wb_sel3(r.kz, Bx0, By0, Bz0),
+        wb_sel3(r.kx, Cx0, Cy0, Cz0), wb_sel3(r.ky, Cx0, Cy0, Cz0), wb_sel3(r.kz, Cx0, Cy0, Cz0),
+        r, tmax, t, V, W, det);
 }
 
 // TriAccel test with the reference's operation order

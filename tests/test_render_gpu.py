@@ -223,3 +223,40 @@ def test_ray_and_sample_counts(gpu, n, cap):
         assert 4 * n * (1 - 1e-4) - 4 <= st["rays"] <= 4 * n
         got = float(film.double().mean())
         assert abs(got - (1 + 0.5 + 0.25 + 0.125)) <= 1e-4 + 4.0 / n * (st["rays"] < 4 * n)
+
+
+def _split_cornell(ntri, **kw):
+    """The Cornell box with its walls and boxes split at edge midpoints into ntri triangles."""
+    sc = scenes.cornell_box(33, 21, **kw)
+    tris, mat, verts = sc["tris"][:-2].tolist(), sc["tri_mat"][:-2].tolist(), sc["verts"].tolist()
+    while len(tris) + 2 < ntri:
+        (a, b, c), m = tris.pop(0), mat.pop(0)
+        verts.append([(x + y) / 2 for x, y in zip(verts[b], verts[c])])
+        k = len(verts) - 1
+        tris += [[k, a, b], [k, c, a]]
+        mat += [m, m]
+    return dict(sc, verts=np.array(verts, np.float32), lights=[(len(tris), 2)],
+                tris=np.array(tris + sc["tris"][-2:].tolist(), np.uint32),
+                tri_mat=np.array(mat + sc["tri_mat"][-2:].tolist(), np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ntri,n,cap,kw", [
+    (34, 1, 0, {}), (34, 63, 0, {}), (34, 255, 64, dict(phong_boxes=20.0)), (34, 257, 0, dict(ggx_boxes=0.2)),
+    (47, 100003, 0, {}), (48, 20001, 1000, dict(ggx_boxes=0.5)), (48, 700001, 0, {}), (49, 5000, 0, {})])
+@pytest.mark.parametrize("entry", ["pt", "ptmis", "ptdirect"])
+def test_few_triangles(gpu, entry, ntri, n, cap, kw):
+    """Scenes small enough for one kernel per frame (48 triangles, and one
+    more) against the queues, which a render binned by material always takes:
+    the same rays and the same record of every sample, bit for bit."""
+    rs = render.Scene(_split_cornell(ntri, **kw))
+    for opts in (dict(max_num_vertices=-1, rr_depth=2), dict(max_num_vertices=2), dict(max_num_vertices=6, min_num_vertices=3),
+                 dict(max_num_vertices=9, rr_depth=1, rr_mode=render.RR_THROUGHPUT, raster_mode=render.RASTER_STRATIFIED)):
+        got = [getattr(rs, "render_" + entry)(n, seed=n + 1, sample_out=True, queue_capacity=cap, shade_order=order, **opts)
+               for order in (render.SHADE_QUEUE, render.SHADE_BY_MATERIAL)]
+        (fa, sa, ra), (fb, sb, rb) = got
+        assert sa["rays"] == sb["rays"] and sa["samples"] == sb["samples"] == n
+        assert np.array_equal(np.asarray(ra.cpu()).view(np.uint32), np.asarray(rb.cpu()).view(np.uint32))
+        # the additions of a pixel in another order: FP32 sums of at most c terms of one sign
+        c = 8.0 * (n / (33 * 21) + 30.0)
+        assert float((fa - fb).abs().max()) <= c * 2.0 ** -24 * 2 * float(fb.abs().max())
