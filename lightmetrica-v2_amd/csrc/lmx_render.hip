@@ -1,4 +1,5 @@
-// lmx_render.hip -- renderer::pt as a wavefront pipeline on gfx950.
+// lmx_render.hip -- renderer::pt as a wavefront pipeline on gfx950 (scenes of a
+// few triangles: one kernel, k_small_paths).
 //
 // Replaces the per-sample CPU loop of the reference
 // (src/liblightmetrica/renderer/renderer_pt.cpp:64-231 driven by
@@ -451,6 +452,8 @@ __global__ __launch_bounds__(256) void k_nee_splat(RParams p, const Ctl* __restr
 // 64: 8420 / 8100, 80: 10440 / 8410; 1 M paths with next-event estimation:
 // 34: 1545 / 2365, 48: 1680 / 2440, 64: 1790 / 2500.
 #define SMALL_TRIS 48u
+#define SMALL_LENGTH 1024       // vertices: a launch stays short of seconds
+#define SMALL_SAMPLES (1u << 26)
 #define SMALL_BLOCK 256
 #define SMALL_WAVES 5           // waves per SIMD, also workgroups per CU
 #define SMALL_WAVES_NEE 4
@@ -482,10 +485,12 @@ RD uint32_t small_hit(const float4* tris, uint32_t ntri, f3 o, f3 d, float tmin,
     return id;
 }
 
-// counts[block] (pinned): rays traced (extension and shadow) by the workgroup.
+// Samples begin .. begin + n - 1, n <= SMALL_SAMPLES.  counts[block] (pinned)
+// grows by the rays traced (extension and shadow) by the workgroup.
 template <bool NEE>
 __global__ __launch_bounds__(SMALL_BLOCK, NEE ? SMALL_WAVES_NEE : SMALL_WAVES) void k_small_paths(
-    RScene s, RParams p, const WTri* __restrict__ tris, uint32_t ntri, uint64_t* __restrict__ counts)
+    RScene s, RParams p, uint32_t begin, uint32_t n, const WTri* __restrict__ tris, uint32_t ntri,
+    uint64_t* __restrict__ counts)
 {
     extern __shared__ float4 ordered[];          // 6 orders x ntri x the three vertices; .w of the first: the id
     __shared__ unsigned long long sum[SMALL_BLOCK / 64];
@@ -499,8 +504,8 @@ __global__ __launch_bounds__(SMALL_BLOCK, NEE ? SMALL_WAVES_NEE : SMALL_WAVES) v
     }
     if (threadIdx.x == 0) taken = 0;
     __syncthreads();
-    const uint32_t first = (uint32_t)((uint64_t)p.total * blockIdx.x / gridDim.x);          // the workgroup's samples
-    const uint32_t count = (uint32_t)((uint64_t)p.total * (blockIdx.x + 1u) / gridDim.x) - first;
+    const uint32_t share = (uint32_t)((uint64_t)n * blockIdx.x / gridDim.x);                // the workgroup's samples
+    const uint32_t count = (uint32_t)((uint64_t)n * (blockIdx.x + 1u) / gridDim.x) - share, first = begin + share;
     bool live = false, start = false, more = true;
     uint32_t rays = 0, sample = 0, seg = 0, pixel = 0;
     f3 o = mk3(0, 0, 0), d = mk3(0, 0, 0);
@@ -568,7 +573,7 @@ __global__ __launch_bounds__(SMALL_BLOCK, NEE ? SMALL_WAVES_NEE : SMALL_WAVES) v
     if (threadIdx.x == 0) {
         uint64_t t = 0;
         for (int w = 0; w < SMALL_BLOCK / 64; w++) t += sum[w];
-        counts[blockIdx.x] = t;
+        counts[blockIdx.x] += t;
     }
 }
 
@@ -870,8 +875,7 @@ static int render_small(lmx_scene* sc, const RParams& rp, const WTri* tris, uint
 {
     const uint32_t most = (uint32_t)sc->cus * (rp.nee == NEE_NONE ? SMALL_WAVES : SMALL_WAVES_NEE);
     const uint32_t want = (uint32_t)(((uint64_t)std::min(rp.total, cap) + SMALL_BLOCK - 1) / SMALL_BLOCK);
-    // a workgroup's share stays within 2^31, so that its counter cannot wrap
-    const uint32_t grid = std::max(rp.total >> 31 ? 2u : 1u, std::min(most, want));
+    const uint32_t grid = std::max(1u, std::min(most, want));
     const size_t lds = 18 * (size_t)ntri * sizeof(float4);
     hipError_t e;
     if (!sc->h_counts) {
@@ -881,8 +885,14 @@ static int render_small(lmx_scene* sc, const RParams& rp, const WTri* tris, uint
             return hip_error(e, "pinned ray counts");
         }
     }
-    if (rp.nee == NEE_NONE) k_small_paths<false><<<grid, SMALL_BLOCK, lds, st>>>(sc->rs, rp, tris, ntri, sc->h_counts);
-    else k_small_paths<true><<<grid, SMALL_BLOCK, lds, st>>>(sc->rs, rp, tris, ntri, sc->h_counts);
+    std::fill(sc->h_counts, sc->h_counts + grid, (uint64_t)0);
+    for (uint64_t b = 0; b < rp.total; b += SMALL_SAMPLES) {
+        const uint32_t n = (uint32_t)std::min<uint64_t>(SMALL_SAMPLES, rp.total - b);
+        if (rp.nee == NEE_NONE)
+            k_small_paths<false><<<grid, SMALL_BLOCK, lds, st>>>(sc->rs, rp, (uint32_t)b, n, tris, ntri, sc->h_counts);
+        else
+            k_small_paths<true><<<grid, SMALL_BLOCK, lds, st>>>(sc->rs, rp, (uint32_t)b, n, tris, ntri, sc->h_counts);
+    }
     k_scale<<<std::max(1, std::min((int)((3 * npix + 255) / 256), sc->cus * 8)), 256, 0, st>>>(
         rp.film, 3 * npix, (float)((double)npix / (double)rp.total));
     if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(st)) != hipSuccess)
@@ -948,10 +958,14 @@ static int render_unidir(lmx_scene* sc, const lmx_render_params* p, int nee, con
     int rc = LMX_OK;
     uint32_t cap = 0, iters = 0;
     uint64_t rays = 0, taken = 0;
-    // few triangles (SMALL_TRIS), and nothing asked for that belongs to the queues
+    // few triangles (SMALL_TRIS), nothing asked for that belongs to the queues,
+    // and paths that end by themselves: the one kernel runs until the longest
+    // has, while the queues return to the host every few segments
+    const bool ends = p->max_num_vertices != -1 ? p->max_num_vertices <= SMALL_LENGTH
+                                                : p->rr_mode == LMX_RR_FIXED && p->rr_prob <= 0.9f && p->rr_depth <= SMALL_LENGTH;
     uint32_t ntri = 0;
     const WTri* tris = trace_triangles(sc->accel, &ntri);
-    const bool small = tris && ntri <= SMALL_TRIS && !timed && !rp.ray_out && p->shade_order == LMX_SHADE_QUEUE;
+    const bool small = ends && tris && ntri <= SMALL_TRIS && !timed && !rp.ray_out && p->shade_order == LMX_SHADE_QUEUE;
     if (small) {
         k_zero<<<zgrid, 256, 0, st>>>(film_rgb, 3 * npix);
         rc = render_small(sc, rp, tris, ntri, p->queue_capacity ? p->queue_capacity : 0xffffffffu, st, npix, &rays, &cap);

@@ -250,7 +250,7 @@ def test_few_triangles(gpu, entry, ntri, n, cap, kw):
     more) against the queues, which a render binned by material always takes:
     the same rays and the same record of every sample, bit for bit."""
     rs = render.Scene(_split_cornell(ntri, **kw))
-    for opts in (dict(max_num_vertices=-1, rr_depth=2), dict(max_num_vertices=2), dict(max_num_vertices=6, min_num_vertices=3),
+    for opts in (dict(max_num_vertices=-1, rr_depth=2), dict(max_num_vertices=-1, rr_prob=0.95), dict(max_num_vertices=2), dict(max_num_vertices=6, min_num_vertices=3),
                  dict(max_num_vertices=9, rr_depth=1, rr_mode=render.RR_THROUGHPUT, raster_mode=render.RASTER_STRATIFIED)):
         got = [getattr(rs, "render_" + entry)(n, seed=n + 1, sample_out=True, queue_capacity=cap, shade_order=order, **opts)
                for order in (render.SHADE_QUEUE, render.SHADE_BY_MATERIAL)]
@@ -260,3 +260,15 @@ def test_few_triangles(gpu, entry, ntri, n, cap, kw):
         # the additions of a pixel in another order: FP32 sums of at most c terms of one sign
         c = 8.0 * (n / (33 * 21) + 30.0)
         assert float((fa - fb).abs().max()) <= c * 2.0 ** -24 * 2 * float(fb.abs().max())
+
+
+@pytest.mark.gpu
+def test_few_triangles_beyond_one_launch(gpu):
+    """More samples than one launch takes (2^26): every one is counted and splat once."""
+    rs = render.Scene(_split_cornell(34))
+    n = (1 << 26) + 7
+    (fa, sa, _), (fb, sb, _) = [rs.render_pt(n, seed=3, max_num_vertices=2, shade_order=order)
+                                for order in (render.SHADE_QUEUE, render.SHADE_BY_MATERIAL)]
+    assert sa["rays"] == sb["rays"] == n and sa["samples"] == sb["samples"] == n
+    # FP32 sums of n / (33 21) terms of one sign in another order, both rounded
+    assert float((fa - fb).abs().max()) <= 2 * 1.1 * n / (33 * 21) * 2.0 ** -24 * float(fb.abs().max())
