@@ -2335,6 +2335,24 @@ int vc_buffers(lmx_scene* sc, uint32_t np, uint32_t maxv, uint32_t B)
     return LMX_OK;
 }
 
+// Buckets of the hash grid for about n photon vertices: the next power of two,
+// within the buffers (vc_buffers), which hold one for every vertex there can
+// be.  With roulette 0.5 at every vertex a photon leaves about one or two,
+// and clearing and scanning the rest bounded the grid kernels: renderer::sppm,
+// 262,144 photons of at most 10 vertices a pass, 8 passes 5,591 us with 2^22
+// buckets, 5,413 with 4 a photon, 5,407 with 2, 5,412 with 1; 4 passes of
+// 2,097,152 photons 9,684, 9,117, 9,040, 9,026; the same photons in the closed
+// Cornell box (longer lists) 48.3 ms, 45.4, 44.8, 46.4.  Below 2^16 buckets
+// nothing is left to save (8,192 photons: 2,316 with 2^17, 2,343 with 2^14).
+#define ROULETTE_BUCKETS 2u
+#define MIN_BUCKETS (1u << 16)
+void vc_buckets(lmx_scene* sc, uint64_t n)
+{
+    n = std::max<uint64_t>(n, MIN_BUCKETS);
+    sc->vc_H = 1024;
+    while (sc->vc_H < n && 2 * (uint64_t)sc->vc_H < sc->vc_start.n) sc->vc_H <<= 1;
+}
+
 // Records one photon phase: the photon subpaths (light subpaths traced by the
 // gen / trace / shade kernels into the photon vertex buffer) and the hash
 // grid over their vertices.
@@ -2444,6 +2462,7 @@ int render_vcm(lmx_scene* sc, const lmx_render_params* p, const lmx_vcm_params* 
     pp.sample_out = nullptr;
     int rc = bd_buffers(sc, B, maxv, bd_conn_per_sample(maxv, BD_VCM, true, connect), true);
     if (rc == LMX_OK) rc = vc_buffers(sc, np, maxv, B);
+    if (rc == LMX_OK) vc_buckets(sc, (uint64_t)np * (maxv - 1));
     const size_t npix = (size_t)sc->width * (size_t)sc->height;
     const int zgrid = std::max(1, std::min((int)((3 * npix + 255) / 256), sc->cus * 8));
     BStep gph, geye;
@@ -2584,6 +2603,7 @@ int render_pm(lmx_scene* sc, const lmx_render_params* p, const lmx_pm_params* v,
     PMArgs pa{(int32_t)pcap, bounded ? p->max_num_vertices : -1, v->finalgather, (float)np};
     int rc = bd_buffers(sc, B, ecap, 1);
     if (rc == LMX_OK) rc = vc_buffers(sc, np, pcap, 1);
+    if (rc == LMX_OK) vc_buckets(sc, std::min<uint64_t>((uint64_t)np * (pcap - 1), ROULETTE_BUCKETS * (uint64_t)np));
     const size_t npix = (size_t)sc->width * (size_t)sc->height;
     const int zgrid = std::max(1, std::min((int)((3 * npix + 255) / 256), sc->cus * 8));
     BStep geye;
@@ -2684,6 +2704,7 @@ int render_ppm(lmx_scene* sc, const lmx_render_params* p, const lmx_ppm_params* 
     PMArgs pa{(int32_t)pcap, bounded ? p->max_num_vertices : -1, 1, (float)np};
     int rc = bd_buffers(sc, N, 2, 1);
     if (rc == LMX_OK) rc = vc_buffers(sc, np, pcap, 1);
+    if (rc == LMX_OK) vc_buckets(sc, std::min<uint64_t>((uint64_t)np * (pcap - 1), ROULETTE_BUCKETS * (uint64_t)np));
     if (rc == LMX_OK && sc->ppm_st.n < 2 * (size_t)N && (e = sc->ppm_st.alloc(2 * (size_t)N)) != hipSuccess)
         rc = hip_error(e, "ppm measurement points");
     const size_t npix = (size_t)sc->width * (size_t)sc->height;
@@ -2807,6 +2828,7 @@ int render_sppm(lmx_scene* sc, const lmx_render_params* p, const lmx_ppm_params*
     PMArgs pa{(int32_t)pcap, bounded ? p->max_num_vertices : -1, 1, (float)np};
     int rc = bd_buffers(sc, npix, 2, 1);
     if (rc == LMX_OK) rc = vc_buffers(sc, np, pcap, 1);
+    if (rc == LMX_OK) vc_buckets(sc, std::min<uint64_t>((uint64_t)np * (pcap - 1), ROULETTE_BUCKETS * (uint64_t)np));
     if (rc == LMX_OK && sc->ppm_st.n < 3 * (size_t)npix && (e = sc->ppm_st.alloc(3 * (size_t)npix)) != hipSuccess)
         rc = hip_error(e, "sppm pixel points");
     const int mgrid = std::max(1, std::min((int)((npix + 255) / 256), sc->cus * 16));

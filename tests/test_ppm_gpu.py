@@ -120,3 +120,24 @@ def test_sppm_furnace_closed_form(gpu):
     C = film.cpu().numpy().astype(np.float64).reshape(-1, 3).mean(axis=1)
     want = sum(Le * rho ** (k - 2) for k in range(2, M + 1))
     assert abs(C.mean() - want) < 4 * C.std() / np.sqrt(len(C)) + 0.015 * want, (C.mean(), want)
+
+
+@pytest.mark.gpu
+def test_photon_grid_sizes(gpu):
+    """The photon grid's buckets follow each render's own photons, within
+    buffers that an earlier one made: renders of a scene that has held other
+    photon counts equal those of a fresh one.  One pass, so that every radius
+    is the initial one; a pixel's photons are summed in another order, c of
+    them of one sign, within 2 c 2^-24."""
+    def sppm(s, photons):
+        return s.render_sppm(8, num_iteration_pass=1, num_photon_trace_samples=photons, initial_radius=0.1, seed=5)[0]
+
+    def vcm(s, photons):
+        return s.render_vcm(24 * 16 * 2, num_iteration_pass=1, num_photon_trace_samples=photons, initial_radius=0.1,
+                            max_num_vertices=6, seed=5)[0]
+    one = render.Scene(scenes.cornell_box(24, 16))
+    for fn, photons in ((sppm, 100), (sppm, 70000), (vcm, 20000), (sppm, 70000), (sppm, 40000), (vcm, 30), (vcm, 20000)):
+        got, want = fn(one, photons), fn(render.Scene(scenes.cornell_box(24, 16)), photons)
+        assert float(want.max()) > 0
+        err = float((got - want).abs().max()) / float(want.abs().max())
+        assert err <= 2 * 8192 * 2.0 ** -24, (fn.__name__, photons, err)
