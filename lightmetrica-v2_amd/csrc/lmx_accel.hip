@@ -1047,9 +1047,9 @@ int trace_counters(lmx_accel* a, uint32_t** counters)
 // whatever the number of rays -- in this file-scope array
 // instead of the accel's counter block.  Every GPU the library runs on holds
 // its own copy until the process ends, shared by every call on that GPU;
-// k_clear_cursors clears them before each launch that reads them, so no value carries over from the previous call (two calls that overlap on one
-// GPU, on different streams, race on it).  On the host, `scratch` only
-// stands in for the device symbol: its device address comes from
+// k_clear_cursors clears them before each launch that reads them, so no value
+// carries over from the previous call (two calls that overlap on one GPU, on
+// different streams, race on it).  On the host, `scratch` only stands in for the device symbol: its device address comes from
 // hipGetSymbolAddress, taken once per device with that device current, and
 // only that address is handed to kernels.
 #define LMX_NOALLOC_SCRATCH_WORDS (9 * CURSOR_STRIDE)
