@@ -766,7 +766,9 @@ void k_trace(const WNode* __restrict__ nodes,
                            __uint_as_float(r.oct | ((uint32_t)r.kx << 3) | ((uint32_t)r.ky << 5) | ((uint32_t)r.kz << 7)));
         w[3] = make_float4(r.Sx, r.Sy, r.Sz, __int_as_float(sp));
         w[4] = make_float4(best_t, h0, h1, hdet);
-        L.key[rank] = coop_key(best_t, best_id);
+        // a NaN tmax of either sign bounds nothing in the loop's comparisons
+        // (TriAccel; the watertight test rejects it): the largest key
+        L.key[rank] = coop_key(best_t == best_t ? best_t : __uint_as_float(0x7fc00000u), best_id);
     }
     trace_wave_sync();
     // queued triangles: each lane's bits from its exclusive prefix on

@@ -219,3 +219,26 @@ def test_last_rays_of_a_wave(gpu, n, subdiv, mode):
     np.testing.assert_array_equal(hg.cpu().numpy().view(np.uint32), hh.view(np.uint32))
     np.testing.assert_array_equal(accel.hit_ids(ho.cpu().numpy()) != accel.MISS, accel.hit_ids(hh) != accel.MISS)
     assert a.info()["stack_overflow"] == 0
+
+
+@pytest.mark.parametrize("mode", [accel.ISECT_TRIACCEL, accel.ISECT_WATERTIGHT])
+@pytest.mark.parametrize("n", [9, 2001, 200003])
+def test_unusual_ranges(gpu, n, mode):
+    """tmin and tmax of NaN (either sign), infinity, -0 and crossed: the same
+    hits as the host walker's, bit for bit, whichever part of the kernel
+    traces the ray."""
+    import torch
+    v, f = scenes.displaced_icosphere(3, seed=5)
+    _, rays = scenes.traversal_rays(v, res=2, n_incoherent=n, seed=n)
+    rays = rays.copy()
+    odd = np.array([0x7fc00000, 0xffc00000, 0x7f800000, 0xff800000, 0x80000000, 0x3f000000], np.uint32).view(np.float32)
+    k = np.arange(len(rays))
+    rays[:, 7] = np.where(k % 8 < 6, odd[k % 8 % 6], rays[:, 7])
+    rays[:, 3] = np.where(k % 11 < 6, odd[k % 11 % 6], rays[:, 3])
+    a = accel.Accel(v, f, isect=mode)
+    d = torch.from_numpy(rays).to(gpu)
+    hg, ho = a.intersect(d).cpu().numpy(), a.occluded(d).cpu().numpy()
+    hh = a.intersect_host(rays)
+    np.testing.assert_array_equal(hg.view(np.uint32), hh.view(np.uint32))
+    np.testing.assert_array_equal(accel.hit_ids(ho) != accel.MISS, accel.hit_ids(hh) != accel.MISS)
+    assert n < 100 or (accel.hit_ids(hh) != accel.MISS).any()
