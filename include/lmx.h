@@ -236,7 +236,7 @@ typedef struct lmx_render_params {
 
 typedef struct lmx_render_stats {
     uint64_t rays;               /* extension rays traced */
-    uint32_t iterations;         /* wavefront iterations; 1 when one kernel takes the frame */
+    uint32_t iterations;         /* wavefront iterations; without queues: launches (1 but for very long frames) */
     uint32_t queue_capacity;     /* capacity used (without queues: paths in flight) */
     double ms;                   /* wall time of the render call */
     uint64_t samples;            /* camera samples taken (num_samples unless render_time > 0) */

@@ -452,8 +452,16 @@ __global__ __launch_bounds__(256) void k_nee_splat(RParams p, const Ctl* __restr
 // 64: 8420 / 8100, 80: 10440 / 8410; 1 M paths with next-event estimation:
 // 34: 1545 / 2365, 48: 1680 / 2440, 64: 1790 / 2500.
 #define SMALL_TRIS 48u
-#define SMALL_LENGTH 1024       // vertices: a launch stays short of seconds
-#define SMALL_SAMPLES (1u << 26)
+//
+// A launch is short whatever the number of samples and the length of their
+// paths: after SMALL_STEPS segments a wave starts no further sample, and what
+// is left of the shares goes to another launch.  (Paths of 1,023 segments in a
+// closed sphere of 20 triangles: 97 ms a launch, with next-event estimation
+// 218 ms; 2^26 of them in one launch would hold the device for 6 and 14 s.  The
+// frames of one launch are not slower for it: 373 us before and after.)
+#define SMALL_LENGTH 1024       // vertices: one path stays short of 50 ms
+#define SMALL_STEPS 4096u
+#define SMALL_SAMPLES (1u << 31)
 #define SMALL_BLOCK 256
 #define SMALL_WAVES 5           // waves per SIMD, also workgroups per CU
 #define SMALL_WAVES_NEE 4
@@ -485,12 +493,14 @@ RD uint32_t small_hit(const float4* tris, uint32_t ntri, f3 o, f3 d, float tmin,
     return id;
 }
 
-// Samples begin .. begin + n - 1, n <= SMALL_SAMPLES.  counts[block] (pinned)
-// grows by the rays traced (extension and shadow) by the workgroup.
+// Samples begin .. begin + n - 1, n <= SMALL_SAMPLES, but for those that an
+// earlier launch over them took (resume).  counts[block] (pinned): the rays
+// traced (extension and shadow) by the workgroup and how many samples of its
+// share are done; ctl->pending is set when some are left.
 template <bool NEE>
 __global__ __launch_bounds__(SMALL_BLOCK, NEE ? SMALL_WAVES_NEE : SMALL_WAVES) void k_small_paths(
-    RScene s, RParams p, uint32_t begin, uint32_t n, const WTri* __restrict__ tris, uint32_t ntri,
-    uint64_t* __restrict__ counts)
+    RScene s, RParams p, uint32_t begin, uint32_t n, int resume, const WTri* __restrict__ tris, uint32_t ntri,
+    SmallCount* __restrict__ counts, Ctl* __restrict__ ctl)
 {
     extern __shared__ float4 ordered[];          // 6 orders x ntri x the three vertices; .w of the first: the id
     __shared__ unsigned long long sum[SMALL_BLOCK / 64];
@@ -502,12 +512,12 @@ __global__ __launch_bounds__(SMALL_BLOCK, NEE ? SMALL_WAVES_NEE : SMALL_WAVES) v
         ordered[k] = make_float4(wb_sel3(kx, v[0], v[1], v[2]), wb_sel3(ky, v[0], v[1], v[2]), wb_sel3(kz, v[0], v[1], v[2]),
                                  v[3]);
     }
-    if (threadIdx.x == 0) taken = 0;
+    if (threadIdx.x == 0) taken = resume ? counts[blockIdx.x].done : 0u;
     __syncthreads();
     const uint32_t share = (uint32_t)((uint64_t)n * blockIdx.x / gridDim.x);                // the workgroup's samples
     const uint32_t count = (uint32_t)((uint64_t)n * (blockIdx.x + 1u) / gridDim.x) - share, first = begin + share;
     bool live = false, start = false, more = true;
-    uint32_t rays = 0, sample = 0, seg = 0, pixel = 0;
+    uint32_t rays = 0, sample = 0, seg = 0, pixel = 0, steps = 0;
     f3 o = mk3(0, 0, 0), d = mk3(0, 0, 0);
     float4 thr = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     float tmax = 0.0f;
@@ -520,7 +530,7 @@ __global__ __launch_bounds__(SMALL_BLOCK, NEE ? SMALL_WAVES_NEE : SMALL_WAVES) v
     };
     while (true) {
         const unsigned long long running = __ballot(live);
-        if (more && 64 - __popcll(running) >= (running ? (NEE ? SMALL_IDLE_NEE : 1) : 1)) {
+        if (more && steps < SMALL_STEPS && 64 - __popcll(running) >= (running ? (NEE ? SMALL_IDLE_NEE : 1) : 1)) {
             if (!live) {
                 const uint32_t k = atomicAdd(&taken, 1u);
                 start = k < count;
@@ -544,6 +554,7 @@ __global__ __launch_bounds__(SMALL_BLOCK, NEE ? SMALL_WAVES_NEE : SMALL_WAVES) v
             if (NEE && no.emit) connect(no, no_pixel, true);
         }
         if (__ballot(live) == 0) break;
+        steps++;
         if (live) {
             float4 h;
             rays++;
@@ -573,7 +584,8 @@ __global__ __launch_bounds__(SMALL_BLOCK, NEE ? SMALL_WAVES_NEE : SMALL_WAVES) v
     if (threadIdx.x == 0) {
         uint64_t t = 0;
         for (int w = 0; w < SMALL_BLOCK / 64; w++) t += sum[w];
-        counts[blockIdx.x] += t;
+        counts[blockIdx.x] = {resume ? counts[blockIdx.x].rays + t : t, min(taken, count)};
+        if (taken < count) ctl->pending = 1u;
     }
 }
 
@@ -585,7 +597,15 @@ __global__ void k_init_ctl(Ctl* ctl)
         }
         ctl->iterations = 0; ctl->rays = 0; ctl->shadow_rays = 0; ctl->stop = 0; ctl->ray_out_n = 0;
         ctl->film_scaled = 0;
+        ctl->pending = 0;
     }
+}
+
+// Clears the film for k_small_paths, and the flag of samples left.
+__global__ void k_small_begin(Ctl* __restrict__ ctl, float* a, size_t n)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0) ctl->pending = 0;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) a[i] = 0.0f;
 }
 
 // Measurement hook: copies the queue about to be traced (the first
@@ -619,6 +639,13 @@ __global__ void k_zero(float* a, size_t n)
 
 __global__ void k_scale(float* a, size_t n, float w)
 {
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) a[i] *= w;
+}
+
+// The same at the end of a render by k_small_paths, when no sample is left.
+__global__ void k_scale_unless_pending(const Ctl* __restrict__ ctl, float* a, size_t n, float w)
+{
+    if (ctl->pending) return;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) a[i] *= w;
 }
 
@@ -871,35 +898,48 @@ int autotune_capacity(lmx_scene* sc, const RParams& rp, hipStream_t st)
 
 // One frame by k_small_paths, with about `cap` paths in flight at most.
 static int render_small(lmx_scene* sc, const RParams& rp, const WTri* tris, uint32_t ntri, uint32_t cap, hipStream_t st,
-                        size_t npix, uint64_t* rays, uint32_t* flight)
+                        size_t npix, uint64_t* rays, uint32_t* flight, uint32_t* launches)
 {
     const uint32_t most = (uint32_t)sc->cus * (rp.nee == NEE_NONE ? SMALL_WAVES : SMALL_WAVES_NEE);
     const uint32_t want = (uint32_t)(((uint64_t)std::min(rp.total, cap) + SMALL_BLOCK - 1) / SMALL_BLOCK);
     const uint32_t grid = std::max(1u, std::min(most, want));
     const size_t lds = 18 * (size_t)ntri * sizeof(float4);
+    const int fgrid = std::max(1, std::min((int)((3 * npix + 255) / 256), sc->cus * 8));
     hipError_t e;
     if (!sc->h_counts) {
-        const size_t bytes = (size_t)sc->cus * std::max(SMALL_WAVES, SMALL_WAVES_NEE) * sizeof(uint64_t);
+        const size_t bytes = (size_t)sc->cus * std::max(SMALL_WAVES, SMALL_WAVES_NEE) * sizeof(SmallCount);
         if ((e = hipHostMalloc((void**)&sc->h_counts, bytes, hipHostMallocDefault)) != hipSuccess) {
             sc->h_counts = nullptr;
             return hip_error(e, "pinned ray counts");
         }
     }
-    std::fill(sc->h_counts, sc->h_counts + grid, (uint64_t)0);
+    *rays = 0;
+    *launches = 0;
+    *flight = grid * SMALL_BLOCK;
+    k_small_begin<<<fgrid, 256, 0, st>>>(sc->ctl.p, rp.film, 3 * npix);
     for (uint64_t b = 0; b < rp.total; b += SMALL_SAMPLES) {
         const uint32_t n = (uint32_t)std::min<uint64_t>(SMALL_SAMPLES, rp.total - b);
-        if (rp.nee == NEE_NONE)
-            k_small_paths<false><<<grid, SMALL_BLOCK, lds, st>>>(sc->rs, rp, (uint32_t)b, n, tris, ntri, sc->h_counts);
-        else
-            k_small_paths<true><<<grid, SMALL_BLOCK, lds, st>>>(sc->rs, rp, (uint32_t)b, n, tris, ntri, sc->h_counts);
+        const bool last = b + n == rp.total;
+        uint64_t done = 0, traced = 0;
+        for (int resume = 0; done < n; resume = 1) {
+            if (resume) k_small_begin<<<1, 64, 0, st>>>(sc->ctl.p, nullptr, 0);
+            auto launch = [&](auto kernel) {
+                kernel<<<grid, SMALL_BLOCK, lds, st>>>(sc->rs, rp, (uint32_t)b, n, resume, tris, ntri, sc->h_counts, sc->ctl.p);
+            };
+            if (rp.nee == NEE_NONE) launch(k_small_paths<false>);
+            else launch(k_small_paths<true>);
+            if (last) k_scale_unless_pending<<<fgrid, 256, 0, st>>>(sc->ctl.p, rp.film, 3 * npix, (float)((double)npix / (double)rp.total));
+            if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(st)) != hipSuccess)
+                return hip_error(e, "small-scene render");
+            ++*launches;
+            done = traced = 0;
+            for (uint32_t k = 0; k < grid; k++) {
+                done += sc->h_counts[k].done;
+                traced += sc->h_counts[k].rays;
+            }
+        }
+        *rays += traced;
     }
-    k_scale<<<std::max(1, std::min((int)((3 * npix + 255) / 256), sc->cus * 8)), 256, 0, st>>>(
-        rp.film, 3 * npix, (float)((double)npix / (double)rp.total));
-    if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(st)) != hipSuccess)
-        return hip_error(e, "small-scene render");
-    *rays = 0;
-    for (uint32_t k = 0; k < grid; k++) *rays += sc->h_counts[k];
-    *flight = grid * SMALL_BLOCK;
     return LMX_OK;
 }
 
@@ -959,19 +999,19 @@ static int render_unidir(lmx_scene* sc, const lmx_render_params* p, int nee, con
     uint32_t cap = 0, iters = 0;
     uint64_t rays = 0, taken = 0;
     // few triangles (SMALL_TRIS), nothing asked for that belongs to the queues,
-    // and paths that end by themselves: the one kernel runs until the longest
-    // has, while the queues return to the host every few segments
+    // and paths that end by themselves: a launch of the one kernel ends when the
+    // last path it started has, while the queues return to the host every few
+    // segments
     const bool ends = p->max_num_vertices != -1 ? p->max_num_vertices <= SMALL_LENGTH
                                                 : p->rr_mode == LMX_RR_FIXED && p->rr_prob <= 0.9f && p->rr_depth <= SMALL_LENGTH;
     uint32_t ntri = 0;
     const WTri* tris = trace_triangles(sc->accel, &ntri);
     const bool small = ends && tris && ntri <= SMALL_TRIS && !timed && !rp.ray_out && p->shade_order == LMX_SHADE_QUEUE;
     if (small) {
-        k_zero<<<zgrid, 256, 0, st>>>(film_rgb, 3 * npix);
-        rc = render_small(sc, rp, tris, ntri, p->queue_capacity ? p->queue_capacity : 0xffffffffu, st, npix, &rays, &cap);
+        rc = render_small(sc, rp, tris, ntri, p->queue_capacity ? p->queue_capacity : 0xffffffffu, st, npix, &rays, &cap,
+                          &iters);
         if (p->queue_capacity) cap = (uint32_t)std::min<uint64_t>(p->queue_capacity, std::max<uint64_t>(p->num_samples, 64));
         taken = p->num_samples;
-        iters = 1;
     } else {
         if (p->queue_capacity == 0 && sc->tuned_cap == 0) rc = autotune_capacity(sc, rp, st);
         cap = p->queue_capacity ? p->queue_capacity : sc->tuned_cap;

@@ -47,6 +47,12 @@ struct RScene {
     int32_t width, height;
 };
 
+// What a workgroup of a small-scene render has done of its share.
+struct SmallCount {
+    uint64_t rays;             // extension and shadow rays traced
+    uint32_t done;             // samples
+};
+
 // Uniform of (sample, slot) from the table or from Philox.
 // Device-side control block.  The counts come in pairs: an iteration that
 // traces queue a and fills queue b = 1 - a reads [a] and writes [b], so that
@@ -64,6 +70,7 @@ struct Ctl {
     uint32_t bin[4];           // material-binned shading: paths per class this iteration
     uint32_t ray_out_n;        // rays copied to RParams::ray_out so far
     uint32_t film_scaled;      // the film was rescaled on the device at the render's end
+    uint32_t pending;          // small scenes: a launch ended with samples left
 };
 
 // Shading classes of material-binned shading: paths that end at their hit
@@ -555,7 +562,7 @@ struct lmx_scene {
     DevBuf<uint32_t> perm;              // material-binned shading, SHADE_CLASSES x cap
     DevBuf<Ctl> ctl;
     Ctl* h_ctl = nullptr;      // pinned
-    uint64_t* h_counts = nullptr;       // pinned: rays per workgroup of a small-scene render
+    lmx::SmallCount* h_counts = nullptr;     // pinned: what each workgroup of a small-scene render has done
     hipGraphExec_t wf_exec = nullptr;   // the wavefront iterations' graph, updated in place per render
     hipStream_t cap_stream = nullptr;   // records that graph and runs nothing
     uint32_t tuned_cap = 0;

@@ -272,3 +272,25 @@ def test_few_triangles_beyond_one_launch(gpu):
     assert sa["rays"] == sb["rays"] == n and sa["samples"] == sb["samples"] == n
     # FP32 sums of n / (33 21) terms of one sign in another order, both rounded
     assert float((fa - fb).abs().max()) <= 2 * 1.1 * n / (33 * 21) * 2.0 ** -24 * float(fb.abs().max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cap,n", [(64, 5000), (256, 1200), (600, 20000)])
+@pytest.mark.parametrize("entry", ["pt", "ptmis", "ptdirect"])
+def test_few_triangles_long_paths(gpu, entry, cap, n):
+    """Paths of 1,023 segments in a closed scene of few triangles, more of
+    them than a launch may start (4,096 segments a wave, four waves to each
+    256 paths in flight): several launches, the samples of each workgroup
+    continued where the last one stopped, and the frame of the queues."""
+    rs = render.Scene(scenes.furnace_sphere(albedo=0.9, Le=1.0, subdiv=0, width=16, height=12))
+    opts = dict(max_num_vertices=1024, rr_depth=2000, seed=9, sample_out=True)
+    fa, sa, ra = getattr(rs, "render_" + entry)(n, queue_capacity=cap, **opts)
+    fb, sb, rb = getattr(rs, "render_" + entry)(n, queue_capacity=1 << 15, shade_order=render.SHADE_BY_MATERIAL, **opts)
+    lanes = (cap + 255) // 256 * 256
+    steps = n * 1023.0 / lanes                 # of a wave, if its lanes never idle
+    assert steps / (4096 + 1023) * 0.9 <= sa["iterations"] <= steps / 4096 * 1.5 + 2
+    assert sa["rays"] == sb["rays"] > 1000 * n and sa["samples"] == sb["samples"] == n
+    assert np.array_equal(np.asarray(ra.cpu()).view(np.uint32), np.asarray(rb.cpu()).view(np.uint32))
+    # FP32 sums of at most 1,023 segments and as many connections of every sample of a pixel, in another order
+    c = 2 * 1024.0 * (n / (16 * 12) + 1)
+    assert float((fa - fb).abs().max()) <= c * 2.0 ** -24 * float(fb.abs().max())
