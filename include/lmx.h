@@ -278,7 +278,10 @@ int lmx_render_ptmis(lmx_scene *scene, const lmx_render_params *params, float *f
  * all strategies.  Uses max_num_vertices (2..32), min_num_vertices, seed,
  * num_samples, raster_mode; queue_capacity is the batch size in samples
  * (0 = autotuned per scene and max_num_vertices: the fastest of 2^19..2^24
- * that fits half of free device memory).  Uniform table width >= 2 (8 + 4 (max_num_vertices - 1)): an
+ * that fits half of free device memory).  The connections of a batch wait in
+ * a queue of 24 slots of 96 B a sample, or, where that takes at most 4 GB and
+ * the batch with it half of free device memory, of as many as its samples can
+ * have.  Uniform table width >= 2 (8 + 4 (max_num_vertices - 1)): an
  * eye block then a light block, each laid out as for lmx_render_pt except
  * 1-2 emitter position, 3 emitter selection, 4-5 emitter direction.
  * sample_out, when given, holds (max_num_vertices + 1)^2 records of 8 floats

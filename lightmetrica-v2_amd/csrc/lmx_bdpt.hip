@@ -1811,9 +1811,10 @@ uint32_t bd_conn_per_sample(uint32_t maxv, int variant, bool bounded, bool conne
 #define BD_ROUND_SLOTS 24u
 
 // But while the worst case of the whole batch takes at most this many bytes,
-// the queue holds it: then one round is certain to be enough and nothing has
-// to be read back to know that no sample is left (about 50 us per batch, 1.2
-// GB for 262,144 samples of renderer::vcm at 10 vertices).
+// and the batch with it at most half of the free memory (bd_buffers), the
+// queue holds it: then one round is certain to be enough and nothing has to be
+// read back to know that no sample is left (about 50 us per batch, 1.2 GB for
+// 262,144 samples of renderer::vcm at 10 vertices).
 #define BD_WHOLE_QUEUE_BYTES (4ull << 30)
 #define BD_SLOT_BYTES 96u
 
@@ -1849,19 +1850,30 @@ void bd_release(lmx_scene* sc)
     sc->bd_nconn = 0;
 }
 
-// Device bytes the scene's batch buffers hold.
-size_t bd_held_bytes(const lmx_scene* sc)
+// Device bytes of the buffers for batches of B samples of up to maxv vertices
+// with nconn connection slots.
+size_t bd_batch_bytes(size_t B, size_t maxv, size_t nconn)
 {
-    const size_t B = sc->bd_batch, nv = B * sc->bd_maxv * 4;
-    return 2 * (nv * 16 + B * 4 + 4 * B * 16 + 2 * B * 16 + 2 * B * 16) + B * sc->bd_maxv * 4 + B * 4 + B * 8 +
-           2 * B * 16 + (B + 1) * 4 + B * 4 + (size_t)sc->bd_nconn * (2 * 16 + 4 * 16);
+    const size_t nv = B * maxv * 4;
+    return 2 * (nv * 16 + B * 4 + 4 * B * 16 + 2 * B * 16 + 2 * B * 16) + B * maxv * 4 + B * 4 + B * 8 +
+           2 * B * 16 + (B + 1) * 4 + B * 4 + nconn * BD_SLOT_BYTES;
 }
 
-// Buffers for batches of B samples of up to maxv vertices and `conn`
-// shadow-queue slots per sample.  With `rounds` (the samplers that connect
-// in rounds), conn is a sample's worst case and the queue holds the whole
-// batch's where that is small, else one round (never less than one sample's
-// worst case).
+// Device bytes the scene's batch buffers hold.
+size_t bd_held_bytes(const lmx_scene* sc) { return bd_batch_bytes(sc->bd_batch, sc->bd_maxv, sc->bd_nconn); }
+
+// Half of the free device memory, what the scene's batch buffers hold counting
+// as free.
+hipError_t bd_budget(const lmx_scene* sc, size_t* bytes)
+{
+    size_t free_b = 0, total_b = 0;
+    const hipError_t e = hipMemGetInfo(&free_b, &total_b);
+    *bytes = (free_b + bd_held_bytes(sc)) / 2;
+    return e;
+}
+
+// Buffers for batches of B samples of up to maxv vertices and nconn
+// shadow-queue slots (conn per sample).
 int bd_buffers_of(lmx_scene* sc, uint32_t B, uint32_t maxv, uint32_t conn, size_t nconn)
 {
     if (nconn > 0xffffffffull) return set_error(LMX_EINVAL, "bdpt buffers: more than 2^32 - 1 connection slots");
@@ -1897,15 +1909,35 @@ int bd_buffers_of(lmx_scene* sc, uint32_t B, uint32_t maxv, uint32_t conn, size_
     return LMX_OK;
 }
 
+// Buffers for batches of B samples of up to maxv vertices and `conn`
+// shadow-queue slots per sample, and what else the render allocates (`others`).
+// With `rounds` (the samplers that connect in rounds), conn is a sample's
+// worst case and the queue holds the whole batch's where that is small, else
+// one round (never less than one sample's worst case).  A queue larger than
+// the render needs makes way when the others find no room beside it; a size
+// that found none is not tried again.
+template <typename F>
+int bd_buffers(lmx_scene* sc, uint32_t B, uint32_t maxv, uint32_t conn, bool rounds, F&& others)
+{
+    const size_t whole = (size_t)B * conn, need = rounds ? bd_round_queue(B, conn) : whole;
+    size_t queue = need, budget = 0;
+    if (whole > need && (uint64_t)whole * BD_SLOT_BYTES <= BD_WHOLE_QUEUE_BYTES && whole < sc->bd_no_room &&
+        ((B <= sc->bd_batch && maxv <= sc->bd_maxv && whole <= sc->bd_nconn) ||
+         (bd_budget(sc, &budget) == hipSuccess && bd_batch_bytes(B, maxv, whole) <= budget)))
+        queue = whole;
+    int rc = bd_buffers_of(sc, B, maxv, conn, queue);
+    if (rc == LMX_OK) rc = others();
+    if (rc == LMX_OK || std::max((size_t)sc->bd_nconn, queue) <= need) return rc;
+    (void)hipGetLastError();
+    if (queue > need) sc->bd_no_room = queue;
+    bd_release(sc);
+    rc = bd_buffers_of(sc, B, maxv, conn, need);
+    return rc == LMX_OK ? others() : rc;
+}
+
 int bd_buffers(lmx_scene* sc, uint32_t B, uint32_t maxv, uint32_t conn, bool rounds = false)
 {
-    const size_t whole = (size_t)B * conn;
-    if (!rounds) return bd_buffers_of(sc, B, maxv, conn, whole);
-    if ((uint64_t)whole * BD_SLOT_BYTES <= BD_WHOLE_QUEUE_BYTES) {
-        if (bd_buffers_of(sc, B, maxv, conn, whole) == LMX_OK) return LMX_OK;
-        (void)hipGetLastError();               // no room for that: rounds need less
-    }
-    return bd_buffers_of(sc, B, maxv, conn, bd_round_queue(B, conn));
+    return bd_buffers(sc, B, maxv, conn, rounds, [] { return LMX_OK; });
 }
 
 // The batch's buffers.
@@ -2116,10 +2148,9 @@ int bd_autotune(lmx_scene* sc, BParams bp, uint64_t num_samples, float* film, hi
     // 2^23 and 2^24 (110 GB at max_num_vertices 10) lift renderer::bdpt on a
     // 1024^2 x 16 spp frame from 342 to 384 and 403 Msamples/s
     static const uint32_t cands[] = {1u << 19, 1u << 20, 1u << 21, 1u << 22, 1u << 23, 1u << 24};
-    size_t free_b = 0, total_b = 0;
-    hipError_t e = hipMemGetInfo(&free_b, &total_b);
+    size_t budget = 0;
+    hipError_t e = bd_budget(sc, &budget);
     if (e != hipSuccess) return hip_error(e, "bdpt autotune: memory info");
-    const size_t budget = (free_b + bd_held_bytes(sc)) / 2;
     const uint32_t conn = bd_conn_per_sample((uint32_t)bp.maxv, bp.variant, bp.bounded != 0);
     const size_t per = bd_bytes_per_sample((uint32_t)bp.maxv, conn);
     bp.sample_out = nullptr;
@@ -2460,8 +2491,8 @@ int render_vcm(lmx_scene* sc, const lmx_render_params* p, const lmx_vcm_params* 
     pp.key = make_uint2((uint32_t)v->photon_seed, (uint32_t)(v->photon_seed >> 32));
     pp.table = v->photon_table; pp.table_width = v->photon_table_width;
     pp.sample_out = nullptr;
-    int rc = bd_buffers(sc, B, maxv, bd_conn_per_sample(maxv, BD_VCM, true, connect), true);
-    if (rc == LMX_OK) rc = vc_buffers(sc, np, maxv, B);
+    int rc = bd_buffers(sc, B, maxv, bd_conn_per_sample(maxv, BD_VCM, true, connect), true,
+                        [&] { return vc_buffers(sc, np, maxv, B); });
     if (rc == LMX_OK) vc_buckets(sc, (uint64_t)np * (maxv - 1));
     const size_t npix = (size_t)sc->width * (size_t)sc->height;
     const int zgrid = std::max(1, std::min((int)((3 * npix + 255) / 256), sc->cus * 8));
@@ -2601,8 +2632,7 @@ int render_pm(lmx_scene* sc, const lmx_render_params* p, const lmx_pm_params* v,
     pp.wsub = 0;
     pp.sample_out = nullptr;
     PMArgs pa{(int32_t)pcap, bounded ? p->max_num_vertices : -1, v->finalgather, (float)np};
-    int rc = bd_buffers(sc, B, ecap, 1);
-    if (rc == LMX_OK) rc = vc_buffers(sc, np, pcap, 1);
+    int rc = bd_buffers(sc, B, ecap, 1, false, [&] { return vc_buffers(sc, np, pcap, 1); });
     if (rc == LMX_OK) vc_buckets(sc, std::min<uint64_t>((uint64_t)np * (pcap - 1), ROULETTE_BUCKETS * (uint64_t)np));
     const size_t npix = (size_t)sc->width * (size_t)sc->height;
     const int zgrid = std::max(1, std::min((int)((3 * npix + 255) / 256), sc->cus * 8));
@@ -2702,11 +2732,12 @@ int render_ppm(lmx_scene* sc, const lmx_render_params* p, const lmx_ppm_params* 
     pp.wsub = 0;
     pp.sample_out = nullptr;
     PMArgs pa{(int32_t)pcap, bounded ? p->max_num_vertices : -1, 1, (float)np};
-    int rc = bd_buffers(sc, N, 2, 1);
-    if (rc == LMX_OK) rc = vc_buffers(sc, np, pcap, 1);
+    int rc = bd_buffers(sc, N, 2, 1, false, [&] {
+        const int rc2 = vc_buffers(sc, np, pcap, 1);
+        if (rc2 != LMX_OK || sc->ppm_st.n >= 2 * (size_t)N || (e = sc->ppm_st.alloc(2 * (size_t)N)) == hipSuccess) return rc2;
+        return hip_error(e, "ppm measurement points");
+    });
     if (rc == LMX_OK) vc_buckets(sc, std::min<uint64_t>((uint64_t)np * (pcap - 1), ROULETTE_BUCKETS * (uint64_t)np));
-    if (rc == LMX_OK && sc->ppm_st.n < 2 * (size_t)N && (e = sc->ppm_st.alloc(2 * (size_t)N)) != hipSuccess)
-        rc = hip_error(e, "ppm measurement points");
     const size_t npix = (size_t)sc->width * (size_t)sc->height;
     const int zgrid = std::max(1, std::min((int)((3 * npix + 255) / 256), sc->cus * 8));
     const int mgrid = std::max(1, std::min((int)((N + 255) / 256), sc->cus * 16));
@@ -2826,11 +2857,13 @@ int render_sppm(lmx_scene* sc, const lmx_render_params* p, const lmx_ppm_params*
     pp.wsub = 0;
     pp.sample_out = nullptr;
     PMArgs pa{(int32_t)pcap, bounded ? p->max_num_vertices : -1, 1, (float)np};
-    int rc = bd_buffers(sc, npix, 2, 1);
-    if (rc == LMX_OK) rc = vc_buffers(sc, np, pcap, 1);
+    int rc = bd_buffers(sc, npix, 2, 1, false, [&] {
+        const int rc2 = vc_buffers(sc, np, pcap, 1);
+        if (rc2 != LMX_OK || sc->ppm_st.n >= 3 * (size_t)npix || (e = sc->ppm_st.alloc(3 * (size_t)npix)) == hipSuccess)
+            return rc2;
+        return hip_error(e, "sppm pixel points");
+    });
     if (rc == LMX_OK) vc_buckets(sc, std::min<uint64_t>((uint64_t)np * (pcap - 1), ROULETTE_BUCKETS * (uint64_t)np));
-    if (rc == LMX_OK && sc->ppm_st.n < 3 * (size_t)npix && (e = sc->ppm_st.alloc(3 * (size_t)npix)) != hipSuccess)
-        rc = hip_error(e, "sppm pixel points");
     const int mgrid = std::max(1, std::min((int)((npix + 255) / 256), sc->cus * 16));
     const float r0 = v->initial_radius, cell = (float)(2.0 * (double)r0);
     VB vb;
@@ -2929,8 +2962,7 @@ int render_ltdirect(lmx_scene* sc, const lmx_render_params* p, float* film_rgb, 
     pp.wsub = 0;
     pp.sample_out = p->sample_out;
     pp.film = film_rgb;
-    int rc = bd_buffers(sc, B, 2, pcap);
-    if (rc == LMX_OK) rc = vc_buffers(sc, B, pcap, 1);
+    int rc = bd_buffers(sc, B, 2, pcap, false, [&] { return vc_buffers(sc, B, pcap, 1); });
     const size_t npix = (size_t)sc->width * (size_t)sc->height;
     const int zgrid = std::max(1, std::min((int)((3 * npix + 255) / 256), sc->cus * 8));
     const int cap_grid = sc->cus * 8;

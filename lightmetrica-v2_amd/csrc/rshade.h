@@ -569,6 +569,7 @@ struct lmx_scene {
     // bidirectional sampler buffers (sized for bd_batch samples, bd_maxv vertices)
     uint32_t bd_batch = 0, bd_maxv = 0, bd_conn = 0;   // bd_conn: shadow-queue slots per sample and round
     uint32_t bd_nconn = 0;              // shadow-queue slots of one connection round
+    size_t bd_no_room = SIZE_MAX;       // a whole batch's slots that did not fit the device
     uint32_t bd_tuned_batch = 0, bd_tuned_key = 0;      // autotuned batch for one (variant, max_num_vertices)
     uint64_t bd_tuned_limit = 0;        // largest candidate the tuning run allowed (render size rounded up)
     DevBuf<float4> bd_vert[2];          // per subpath vertex: 4 float4 (see lmx_bdpt.hip)

@@ -164,3 +164,63 @@ def test_connection_rounds_beyond_the_queue(gpu, sampler, maxv, n):
     a, b = one.cpu().numpy().astype(np.float64), many.cpu().numpy().astype(np.float64)
     per_pixel = st["rays"] / 64.0
     assert a.min() > 0.5 and np.abs(a - b).max() <= per_pixel * 2.0 ** -24 * b.max()
+
+
+@pytest.fixture
+def little_memory(gpu):
+    """Leaves 3,000 MB of the device free, the rest held by tensors."""
+    import gc
+    import torch
+    gc.collect()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    hold = []
+    for _ in range(10):                        # memory freed just before comes back late
+        extra = torch.cuda.mem_get_info()[0] - (3000 << 20)
+        if extra < 64 << 20:
+            break
+        hold.append(torch.empty(extra, dtype=torch.uint8, device=gpu))
+    yield lambda: torch.cuda.mem_get_info()[0]
+    hold.clear()
+    torch.cuda.empty_cache()
+
+
+def test_connection_queue_takes_half_of_free_memory_at_most(gpu, little_memory):
+    """A batch whose worst case takes 1.8 GB in all where 3 GB are free waits
+    in the queue of 24 slots a sample (1.2 GB); another render of it keeps the
+    buffers; the film is that of batches that hold their worst case."""
+    rs = render.Scene(scenes.cornell_box(16, 16))
+    n = 300000
+    free = little_memory()
+    assert free < 3100 << 20
+    film, st, _ = rs.render_vcm_bdpt(n, max_num_vertices=10, seed=3, batch=n)
+    used = free - little_memory()
+    assert st["batches"] == 1 and 1000 << 20 < used < free // 2
+    again = rs.render_vcm_bdpt(n, max_num_vertices=10, seed=3, batch=n)[0]
+    assert abs(free - used - little_memory()) < 16 << 20
+    small = render.Scene(scenes.cornell_box(16, 16)).render_vcm_bdpt(n, max_num_vertices=10, seed=3, batch=50000)[0]
+    # FP32 sums of up to 46 strategies of every sample of a pixel in another order
+    tol = 46.0 * n / 256 * 2.0 ** -24 * float(small.max())
+    assert float((film - small).abs().max()) <= tol and float((again - small).abs().max()) <= tol
+
+
+def test_connection_queue_makes_way_for_photons(gpu, little_memory):
+    """renderer::vcm where the batch's worst case (1.2 GB) and the photon
+    buffers (2.1 GB) do not fit together but the queue of 24 slots a sample
+    and the photons do; and photon mapping after a render that left the scene
+    a large queue."""
+    def vcm(s, photons):
+        return s.render_vcm(200000, num_iteration_pass=1, num_photon_trace_samples=photons, initial_radius=1e-3,
+                            max_num_vertices=10, seed=3)[0]
+    rs = render.Scene(scenes.cornell_box(16, 16))
+    film = vcm(rs, 1950000)
+    assert float(film.max()) > 0
+    other = vcm(rs, 1950000)
+    assert float((film - other).abs().max()) <= 1e-3 * float(film.max())
+    del rs
+    rs = render.Scene(scenes.cornell_box(16, 16))
+    rs.render_vcm_bdpt(200000, max_num_vertices=10, seed=3, batch=200000)
+    free = little_memory()
+    assert float(rs.render_pm(100000, num_photon_trace_samples=1900000, radius=0.01, max_num_vertices=10, seed=3,
+                              batch=100000)[0].max()) > 0
+    assert little_memory() < free
