@@ -995,7 +995,7 @@ static int render_unidir(lmx_scene* sc, const lmx_render_params* p, int nee, con
     rp.ray_out = p->ray_out && p->ray_out_cap ? reinterpret_cast<float4*>(p->ray_out) : nullptr;
     rp.ray_out_cap = rp.ray_out ? p->ray_out_cap : 0u;
     const int zgrid = std::max(1, std::min((int)((3 * npix + 255) / 256), sc->cus * 8));
-    int rc = LMX_OK;
+    int rc = lmx_accel_upload(sc->accel);   // a scene of another device is refused before anything is launched
     uint32_t cap = 0, iters = 0;
     uint64_t rays = 0, taken = 0;
     // few triangles (SMALL_TRIS), nothing asked for that belongs to the queues,
@@ -1007,12 +1007,12 @@ static int render_unidir(lmx_scene* sc, const lmx_render_params* p, int nee, con
     uint32_t ntri = 0;
     const WTri* tris = trace_triangles(sc->accel, &ntri);
     const bool small = ends && tris && ntri <= SMALL_TRIS && !timed && !rp.ray_out && p->shade_order == LMX_SHADE_QUEUE;
-    if (small) {
+    if (rc == LMX_OK && small) {
         rc = render_small(sc, rp, tris, ntri, p->queue_capacity ? p->queue_capacity : 0xffffffffu, st, npix, &rays, &cap,
                           &iters);
         if (p->queue_capacity) cap = (uint32_t)std::min<uint64_t>(p->queue_capacity, std::max<uint64_t>(p->num_samples, 64));
         taken = p->num_samples;
-    } else {
+    } else if (rc == LMX_OK) {
         if (p->queue_capacity == 0 && sc->tuned_cap == 0) rc = autotune_capacity(sc, rp, st);
         cap = p->queue_capacity ? p->queue_capacity : sc->tuned_cap;
         if (!timed) cap = (uint32_t)std::min<uint64_t>(cap, std::max<uint64_t>(p->num_samples, 64));

@@ -100,3 +100,17 @@ def test_guide_errors(rs):
     assert lib.lmx_guide_eval(g._h, None, 4, None, None) == -1
     x = torch.rand((0, 7), device="cuda")
     assert g.eval(x).shape == (0, 41)
+
+
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="a scene is refused on another device than its own: needs two")
+@pytest.mark.parametrize("order", [render.SHADE_QUEUE, render.SHADE_BY_MATERIAL])
+@pytest.mark.parametrize("entry", ["render_pt", "render_ptdirect", "render_ptmis"])
+def test_scene_of_another_device(entry, order):
+    """The one kernel for few triangles and the queues both refuse it."""
+    with torch.cuda.device(0):
+        rs = render.Scene(scenes.cornell_box(16, 16))
+    with torch.cuda.device(1):
+        with pytest.raises(LmxError, match="another device"):
+            getattr(rs, entry)(1024, max_num_vertices=5, queue_capacity=1024, shade_order=order)
+    with torch.cuda.device(0):
+        assert float(getattr(rs, entry)(1024, max_num_vertices=5, shade_order=order)[0].max()) > 0
