@@ -41,6 +41,7 @@
 #include <mutex>
 #include <string>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "lmx.h"
@@ -81,8 +82,9 @@ struct lmx_accel {
     WNode* d_nodes = nullptr;
     WTri* d_tris = nullptr;
     uint32_t* d_counters = nullptr;   // 8 region cursors, a free line, the stack-overflow flag; CURSOR_STRIDE words apart
-    int grid = 0;                     // waves of a launch
-    int grid_occl = 0;                // waves of an occlusion launch over many rays
+    int grid_full = 0;                // waves that the device holds at once
+    int grid = 0;                     // waves of a launch over few rays, or over a queue (trace_shape)
+    bool large = false;               // the tree exceeds an XCD's L2
     int stack_depth = 0;              // LDS stack entries per lane
     size_t lds_bytes = 0;
 };
@@ -500,7 +502,8 @@ __device__ __forceinline__ void coop_trace(CoopLds& L, uint32_t* node, uint32_t 
 // workgroups per CU (22 at depth 8, where the registers allow 20).
 // ANYHIT: stop at the first accepted triangle (shadow rays); the hit record
 // then names that triangle, not necessarily the closest.
-template <int ISECT, bool ANYHIT>
+// TAIL: end in coop_trace; without it (trace_shape) the loop runs to the end.
+template <int ISECT, bool ANYHIT, bool TAIL>
 __global__ __launch_bounds__(TRACE_WAVE) __attribute__((amdgpu_waves_per_eu(LMX_TRACE_WAVES_PER_EU)))
 void k_trace(const WNode* __restrict__ nodes,
                                                       const WTri* __restrict__ tris,
@@ -523,7 +526,7 @@ void k_trace(const WNode* __restrict__ nodes,
         __ballot(lane < 8u && region_dyn_start(lane & 7u, nray, gridDim.x, claim) < region_end(lane & 7u, nray)) ? 8u : 0u;
     __shared__ TraceLds lds;
     TraceTables& s_tab = lds.tab;
-    if (regions_left != 0 || claim > coop_max) {   // else the one-ray-per-lane loop runs no iteration
+    if (!TAIL || regions_left != 0 || claim > coop_max) {   // else the one-ray-per-lane loop runs no iteration
         const uint4* src = reinterpret_cast<const uint4*>(&g_trace_tables);
         uint4* dst = reinterpret_cast<uint4*>(&s_tab);
         for (uint32_t i = lane; i < (uint32_t)(sizeof(TraceTables) / 16); i += TRACE_WAVE) dst[i] = src[i];
@@ -656,7 +659,9 @@ void k_trace(const WNode* __restrict__ nodes,
         // single loop back-edge: with no ray in any lane and work left, the
         // body below does nothing but reload the root.  The last rays of the
         // wave go to coop_trace.
-        if (regions_left == 0 && pool_cnt == 0) {
+        if (!TAIL) {
+            if (__ballot(valid) == 0 && regions_left == 0 && pool_cnt == 0) break;
+        } else if (regions_left == 0 && pool_cnt == 0) {
             const uint32_t left = (uint32_t)__popcll(__ballot(valid));
             if (left == 0) break;
             if (left <= coop_max) {
@@ -745,6 +750,8 @@ void k_trace(const WNode* __restrict__ nodes,
         }
     }
     if (done) write_hit<ISECT>(hits, ray_id, best_t, best_id, h0, h1, hdet);
+
+    if (!TAIL) return;
 
     // ---- the wave's last rays
     const uint64_t act = __ballot(valid);
@@ -951,24 +958,14 @@ int lmx_accel_upload(lmx_accel* a)
     a->lds_bytes = (size_t)a->stack_depth * TRACE_WAVE * sizeof(uint2);
     int per_cu = 0;
     if (a->host.isect == WBVH_ISECT_WATERTIGHT)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_trace<WBVH_ISECT_WATERTIGHT, false>, TRACE_WAVE, a->lds_bytes);
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_trace<WBVH_ISECT_WATERTIGHT, false, true>, TRACE_WAVE, a->lds_bytes);
     else
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_trace<WBVH_ISECT_TRIACCEL, false>, TRACE_WAVE, a->lds_bytes);
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_trace<WBVH_ISECT_TRIACCEL, false, true>, TRACE_WAVE, a->lds_bytes);
     if (e != hipSuccess) return hip_error(e, "lmx_accel_upload: occupancy query");
-    // Waves per CU.  The 64 rays of a wave each walk their own part of the
-    // tree, and where the tree is larger than an XCD's 4 MB of L2 what more
-    // waves gain in latency hidden they lose in the 32 KB L1: 8,388,608 rays
-    // over 75 MB of tree take 947 us with 20 waves (what the registers
-    // allow), 932 with 16, 984 with 14; renderer::vcm passes over as much 5 %
-    // less with 16 than with 20.  A tree within the L2 (the Cornell box) is
-    // traced 2 % faster by 20 waves than by 16.  Shadow rays of a large
-    // batch, each from another place, thrash it sooner: 3,000,001 of them
-    // over 18 MB take 887 us with 20 waves, 836 with 16, 746 with 12, and 812
-    // with 10.
     per_cu = std::max(1, per_cu);
-    const bool large = nb + tb > ((size_t)4 << 20);
-    a->grid = std::max(8, cus * (large ? std::min(per_cu, 16) : per_cu));
-    a->grid_occl = std::max(8, cus * (large ? std::min(per_cu, 12) : per_cu));
+    a->large = nb + tb > ((size_t)4 << 20);
+    a->grid_full = std::max(8, cus * per_cu);
+    a->grid = std::max(8, cus * (a->large ? std::min(per_cu, 16) : per_cu));
     a->device = dev;
     return LMX_OK;
 }
@@ -977,30 +974,81 @@ int lmx_accel_upload(lmx_accel* a)
 
 namespace lmx {
 
+// Waves of a launch over at most n_max rays, and whether they end in
+// coop_trace.  counted: the host knows that there are n_max.
+//
+// A tree within an XCD's 4 MB of L2 is traced by all the waves the registers
+// allow, 20 per CU.  Over a larger one, the 64 rays of a wave each walk their
+// own part of it, and what more waves gain in latency hidden they lose in the
+// 32 KB L1 when neighbouring rays have nothing in common; rays that do have
+// (a camera's, shadow rays of neighbouring points) are faster with 20 at any
+// length.  Few rays per wave gain from 16 either way, as the waves that end
+// first leave more of the L1 to the others, and so do queues (renderer::vcm
+// passes 5 % over a 75 MB tree).  Except where a chunk of 64 rays a wave is
+// enough with 20 and not with 16, or nearly so.  us with 20 and 16 waves per CU, a displaced
+// sphere of n triangles:
+//   closest hit, 82 k triangles, camera rays: 1 M 154 / 147, 4 M 385 / 394,
+//     8 M 697 / 733, 12 M 956 / 1014; scattered: 1 M 149 / 145, 8 M 789 / 811;
+//   1.3 M triangles, camera: 2 M 280 / 278, 8 M 825 / 880; scattered: 2 M
+//     303 / 286, 8 M 1058 / 1003;
+//   TriAccel, 328 k triangles, camera: 1 M 172 / 170, 4 M 414 / 435;
+//     scattered: 1 M 179 / 177, 4 M 494 / 512;
+//   300,000 rays, 82 k triangles: camera 59 / 96, scattered 55 / 91, occlusion
+//     96 / 119, of neighbours 87 / 110; 340,000 rays: 100 / 99, 99 / 94,
+//     131 / 123, 123 / 130; 262,144 rays: 71 / 64, 55 / 52, 90 / 87, 89 / 89;
+//   occlusion, 328 k triangles, scattered: 0.9 M 316 / 300, 1.2 M 384 / 366;
+//     neighbours: 229 / 231, 266 / 277; TriAccel, neighbours: 239 / 250,
+//     285 / 303.
+// From 400 rays a wave on (2 M) closest-hit batches take 20, but for trees
+// beyond the 256 MB last-level cache (5.2 M triangles, 8 M rays: camera 910 /
+// 946, scattered 1364 / 1311).
+//
+// In long batches the tail does not matter, and the loop is faster without
+// the code that hands over to it, in scattered rays above all; with it 20
+// waves were up to 10 % slower there than before the tail came.  Occlusion
+// from 256 rays a wave on (1.3 M), with and without: 3 M rays, 328 k
+// triangles, scattered 734 / 711, neighbours 487 / 496; 8 M: 1778 / 1643,
+// 1057 / 1067 (12 waves with the tail: 1659, 1288).  Closest hit: 12 M rays,
+// 328 k triangles, scattered 1278 / 1257, camera 1038 / 1046; 8 M rays still
+// gain from the tail (916 / 917, 754 / 766): from 2,048 rays a wave on.
+struct TraceShape {
+    uint32_t grid;
+    bool tail;
+};
+
+static TraceShape trace_shape(const lmx_accel* a, uint32_t n_max, bool anyhit, bool counted)
+{
+    const uint64_t per_wave = n_max / (uint64_t)a->grid_full;
+    const bool triaccel = a->host.isect == WBVH_ISECT_TRIACCEL;
+    const size_t bytes = a->host.nodes.size() * sizeof(WNode) + a->host.tris.size() * sizeof(WTri);
+    TraceShape t = {(uint32_t)a->grid, true};
+    if (counted && a->large) {
+        t.tail = per_wave < (anyhit ? 256u : 2048u);
+        const bool chunk = n_max > (uint64_t)LMX_CLAIM_CHUNK * a->grid && per_wave < LMX_CLAIM_CHUNK + 6u;
+        const bool full = chunk || (anyhit ? !t.tail || triaccel : per_wave >= 400u && bytes <= ((size_t)256 << 20));
+        if (full) t.grid = (uint32_t)a->grid_full;
+    }
+    // a wave per ray as long as there are waves (whole rounds of the 8
+    // regions, so that the fixed chunks cover every region)
+    t.grid = (uint32_t)std::min<uint64_t>(t.grid, ((uint64_t)n_max + 7u) / 8u * 8u);
+    return t;
+}
+
 // Enqueues one traversal launch of an accel already resident on the current
 // device, with its region cursors at `counters` (8 words,
 // CURSOR_STRIDE apart, of device memory); the stack-overflow flag is always
 // the accel's own.
-static int trace_grid(const lmx_accel* a, uint32_t n_max, bool many_occl = false)
-{
-    // a wave per ray as long as there are waves (whole rounds of the 8
-    // regions, so that the fixed chunks cover every region)
-    return (int)std::min<uint64_t>((uint64_t)(many_occl ? a->grid_occl : a->grid), ((uint64_t)n_max + 7u) / 8u * 8u);
-}
-
 static int enqueue_trace(const lmx_accel* a, uint32_t* counters, const WRay* rays, uint32_t n,
                          const uint32_t* n_dev, uint32_t n_max, WHit* hits, hipStream_t s, bool anyhit,
                          bool cursors_clear = false)
 {
     uint32_t* overflow = a->d_counters + 9 * CURSOR_STRIDE;
-    // (fewer waves only pay while each has several rounds of rays: at one
-    // round, 200,000 shadow rays, 12 waves per CU take 129 us and 16 take 98)
-    const bool many_occl = anyhit && !n_dev && n >= 4u * TRACE_WAVE * (uint32_t)a->grid_occl;
-    const int grid = trace_grid(a, n_max, many_occl);
+    const TraceShape shape = trace_shape(a, n_max, anyhit, !n_dev);
+    const uint32_t grid = shape.grid;
     const uint32_t node_bytes = (uint32_t)(a->host.nodes.size() * sizeof(WNode));   // < 4 GB, the builder's bound
     // a count the host knows goes with the launch, and when the fixed chunks
     // cover the rays no wave reads a cursor
-    if (!cursors_clear && (n_dev || trace_has_dynamic(n, (uint32_t)grid))) k_clear_cursors<<<1, 64, 0, s>>>(counters);
+    if (!cursors_clear && (n_dev || trace_has_dynamic(n, grid))) k_clear_cursors<<<1, 64, 0, s>>>(counters);
     // the list words of coop_trace hold 28-bit indices
     const uint32_t coop_max =
         a->host.nodes.size() <= (1u << COOP_TAG_SHIFT) && a->host.tris.size() <= (1u << COOP_TAG_SHIFT) ? COOP_RAYS : 0u;
@@ -1009,10 +1057,16 @@ static int enqueue_trace(const lmx_accel* a, uint32_t* counters, const WRay* ray
         kernel<<<grid, TRACE_WAVE, a->lds_bytes, s>>>(a->d_nodes, a->d_tris, rays, hits, counters, overflow,
                                                       a->stack_depth, REFILL_MIN, node_bytes, n, n_dev, coop_max);
     };
-    if (wt && !anyhit) launch(k_trace<WBVH_ISECT_WATERTIGHT, false>);
-    else if (wt) launch(k_trace<WBVH_ISECT_WATERTIGHT, true>);
-    else if (!anyhit) launch(k_trace<WBVH_ISECT_TRIACCEL, false>);
-    else launch(k_trace<WBVH_ISECT_TRIACCEL, true>);
+    auto of = [&](auto isect, auto any) {
+        if (shape.tail) launch(k_trace<isect, any, true>);
+        else launch(k_trace<isect, any, false>);
+    };
+    constexpr std::integral_constant<int, WBVH_ISECT_WATERTIGHT> watertight;
+    constexpr std::integral_constant<int, WBVH_ISECT_TRIACCEL> triaccel;
+    if (wt && !anyhit) of(watertight, std::false_type{});
+    else if (wt) of(watertight, std::true_type{});
+    else if (!anyhit) of(triaccel, std::false_type{});
+    else of(triaccel, std::true_type{});
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_error(e, "trace launch");
     return LMX_OK;

@@ -242,3 +242,31 @@ def test_unusual_ranges(gpu, n, mode):
     np.testing.assert_array_equal(hg.view(np.uint32), hh.view(np.uint32))
     np.testing.assert_array_equal(accel.hit_ids(ho) != accel.MISS, accel.hit_ids(hh) != accel.MISS)
     assert n < 100 or (accel.hit_ids(hh) != accel.MISS).any()
+
+
+@pytest.mark.parametrize("mode", [accel.ISECT_TRIACCEL, accel.ISECT_WATERTIGHT])
+def test_long_batches(gpu, mode):
+    """Batches long enough for the launch shapes of a tree beyond an XCD's L2
+    (81,920 triangles): 16 or 20 waves per CU, and the loop without the part
+    that finishes a wave's last rays (occlusion from 256 rays a wave on,
+    closest hits from 2,048).  The same rays in batches below all of those
+    lines: the same hits bit for bit, the same rays occluded."""
+    import torch
+    v, f = scenes.displaced_icosphere(6, seed=17)
+    _, rays = scenes.traversal_rays(v, res=2, n_incoherent=1 << 20, seed=4)
+    a = accel.Accel(v, f, isect=mode)
+    one = torch.from_numpy(rays).to(gpu)
+    waves = 20 * torch.cuda.get_device_properties(gpu).multi_processor_count
+    for n in (256 * waves - 1, 256 * waves, 400 * waves, 2048 * waves + 77):
+        k = torch.arange(n, device=gpu) % one.shape[0]
+        d = one[k].contiguous()
+        d[:, 7] = torch.where(k % 3 == 0, 0.9 + 1e-7 * torch.arange(n, device=gpu), d[:, 7])
+        hit, occ = a.intersect(d).view(torch.int32), a.occluded(d).view(torch.int32)[:, 3]
+        for b in range(0, n, 1 << 20):
+            part = d[b:b + (1 << 20)]
+            assert torch.equal(hit[b:b + (1 << 20)], a.intersect(part).view(torch.int32)), (n, b)
+            assert torch.equal(occ[b:b + (1 << 20)] == -1, a.occluded(part).view(torch.int32)[:, 3] == -1), (n, b)
+        assert torch.equal(occ == -1, hit[:, 3] == -1)
+    assert a.info()["stack_overflow"] == 0
+    np.testing.assert_array_equal(hit[-100003:].cpu().numpy().view(np.uint32),
+                                  a.intersect_host(d[-100003:].cpu().numpy()).view(np.uint32))
