@@ -410,10 +410,20 @@ __device__ __forceinline__ bool coop_slot_hit(float nox, float noy, float noz, u
     return tn <= tf * WBVH_FAR_SCALE;
 }
 
-// Lists on entry: node[0, nnode) and L.tri[0, ntri); cap: words of `node`.
-// A step takes more than one node only while the children of all of them
-// fit below cap - 7 depth; with one node a step the list grows by at most 7
-// a level, so it never passes cap.
+// Lists on entry: node[0, nnode) and L.tri[0, ntri); cap: words of `node`;
+// depth: the tree's levels (a node has `depth` - 1 levels below it at most).
+//
+// The node list never passes cap = 128 depth.  On entry it holds, for each of
+// at most COOP_RAYS = 12 rays, up to 7 waiting children a level and the node
+// chosen next: at most 84 (depth - 1) + 12, less than room = cap - 7 depth.  A
+// step that takes up to 8 nodes adds at most 56 and is taken only while they
+// fit below room.  Else a step takes the last node alone, at place p, and puts
+// its at most 8 children, one level down, at p .. p + 7: a node's place plus 7
+// times the levels below it stays what it was or falls, and was at most room +
+// 7 depth when such steps began.  (Trees from the builder stay far below: long
+// slivers through one another, 12 levels, 243 of 1,536 words.)  The triangle
+// list holds at most COOP_TRI_WORDS on entry; nodes are tested only in steps
+// that take all of it, and leave at most 8 x 24.
 template <int ISECT, bool ANYHIT>
 __device__ __forceinline__ void coop_trace(CoopLds& L, uint32_t* node, uint32_t nnode, uint32_t ntri, uint32_t cap,
                                            uint32_t depth, __amdgpu_buffer_rsrc_t nrs, const WTri* __restrict__ tris)

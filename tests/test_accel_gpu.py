@@ -270,3 +270,56 @@ def test_long_batches(gpu, mode):
     assert a.info()["stack_overflow"] == 0
     np.testing.assert_array_equal(hit[-100003:].cpu().numpy().view(np.uint32),
                                   a.intersect_host(d[-100003:].cpu().numpy()).view(np.uint32))
+
+
+def _slivers(n, rng):
+    """Thin triangles along the diagonal of the unit cube: nearly every box
+    of the tree spans the cube."""
+    a, d = 0.02 * rng.random((n, 3)), 0.02 * rng.random((n, 3))
+    return np.stack([a, 1.0 - d, a + 0.004 * rng.random((n, 3))], axis=1)
+
+
+def _shells(n, rng):
+    """Rings of small triangles around the x axis, in clusters of geometric
+    spacing: a tree of many levels whose nodes' boxes all hold the axis."""
+    c, s, i = np.meshgrid(np.arange(n), np.arange(8), np.arange(8), indexing="ij")
+    x = 0.7 ** c
+    a = 2.0 * np.pi * (i + 0.5) / 8
+    x0, r = x - 0.27 * x * (s + 1) / 8, 0.3 * x
+    def ring(dx, da):
+        return np.stack([x0 + dx * x, r * np.cos(a + da), r * np.sin(a + da)], axis=-1)
+    return np.stack([ring(0, 0), ring(0.006, 0), ring(0, 0.05)], axis=-2).reshape(-1, 3, 3)
+
+
+@pytest.mark.parametrize("mode", [accel.ISECT_TRIACCEL, accel.ISECT_WATERTIGHT])
+@pytest.mark.parametrize("make,size", [(_slivers, 70), (_slivers, 3000), (_slivers, 6000), (_shells, 9), (_shells, 90)])
+def test_last_rays_in_deep_trees(gpu, make, size, mode):
+    """The last rays of a wave in trees whose boxes overlap or nest over many
+    levels, so that a ray has many nodes waiting at every level when all lanes
+    take it over and most nodes it visits have several children hit.  Waves of
+    12 and 13 rays, and of 64 of which 12 go through everything and the rest
+    end early; bit-exact against the host walker."""
+    import torch
+    rng = np.random.default_rng(size)
+    t = make(size, rng).astype(np.float32)
+    v, f = t.reshape(-1, 3), np.arange(3 * len(t), dtype=np.uint32).reshape(-1, 3)
+    a = accel.Accel(v, f, isect=mode)
+    waves = 20 * torch.cuda.get_device_properties(gpu).multi_processor_count
+    for per in (12, 13, 64):
+        n = per * waves
+        rays = np.empty((n, 8), np.float32)
+        if make is _slivers:
+            m = rng.random((n, 1))
+            rays[:, 0:3] = np.where(rng.random((n, 1)) < 0.5, m + 0.05 * (rng.random((n, 3)) - 0.5), rng.random((n, 3)))
+            rays[:, 4:7] = 2.0 * rng.random((n, 3)) - 1.0
+        else:
+            rays[:, 0:3] = 0.0
+            rays[:, 4] = 1.0
+            rays[:, 5:7] = 0.3 * (rng.random((n, 2)) - 0.5)
+        rays[:, 3] = 0.0
+        rays[:, 7] = np.where(np.arange(n) % per < 12, 1e30, 0.3 * rng.random(n) ** 6)
+        d = torch.from_numpy(rays).to(gpu)
+        hg, ho, hh = a.intersect(d).cpu().numpy(), a.occluded(d).cpu().numpy(), a.intersect_host(rays)
+        np.testing.assert_array_equal(hg.view(np.uint32), hh.view(np.uint32))
+        np.testing.assert_array_equal(accel.hit_ids(ho) != accel.MISS, accel.hit_ids(hh) != accel.MISS)
+    assert a.info()["stack_overflow"] == 0
