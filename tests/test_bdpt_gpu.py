@@ -166,6 +166,22 @@ def test_connection_rounds_beyond_the_queue(gpu, sampler, maxv, n):
     assert a.min() > 0.5 and np.abs(a - b).max() <= per_pixel * 2.0 ** -24 * b.max()
 
 
+@pytest.mark.parametrize("sampler,maxv,n,batch", [("bdpt", -1, 150063, 50021), ("vcm_bdpt", 32, 250000, 100003)])
+def test_batches_of_several_rounds(gpu, sampler, maxv, n, batch):
+    """Batches beyond the queue's budget that come again: the recorded step
+    holds one connection round, the others follow it, then the next batch;
+    the last batch is ragged in one case.  The film of small batches, as
+    above."""
+    sc = scenes.furnace_sphere(albedo=0.5, Le=1.0, subdiv=2, width=8, height=8)
+    rs = render.Scene(sc)
+    large, st, _ = getattr(rs, "render_" + sampler)(n, max_num_vertices=maxv, seed=3, batch=batch)
+    small, sm, _ = getattr(render.Scene(sc), "render_" + sampler)(n, max_num_vertices=maxv, seed=3, batch=8000)
+    assert st["batches"] == 3 and sm["batches"] == (n + 7999) // 8000
+    assert st["rays"] == sm["rays"] and st["rays"] > 3 * n
+    a, b = large.cpu().numpy().astype(np.float64), small.cpu().numpy().astype(np.float64)
+    assert a.min() > 0.5 and np.abs(a - b).max() <= st["rays"] / 64.0 * 2.0 ** -24 * b.max()
+
+
 @pytest.fixture
 def little_memory(gpu):
     """Leaves 3,000 MB of the device free, the rest held by tensors."""

@@ -235,6 +235,7 @@ def _split_cornell(ntri, **kw):
         k = len(verts) - 1
         tris += [[k, a, b], [k, c, a]]
         mat += [m, m]
+    assert len(tris) + 2 == ntri
     return dict(sc, verts=np.array(verts, np.float32), lights=[(len(tris), 2)],
                 tris=np.array(tris + sc["tris"][-2:].tolist(), np.uint32),
                 tri_mat=np.array(mat + sc["tri_mat"][-2:].tolist(), np.uint32))
@@ -242,7 +243,7 @@ def _split_cornell(ntri, **kw):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("ntri,n,cap,kw", [
-    (34, 1, 0, {}), (34, 63, 0, {}), (34, 255, 64, dict(phong_boxes=20.0)), (34, 257, 0, dict(ggx_boxes=0.2)),
+    (36, 1, 0, {}), (36, 63, 0, {}), (36, 255, 64, dict(phong_boxes=20.0)), (36, 257, 0, dict(ggx_boxes=0.2)),
     (47, 100003, 0, {}), (48, 20001, 1000, dict(ggx_boxes=0.5)), (48, 700001, 0, {}), (49, 5000, 0, {})])
 @pytest.mark.parametrize("entry", ["pt", "ptmis", "ptdirect"])
 def test_few_triangles(gpu, entry, ntri, n, cap, kw):
@@ -263,9 +264,33 @@ def test_few_triangles(gpu, entry, ntri, n, cap, kw):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("ntri", [1, 2, 4])
+@pytest.mark.parametrize("entry", ["pt", "ptmis", "ptdirect"])
+def test_fewest_triangles(gpu, entry, ntri):
+    """A light of one triangle or two facing the camera, and one over a
+    floor, against the queues: the same rays and records, bit for bit."""
+    sc = scenes.cornell_box(31, 17)
+    quad = [[-1, -0.4, 0], [1, -0.4, 0], [1, 0.9, 0.1], [-1, 0.9, 0.1]]
+    floor = [[-2, -0.5, 2], [2, -0.5, 2], [2, -0.5, -2], [-2, -0.5, -2]]
+    tris, mat = [[0, 1, 2], [0, 2, 3], [4, 5, 6], [4, 6, 7]], [3, 3, 0, 0]
+    rs = render.Scene(dict(sc, verts=np.array(quad + floor, np.float32), tris=np.array(tris[:ntri], np.uint32),
+                           tri_mat=np.array(mat[:ntri], np.uint32), lights=[(0, min(ntri, 2))]))
+    n = 20011
+    for opts in (dict(max_num_vertices=-1, rr_depth=1), dict(max_num_vertices=2), dict(max_num_vertices=5)):
+        (fa, sa, ra), (fb, sb, rb) = [
+            getattr(rs, "render_" + entry)(n, seed=7, sample_out=True, shade_order=order, **opts)
+            for order in (render.SHADE_QUEUE, render.SHADE_BY_MATERIAL)]
+        assert sa["rays"] == sb["rays"] >= n and sa["samples"] == n
+        assert entry == "ptdirect" or float(fa.max()) > 1.0
+        assert np.array_equal(np.asarray(ra.cpu()).view(np.uint32), np.asarray(rb.cpu()).view(np.uint32))
+        # FP32 sums of a pixel's terms of one sign in another order
+        assert float((fa - fb).abs().max()) <= 8.0 * (n / (31 * 17) + 30.0) * 2.0 ** -24 * 2 * float(fb.abs().max())
+
+
+@pytest.mark.gpu
 def test_few_triangles_beyond_one_launch(gpu):
-    """More samples than one launch takes (2^26): every one is counted and splat once."""
-    rs = render.Scene(_split_cornell(34))
+    """More samples than a path tracer's frame usually has (2^26): every one is counted and splat once."""
+    rs = render.Scene(_split_cornell(36))
     n = (1 << 26) + 7
     (fa, sa, _), (fb, sb, _) = [rs.render_pt(n, seed=3, max_num_vertices=2, shade_order=order)
                                 for order in (render.SHADE_QUEUE, render.SHADE_BY_MATERIAL)]
