@@ -237,7 +237,8 @@ typedef struct lmx_render_params {
 typedef struct lmx_render_stats {
     uint64_t rays;               /* extension rays traced */
     uint32_t iterations;         /* wavefront iterations; without queues: launches (1 but for very long frames) */
-    uint32_t queue_capacity;     /* capacity used (without queues: paths in flight) */
+    uint32_t queue_capacity;     /* queue_capacity or the tuned one, at most num_samples (but 64); with neither
+                                    queues nor queue_capacity: the paths in flight.  Batch samplers: the batch */
     double ms;                   /* wall time of the render call */
     uint64_t samples;            /* camera samples taken (num_samples unless render_time > 0) */
     uint64_t dropped;            /* lmx_render_vcm: merges dropped because their contribution was not

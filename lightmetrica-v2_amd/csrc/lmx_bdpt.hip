@@ -2297,7 +2297,7 @@ int render_bidir(lmx_scene* sc, const lmx_render_params* p, int variant, const c
         while (rc == LMX_OK && b < nbatch) {
             if ((rc = bd_run_batch(sc, bp, g, true, st)) != LMX_OK) break;
             if ((e = hipStreamSynchronize(st)) != hipSuccess) {
-                rc = hip_error(e, "graph launch");
+                rc = hip_error(e, "bdpt batch");
                 break;
             }
             b++;
@@ -2421,8 +2421,9 @@ int vc_enqueue_photons(lmx_scene* sc, const BParams& pp, hipStream_t st, bool gr
     return e == hipSuccess ? LMX_OK : hip_error(e, "vcm photon launch");
 }
 
-// renderer::vcm, modes vcm and bdpm: per pass the photon graph, then the eye
-// batches (each one graph: subpaths, connections, shadow rays, merges); the
+// renderer::vcm, modes vcm and bdpm: per pass the photon phase, then the eye
+// batches (subpaths, connections, shadow rays, merges), each recorded as a
+// graph when it comes again; the
 // film holds the sum of every pass's splats, scaled at the end by
 // W H / (N_eye passes) -- the mean of the per-pass images that the
 // reference's running rescale (renderer_vcm.cpp:752-757) keeps.
@@ -2565,7 +2566,7 @@ int pm_enqueue_eye(lmx_scene* sc, const BParams& bp, const PMArgs& pa, hipStream
     return e == hipSuccess ? LMX_OK : hip_error(e, "pm launch");
 }
 
-// renderer::pm: the photon graph (roulette light subpaths, the grid over
+// renderer::pm: the photon phase (roulette light subpaths, the grid over
 // their diffuse and glossy vertices), then the eye batches; film scaled by
 // W H / N as the scheduler does (scheduler.cpp:281-288).
 int render_pm(lmx_scene* sc, const lmx_render_params* p, const lmx_pm_params* v, float* film_rgb, void* stream,
@@ -2668,7 +2669,7 @@ int render_pm(lmx_scene* sc, const lmx_render_params* p, const lmx_pm_params* v,
 }
 
 // renderer::ppm: the measurement points (one eye batch of every sample,
-// subpaths of 2 vertices), then per pass the photon graph and the
+// subpaths of 2 vertices), then per pass the photon phase and the
 // progressive update, then the film.
 int render_ppm(lmx_scene* sc, const lmx_render_params* p, const lmx_ppm_params* v, float* film_rgb, void* stream,
                lmx_render_stats* stats)
@@ -2795,7 +2796,7 @@ int render_ppm(lmx_scene* sc, const lmx_render_params* p, const lmx_ppm_params* 
 }
 
 // renderer::sppm: per pass the pixels' points (one eye batch of W H
-// samples, 2-vertex subpaths), the photon graph, the per-pixel update; the
+// samples, 2-vertex subpaths), the photon phase, the per-pixel update; the
 // film written after the last pass.
 int render_sppm(lmx_scene* sc, const lmx_render_params* p, const lmx_ppm_params* v, float* film_rgb, void* stream,
                 lmx_render_stats* stats)
@@ -2917,7 +2918,7 @@ int render_sppm(lmx_scene* sc, const lmx_render_params* p, const lmx_ppm_params*
     return rc;
 }
 
-// renderer::ltdirect: batches of B light subpaths through the photon graph
+// renderer::ltdirect: batches of B light subpaths through the photon phase
 // (no grid), their camera connections, the any-hit trace, the splat; film
 // scaled by W H / N.
 int render_ltdirect(lmx_scene* sc, const lmx_render_params* p, float* film_rgb, void* stream, lmx_render_stats* stats)

@@ -442,8 +442,7 @@ RD void guide_inputs(const GuideDev& G, f3 p, f3 n, f3 wi, float* x)
 
 struct Mix {
     f3 mu[8];
-    float mlen[8], kap[8], pi[8], alpha, sig;
-    bool kclamp[8];
+    float kap[8], pi[8], alpha;
 };
 
 // The mixture's arithmetic uses the hardware's exp / log / reciprocal /
@@ -462,13 +461,9 @@ RD void mix_decode(const float* y, Mix& m)
     for (int k = 0; k < 8; k++) {
         const f3 r = mk3(y[3 * k], y[3 * k + 1], y[3 * k + 2]);
         const float l = mx_sqrt(dot(r, r));
-        m.mlen[k] = l;
         const float il = mx_div(1.0f, l);
         m.mu[k] = l > 0.0f ? mk3(r.x * il, r.y * il, r.z * il) : mk3(0.0f, 0.0f, 1.0f);
-        float lk = y[24 + k];
-        m.kclamp[k] = lk < LOGK_MIN || lk > LOGK_MAX;
-        lk = fminf(fmaxf(lk, LOGK_MIN), LOGK_MAX);
-        m.kap[k] = mx_exp(lk);
+        m.kap[k] = mx_exp(fminf(fmaxf(y[24 + k], LOGK_MIN), LOGK_MAX));
     }
     float mx = y[32];
 #pragma unroll
@@ -479,8 +474,7 @@ RD void mix_decode(const float* y, Mix& m)
     const float is = mx_div(1.0f, s);
 #pragma unroll
     for (int k = 0; k < 8; k++) m.pi[k] *= is;
-    m.sig = mx_div(1.0f, 1.0f + mx_exp(-y[40]));
-    m.alpha = ALPHA_MIN + ALPHA_SPAN * m.sig;
+    m.alpha = ALPHA_MIN + ALPHA_SPAN * mx_div(1.0f, 1.0f + mx_exp(-y[40]));
 }
 
 // kappa >= e^-4, so 1 - e^{-2 kappa} >= 0.036 keeps its relative error

@@ -438,7 +438,7 @@ __global__ __launch_bounds__(256) void k_nee_splat(RParams p, const Ctl* __restr
 // lie in LDS in each of the six orders of axes that the watertight test can
 // want: a lane reads its order, three 16-byte reads with at most six addresses
 // in a wave, instead of choosing each coordinate (18 of 62 instructions of a
-// test; a 1 M path Cornell box with up to 9 vertices, 34 triangles: 545 -> 460
+// test; a 1 M path Cornell box with up to 9 vertices, 36 triangles: 545 -> 460
 // us).  A workgroup owns a contiguous share of the samples and its lanes take
 // the next one when a path ends (a fixed stride of samples per lane: 460, this:
 // 379), at 5 waves a SIMD (4: 379, 5: 362, 6 with spills: 364).  With
@@ -448,9 +448,11 @@ __global__ __launch_bounds__(256) void k_nee_splat(RParams p, const Ctl* __restr
 // registers' limit).  The wavefront pipeline takes 690 and 2370.
 //
 // SMALL_TRIS: Cornell boxes of split triangles, 16.8 M paths, us here and in
-// the wavefront pipeline: 34: 3700 / 9150, 48: 6350 / 6860 to 7750,
+// the wavefront pipeline: 36: 3700 / 9150, 48: 6350 / 6860 to 7750,
 // 64: 8420 / 8100, 80: 10440 / 8410; 1 M paths with next-event estimation:
-// 34: 1545 / 2365, 48: 1680 / 2440, 64: 1790 / 2500.
+// 36: 1545 / 2365, 48: 1680 / 2440, 64: 1790 / 2500.  So with next-event
+// estimation the one kernel is ahead beyond 64; the line is that of
+// renderer::pt, where it is not.
 #define SMALL_TRIS 48u
 //
 // A launch is short whatever the number of samples and the length of their
