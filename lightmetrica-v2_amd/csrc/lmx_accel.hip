@@ -83,6 +83,7 @@ struct lmx_accel {
     WTri* d_tris = nullptr;
     uint32_t* d_counters = nullptr;   // 8 region cursors, a free line, the stack-overflow flag; CURSOR_STRIDE words apart
     int grid_full = 0;                // waves that the device holds at once
+    int grid_occl = 0;                // waves of a launch over many occlusion rays
     int grid = 0;                     // waves of a launch over few rays, or over a queue (trace_shape)
     bool large = false;               // the tree exceeds an XCD's L2
     int stack_depth = 0;              // LDS stack entries per lane
@@ -975,6 +976,7 @@ int lmx_accel_upload(lmx_accel* a)
     per_cu = std::max(1, per_cu);
     a->large = nb + tb > ((size_t)4 << 20);
     a->grid_full = std::max(8, cus * per_cu);
+    a->grid_occl = std::max(8, cus * std::min(per_cu, 19));
     a->grid = std::max(8, cus * (a->large ? std::min(per_cu, 16) : per_cu));
     a->device = dev;
     return LMX_OK;
@@ -995,8 +997,8 @@ namespace lmx {
 // length.  Few rays per wave gain from 16 either way, as the waves that end
 // first leave more of the L1 to the others, and so do queues (renderer::vcm
 // passes 5 % over a 75 MB tree).  Except where a chunk of 64 rays a wave is
-// enough with 20 and not with 16, or nearly so.  us with 20 and 16 waves per CU, a displaced
-// sphere of n triangles:
+// enough with 20 and not with 16, or nearly so.  us with 20 and 16 waves per
+// CU, a displaced sphere of n triangles:
 //   closest hit, 82 k triangles, camera rays: 1 M 154 / 147, 4 M 385 / 394,
 //     8 M 697 / 733, 12 M 956 / 1014; scattered: 1 M 149 / 145, 8 M 789 / 811;
 //   1.3 M triangles, camera: 2 M 280 / 278, 8 M 825 / 880; scattered: 2 M
@@ -1014,13 +1016,15 @@ namespace lmx {
 // 946, scattered 1364 / 1311).
 //
 // In long batches the tail does not matter, and the loop is faster without
-// the code that hands over to it, in scattered rays above all; with it 20
-// waves were up to 10 % slower there than before the tail came.  Occlusion
-// from 256 rays a wave on (1.3 M), with and without: 3 M rays, 328 k
-// triangles, scattered 734 / 711, neighbours 487 / 496; 8 M: 1778 / 1643,
-// 1057 / 1067 (12 waves with the tail: 1659, 1288).  Closest hit: 12 M rays,
-// 328 k triangles, scattered 1278 / 1257, camera 1038 / 1046; 8 M rays still
-// gain from the tail (916 / 917, 754 / 766): from 2,048 rays a wave on.
+// the code that hands over to it.  Occlusion from 256 rays a wave on (1.3 M):
+// with 20 waves and the tail, scattered rays took up to 12 % longer than
+// before the tail came, with 12 waves neighbouring rays up to 20 % longer.  us
+// with 20, 19 and 16 waves without it, and before it came, 328 k triangles:
+// 3 M rays scattered 813, 798, 763, 807, of neighbouring points 499, 503, 526,
+// 511; 8 M rays 1991, 1977, 1897, 1991 and 1070, 1086, 1142, 1101.  19 is the
+// count with which neither loses.  Closest hit: 12 M rays, 328 k triangles,
+// scattered 1278 with the tail, 1257 without, camera 1038 / 1046; 8 M rays
+// still gain from the tail (916 / 917, 754 / 766): from 2,048 rays a wave on.
 struct TraceShape {
     uint32_t grid;
     bool tail;
@@ -1035,8 +1039,9 @@ static TraceShape trace_shape(const lmx_accel* a, uint32_t n_max, bool anyhit, b
     if (counted && a->large) {
         t.tail = per_wave < (anyhit ? 256u : 2048u);
         const bool chunk = n_max > (uint64_t)LMX_CLAIM_CHUNK * a->grid && per_wave < LMX_CLAIM_CHUNK + 6u;
-        const bool full = chunk || (anyhit ? !t.tail || triaccel : per_wave >= 400u && bytes <= ((size_t)256 << 20));
+        const bool full = chunk || (anyhit ? triaccel : per_wave >= 400u && bytes <= ((size_t)256 << 20));
         if (full) t.grid = (uint32_t)a->grid_full;
+        if (anyhit && !t.tail) t.grid = (uint32_t)a->grid_occl;
     }
     // a wave per ray as long as there are waves (whole rounds of the 8
     // regions, so that the fixed chunks cover every region)
