@@ -82,10 +82,8 @@ struct lmx_accel {
     WNode* d_nodes = nullptr;
     WTri* d_tris = nullptr;
     uint32_t* d_counters = nullptr;   // 8 region cursors, a free line, the stack-overflow flag; CURSOR_STRIDE words apart
-    int grid_full = 0;                // waves that the device holds at once
-    int grid_occl = 0;                // waves of a launch over many occlusion rays
-    int grid = 0;                     // waves of a launch over few rays, or over a queue (trace_shape)
-    bool large = false;               // the tree exceeds an XCD's L2
+    int cus = 0;
+    int per_cu = 0;                   // waves a CU holds at once
     int stack_depth = 0;              // LDS stack entries per lane
     size_t lds_bytes = 0;
 };
@@ -973,11 +971,8 @@ int lmx_accel_upload(lmx_accel* a)
     else
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_trace<WBVH_ISECT_TRIACCEL, false, true>, TRACE_WAVE, a->lds_bytes);
     if (e != hipSuccess) return hip_error(e, "lmx_accel_upload: occupancy query");
-    per_cu = std::max(1, per_cu);
-    a->large = nb + tb > ((size_t)4 << 20);
-    a->grid_full = std::max(8, cus * per_cu);
-    a->grid_occl = std::max(8, cus * std::min(per_cu, 19));
-    a->grid = std::max(8, cus * (a->large ? std::min(per_cu, 16) : per_cu));
+    a->cus = cus;
+    a->per_cu = std::max(1, per_cu);
     a->device = dev;
     return LMX_OK;
 }
@@ -1000,20 +995,25 @@ namespace lmx {
 // enough with 20 and not with 16, or nearly so.  us with 20 and 16 waves per
 // CU, a displaced sphere of n triangles:
 //   closest hit, 82 k triangles, camera rays: 1 M 154 / 147, 4 M 385 / 394,
-//     8 M 697 / 733, 12 M 956 / 1014; scattered: 1 M 149 / 145, 8 M 789 / 811;
-//   1.3 M triangles, camera: 2 M 280 / 278, 8 M 825 / 880; scattered: 2 M
-//     303 / 286, 8 M 1058 / 1003;
+//     8 M 697 / 733 (18: 716), 12 M 956 / 1014; scattered: 1 M 149 / 145, 8 M
+//     789 / 811 (795);
+//   1.3 M triangles, camera: 2 M 280 / 278, 8 M 829 / 880 (854); scattered:
+//     2 M 303 / 286, 8 M 1058 / 1003 (1028); half and half 8 M 929 / 919 (913);
 //   TriAccel, 328 k triangles, camera: 1 M 172 / 170, 4 M 414 / 435;
-//     scattered: 1 M 179 / 177, 4 M 494 / 512;
+//     scattered: 1 M 179 / 177, 4 M 494 / 512; 8 M 805 / 868 (834), 1025 /
+//     1064 (1032);
 //   300,000 rays, 82 k triangles: camera 59 / 96, scattered 55 / 91, occlusion
 //     96 / 119, of neighbours 87 / 110; 340,000 rays: 100 / 99, 99 / 94,
 //     131 / 123, 123 / 130; 262,144 rays: 71 / 64, 55 / 52, 90 / 87, 89 / 89;
 //   occlusion, 328 k triangles, scattered: 0.9 M 316 / 300, 1.2 M 384 / 366;
 //     neighbours: 229 / 231, 266 / 277; TriAccel, neighbours: 239 / 250,
 //     285 / 303.
-// From 400 rays a wave on (2 M) closest-hit batches take 20, but for trees
-// beyond the 256 MB last-level cache (5.2 M triangles, 8 M rays: camera 910 /
-// 946, scattered 1364 / 1311).
+// From 400 rays a wave on (2 M) closest-hit batches take 18, with which no
+// order of rays is slower than it was with 20 before the tail came (82 k
+// triangles, 8 M rays: camera 718, scattered 816; 1.3 M: 869, 1074), with
+// TriAccel 20 (328 k: 831, 1086), but for trees beyond the 256 MB last-level
+// cache (5.2 M triangles, 8 M rays, 20 and 16: camera 910 / 946, scattered
+// 1364 / 1311).
 //
 // In long batches the tail does not matter, and the loop is faster without
 // the code that hands over to it.  Occlusion from 256 rays a wave on (1.3 M):
@@ -1032,17 +1032,20 @@ struct TraceShape {
 
 static TraceShape trace_shape(const lmx_accel* a, uint32_t n_max, bool anyhit, bool counted)
 {
-    const uint64_t per_wave = n_max / (uint64_t)a->grid_full;
+    constexpr int ALL = 20;
+    const uint64_t per_wave = n_max / ((uint64_t)a->cus * (uint64_t)a->per_cu);
     const bool triaccel = a->host.isect == WBVH_ISECT_TRIACCEL;
     const size_t bytes = a->host.nodes.size() * sizeof(WNode) + a->host.tris.size() * sizeof(WTri);
-    TraceShape t = {(uint32_t)a->grid, true};
-    if (counted && a->large) {
+    const bool large = bytes > ((size_t)4 << 20);
+    int waves = large ? 16 : ALL;          // per CU
+    TraceShape t = {0, true};
+    if (counted && large) {
         t.tail = per_wave < (anyhit ? 256u : 2048u);
-        const bool chunk = n_max > (uint64_t)LMX_CLAIM_CHUNK * a->grid && per_wave < LMX_CLAIM_CHUNK + 6u;
-        const bool full = chunk || (anyhit ? triaccel : per_wave >= 400u && bytes <= ((size_t)256 << 20));
-        if (full) t.grid = (uint32_t)a->grid_full;
-        if (anyhit && !t.tail) t.grid = (uint32_t)a->grid_occl;
+        if (n_max > (uint64_t)LMX_CLAIM_CHUNK * 16u * (uint64_t)a->cus && per_wave < LMX_CLAIM_CHUNK + 6u) waves = ALL;
+        else if (anyhit) waves = !t.tail ? 19 : triaccel ? ALL : 16;
+        else if (per_wave >= 400u && bytes <= ((size_t)256 << 20)) waves = triaccel || !t.tail ? ALL : 18;
     }
+    t.grid = (uint32_t)std::max(8, a->cus * std::min(a->per_cu, waves));
     // a wave per ray as long as there are waves (whole rounds of the 8
     // regions, so that the fixed chunks cover every region)
     t.grid = (uint32_t)std::min<uint64_t>(t.grid, ((uint64_t)n_max + 7u) / 8u * 8u);
