@@ -31,7 +31,7 @@
 //   * the last rays of each wave, and a batch with few rays per wave from
 //     the start, are traced by all its lanes together, eight to a node
 //     (coop_trace): the serial chain of the longest ray, not throughput,
-//     bounds them.
+//     bounds them (long batches do without: trace_shape).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

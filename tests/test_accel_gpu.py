@@ -224,9 +224,9 @@ def test_last_rays_of_a_wave(gpu, n, subdiv, mode):
 @pytest.mark.parametrize("mode", [accel.ISECT_TRIACCEL, accel.ISECT_WATERTIGHT])
 @pytest.mark.parametrize("n", [9, 2001, 200003])
 def test_unusual_ranges(gpu, n, mode):
-    """tmin and tmax of NaN (either sign), infinity, -0 and crossed: the same
-    hits as the host walker's, bit for bit, whichever part of the kernel
-    traces the ray."""
+    """tmin and tmax of NaN (either sign), infinity, -0 and crossed, and
+    origins and directions that are not finite: the same hits as the host
+    walker's, bit for bit, whichever part of the kernel traces the ray."""
     import torch
     v, f = scenes.displaced_icosphere(3, seed=5)
     _, rays = scenes.traversal_rays(v, res=2, n_incoherent=n, seed=n)
@@ -235,6 +235,7 @@ def test_unusual_ranges(gpu, n, mode):
     k = np.arange(len(rays))
     rays[:, 7] = np.where(k % 8 < 6, odd[k % 8 % 6], rays[:, 7])
     rays[:, 3] = np.where(k % 11 < 6, odd[k % 11 % 6], rays[:, 3])
+    rays[5::37, 0], rays[7::41, 5], rays[11::43, 6], rays[3::47, 1] = np.inf, np.nan, -np.inf, np.nan
     a = accel.Accel(v, f, isect=mode)
     d = torch.from_numpy(rays).to(gpu)
     hg, ho = a.intersect(d).cpu().numpy(), a.occluded(d).cpu().numpy()
