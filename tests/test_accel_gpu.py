@@ -195,11 +195,11 @@ def test_occlusion_matches_closest_hit(gpu, tmax_scale):
 
 @pytest.mark.parametrize("mode", [accel.ISECT_TRIACCEL, accel.ISECT_WATERTIGHT])
 @pytest.mark.parametrize("subdiv", [0, 2, 5])
-@pytest.mark.parametrize("n", [1, 7, 9, 63, 4097, 12 * 4096 + 5, 13 * 5120 + 1])
+@pytest.mark.parametrize("n", [1, 7, 9, 63, 4097, 8 * 5120, 8 * 5120 + 1, 12 * 4096 + 5, 13 * 5120 + 1])
 def test_last_rays_of_a_wave(gpu, n, subdiv, mode):
     """The part of the kernel that traces a wave's last rays with all its
-    lanes: alone (one ray per wave, up to 12), and after the one-ray-per-lane
-    loop (13 and more); trees of one level and of many; tmin below 0, finite
+    lanes: alone (one ray per wave, up to 8), and after the one-ray-per-lane
+    loop (64 a wave); trees of one level and of many; tmin below 0, finite
     tmax, zero direction components and rays that cannot hit.  Bit-exact
     against the host walker over the same BVH, which visits one ray at a
     time; an occlusion query agrees with the closest hit."""
@@ -298,15 +298,15 @@ def test_last_rays_in_deep_trees(gpu, make, size, mode):
     """The last rays of a wave in trees whose boxes overlap or nest over many
     levels, so that a ray has many nodes waiting at every level when all lanes
     take it over and most nodes it visits have several children hit.  Waves of
-    12 and 13 rays, and of 64 of which 12 go through everything and the rest
-    end early; bit-exact against the host walker."""
+    8 rays, and of 64 of which 12 go through everything and the rest end early;
+    bit-exact against the host walker."""
     import torch
     rng = np.random.default_rng(size)
     t = make(size, rng).astype(np.float32)
     v, f = t.reshape(-1, 3), np.arange(3 * len(t), dtype=np.uint32).reshape(-1, 3)
     a = accel.Accel(v, f, isect=mode)
     waves = 20 * torch.cuda.get_device_properties(gpu).multi_processor_count
-    for per in (12, 13, 64):
+    for per in (8, 64):
         n = per * waves
         rays = np.empty((n, 8), np.float32)
         if make is _slivers:
